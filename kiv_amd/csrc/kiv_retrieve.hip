@@ -42,6 +42,8 @@ constexpr int kScanThreads = 256;   // coarse scan block (4 waves)
 // 7.36 and 6.26 with 4-wave blocks; 1-wave blocks help the HBM tier only,
 // 8- and 16-wave blocks are slower.
 constexpr int kScanMfmaThreads = 128;
+constexpr int kScanRowsPerSlice = 64;  // query rows per grid-z slice of the MFMA coarse scan
+constexpr int64_t kCoarseKeyBytes = int64_t(64) << 20;  // coarse keys of one pass of a long query
 constexpr int kSelThreads = 512;       // select block (8 waves)
 constexpr int kWideSelThreads = 1024;  // fine select block for rows of many candidates (16 waves)
 constexpr int kMaxWords = 4096;     // bitmap words ranked in LDS (131072 pages)
@@ -858,19 +860,24 @@ __global__ void __launch_bounds__(kScanThreads) coarse_scan_kernel(
 // each per instruction; D[row 4(l/16)+i][page l%16] comes back in the
 // lane's i-th accumulator.  Products of 16-bit values are exact in fp32
 // and accumulate in fp32, like the dot products of the scalar kernel.
-// Every summary byte is loaded once, the query rows by ordinary loads
-// issued together with it; no LDS, no barrier.
+// Every summary byte is loaded once per slice of query rows (grid z; one
+// slice when the page bounds are written, which take the maximum over all
+// rows), the query rows by ordinary loads issued together with it, the next
+// 16 while the current ones are scored; no LDS, no barrier.
 constexpr int kScanMfmaPages = 16;  // pages per wave
 
-template <int DT, int KT>  // KT = head_dim / 32
+// KT = head_dim / 32.  SL: this block takes the query rows of slice
+// blockIdx.z (no page bounds); the unsliced instance stays free of the
+// slices' prefetch registers (NS shape's scan 5.0 against 5.16 us).
+template <int DT, int KT, bool SL>
 __global__ void __launch_bounds__(kScanMfmaThreads) coarse_scan_mfma_kernel(
     const char *__restrict__ summ, int64_t n_pages, int kr, const char *__restrict__ q, int64_t qs0,
     int64_t qs1, int64_t qs2, int hq, int hkv, int qlen, float scale, int round, uint32_t *__restrict__ keys,
     int64_t ld, const float *__restrict__ rad2, uint32_t *__restrict__ ubk, uint32_t *__restrict__ lbk,
-    const int32_t *__restrict__ ctl, AppendRows ap) {
+    const int32_t *__restrict__ ctl, AppendRows ap, int zrows) {
   static_assert(DT != DT_F32, "16-bit dtypes only");
   if ((ap.count > 0 || ap.hot_count > 0) && blockIdx.x == gridDim.x - 1) {
-    append_rows(ap, blockIdx.y);  // the step's evicted rows (an extra block per kv row)
+    if (blockIdx.z == 0) append_rows(ap, blockIdx.y);  // the step's evicted rows (an extra block per kv row)
     return;
   }
   constexpr int64_t kRowBytes = (int64_t)KT * 64;  // 32 two-byte elements per K step
@@ -896,8 +903,10 @@ __global__ void __launch_bounds__(kScanMfmaThreads) coarse_scan_mfma_kernel(
   // Loads in the order they are used: the first 16 query rows' operands
   // and, for the bounds, the page row's radius and |s|, then the summaries,
   // so that the rows' norms are computed while the summaries are in flight.
+  const int mz = SL ? (int)blockIdx.z * zrows : 0, mend = SL ? min(GQ, mz + zrows) : GQ;  // this slice's query rows
   uint4 q0[KT];
-  q_tile(0, q0);
+  q_tile(mz, q0);
+  if constexpr (SL) ubk = nullptr;
   const float rad = ubk ? rad2[2 * (pc * kr + r)] : 0.f, sn = ubk ? rad2[2 * (pc * kr + r) + 1] : 0.f;
   uint4 x[KT];
 #pragma unroll
@@ -924,11 +933,12 @@ __global__ void __launch_bounds__(kScanMfmaThreads) coarse_scan_mfma_kernel(
   };
   const float qn0 = ubk ? q_norm(q0) : 0.f;
   float hi = -INFINITY, lo = -INFINITY;
-  for (int m0 = 0; m0 < GQ; m0 += 16) {
+  for (int m0 = mz; m0 < mend; m0 += 16) {
     uint4 qa[KT];
-    if (m0 == 0) {
+    if (SL || m0 == 0) {
 #pragma unroll
       for (int kk = 0; kk < KT; ++kk) qa[kk] = q0[kk];
+      if (SL && m0 + 16 < mend) q_tile(m0 + 16, q0);
     } else {
       q_tile(m0, qa);
     }
@@ -2724,7 +2734,15 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
       // lists; long ones (or several passes) get the union kernels.
       union_src = passes == 1 && (int64_t)rows * kc <= kRowListInScan ? UNION_ROWS : UNION_LIST;
       const int64_t ld = ((int64_t)N + 63) & ~int64_t(63);
-      const int rows_pass = B * hq * Qb;
+      // Positions per coarse pass: the fine scan's Qb (all of them when one
+      // pass serves the query), or more while the rows' keys stay within
+      // kCoarseKeyBytes.  The coarse kernels keep no query rows in LDS, and
+      // a launch over few rows is all latency (200 positions of 28 heads
+      // over 1,024 pages in 8 passes: scan 110 us and select 55 us; in one
+      // pass of kScanRowsPerSlice rows a block 20 and 30 us).
+      const int64_t q_keys = (int64_t)B * hq * ld * 4;  // bytes of one position's keys
+      const int Qc = passes == 1 ? Q : (int)std::min<int64_t>(Q, std::max<int64_t>(Qb, kCoarseKeyBytes / q_keys));
+      const int rows_pass = B * hq * Qc;
       if ((rc = s->coarse_keys.ensure((size_t)rows_pass * ld * 4, st, false))) return rc;
       if ((rc = s->row_pages.ensure((size_t)rows * kc * 4, st, false))) return rc;
       if ((rc = s->page_list.ensure((size_t)N * 4, st, false))) return rc;
@@ -2732,29 +2750,33 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
       const bool mfma = dt != KIV_DTYPE_F32 && D % 32 == 0 && (kt <= 4 || kt == 6 || kt == 8 || kt == 16) &&
                         s->summ_dim == D;
       int row0 = 0;
-      for (int pass = 0; pass < passes; ++pass) {
-        const int Qp = std::min(Qb, Q - pass * Qb);
+      for (int pos0 = 0; pos0 < Q; pos0 += Qc) {
+        const int Qp = std::min(Qc, Q - pos0);
         const int rows_p = B * hq * Qp;
-        const char *qp = (const char *)a->q + pass * qstep;
+        const char *qp = (const char *)a->q + (int64_t)pos0 * a->q_stride[2] * eb;
         // The step's evicted rows ride on the first pass's launch.
         AppendRows apass{};
-        if (pass == 0) apass = ap;
+        if (pos0 == 0) apass = ap;
         const int extra = apass.count > 0 || apass.hot_count > 0 ? 1 : 0;
         s->prof_begin(KIV_STAGE_COARSE_SCAN, st);
         if (mfma) {
           const int pages_per_block = (kScanMfmaThreads / 64) * kScanMfmaPages;
           const int blocks = (int)(((int64_t)N + pages_per_block - 1) / pages_per_block);
+          const int zrows = pr.ub ? G * Qp : std::min(G * Qp, kScanRowsPerSlice);
+          const unsigned zn = (unsigned)((G * Qp + zrows - 1) / zrows);
           rc = with_dt(dt, [&](auto dtc) {
             constexpr int DTV = decltype(dtc)::value;
             if constexpr (DTV == DT_F32) {
               return (int)KIV_ERR_UNSUPPORTED;
             } else {
               return with_kt(kt, [&](auto ktc) {
-                hipLaunchKernelGGL((coarse_scan_mfma_kernel<DTV, decltype(ktc)::value>),
-                                   dim3(blocks + extra, s->kr), dim3(kScanMfmaThreads), 0, st, (const char *)s->summ.ptr,
-                                   (int64_t)N, s->kr, qp, a->q_stride[0], a->q_stride[1], a->q_stride[2], hq, hkv,
-                                   Qp, a->scaling, round, (uint32_t *)s->coarse_keys.ptr, ld,
-                                   (const float *)s->radius.ptr, (uint32_t *)pr.ub, (uint32_t *)pr.lb, pr.ctl, apass);
+                constexpr int KTV = decltype(ktc)::value;
+                auto kern = zn > 1 ? coarse_scan_mfma_kernel<DTV, KTV, true> : coarse_scan_mfma_kernel<DTV, KTV, false>;
+                hipLaunchKernelGGL(kern, dim3(blocks + extra, s->kr, zn), dim3(kScanMfmaThreads), 0, st,
+                                   (const char *)s->summ.ptr, (int64_t)N, s->kr, qp, a->q_stride[0], a->q_stride[1],
+                                   a->q_stride[2], hq, hkv, Qp, a->scaling, round, (uint32_t *)s->coarse_keys.ptr, ld,
+                                   (const float *)s->radius.ptr, (uint32_t *)pr.ub, (uint32_t *)pr.lb, pr.ctl, apass,
+                                   zrows);
                 return (int)KIV_OK;
               });
             }

@@ -953,3 +953,37 @@ def test_long_query_retrieval(cuda, name, w, batch, positions):
     q = (q + 0.2 * torch.randn(q.shape, generator=g)).to(w.dtype)
     store, oracle, cfg = build(w, data, cuda)
     check_retrieval(store, oracle, cfg, w, data, q)
+
+
+LONG_EDGES = [
+    # name, workload, batch, positions
+    # the query's coarse keys (4,100 rows of 4,200 pages) pass the limit of one coarse pass.
+    # fp16: a segment's 128 two-token pages spread a row's scores over about 6 * 0.3 / sqrt(2) = 1.3,
+    # 0.01 apart, and one rounding step at a score of 5 is 0.03 in bf16 (nearly every row's
+    # boundary is a tie: 14% of rows determined) but 0.004 in fp16
+    ("two_coarse_passes", Workload("le1", 4, 2, 32, torch.float16, hot=16, cold=8400 + 1, top_pages=32, top_p=64,
+                                   segment=256, page_size=2), 1, 1025),
+    # row counts one past and one short of the scans' 16- and 64-row tiles, pages off 16 tokens
+    ("rows_65_page_24_d96", Workload("le2", 10, 2, 96, torch.float16, hot=16, cold=3000 + 7, top_pages=64, top_p=150,
+                                     segment=256, page_size=24), 1, 13),
+    ("rows_63_page_128", Workload("le3", 28, 4, 128, torch.bfloat16, hot=16, cold=128 * 40 + 5, top_pages=40,
+                                  top_p=256, segment=512), 1, 9),
+    ("d256_batch2_page_64", Workload("le4", 4, 1, 256, torch.bfloat16, hot=16, cold=64 * 60 + 63, top_pages=30,
+                                     top_p=100, segment=512, page_size=64), 2, 40),
+    ("d192_one_candidate_tile", Workload("le5", 32, 1, 192, torch.float16, hot=16, cold=16 * 15 + 15, top_pages=15,
+                                         top_p=200, segment=64, page_size=16), 1, 18),
+]
+
+
+@pytest.mark.parametrize("tier", ["host", "hbm"])
+@pytest.mark.parametrize("name,w,batch,positions", LONG_EDGES, ids=[c[0] for c in LONG_EDGES])
+def test_long_query_edges(cuda, name, w, batch, positions, tier):
+    """Long queries at the edges of the scans' tiles and passes, against the
+    oracle's bar, twice in a row (keys left behind would show in the second)."""
+    data = generate(w, seed=17, batch=batch)
+    g = torch.Generator().manual_seed(18)
+    store, oracle, cfg = build(w, data, cuda, cold_tier=tier)
+    for call in range(2):
+        q = data["q"].float().repeat(1, 1, positions, 1)
+        q = (q + 0.2 * torch.randn(q.shape, generator=g)).to(w.dtype)
+        check_retrieval(store, oracle, cfg, w, data, q, min_det_c=0.3)
