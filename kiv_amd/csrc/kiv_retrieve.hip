@@ -2006,8 +2006,7 @@ __global__ void __launch_bounds__(256) fine_scan_mfma_kernel(
     int partial_len, int page_size, int tpi, int hkv, const char *__restrict__ q, int64_t qs0,
     int64_t qs1, int64_t qs2, int hq, int qlen, float scale, int round, uint32_t *__restrict__ out, int64_t ld,
     const float *__restrict__ coarse_stats, int rows, int n_pages, int32_t *pages_out, int32_t *union_out,
-    float *stats_out, double *stats_accum, char *__restrict__ k_stage, const char *__restrict__ k_read,
-    SelectPlan sp) {
+    float *stats_out, double *stats_accum, char *__restrict__ k_stage, SelectPlan sp) {
   static_assert(DT != DT_F32, "16-bit dtypes only");
   constexpr int D = 32 * KT, CPR = D / 8, ROW = D + 8;  // LDS rows padded by 16 bytes
   extern __shared__ uint4 smem4[];
@@ -2072,7 +2071,6 @@ __global__ void __launch_bounds__(256) fine_scan_mfma_kernel(
       cand0 = (int64_t)U * page_size + (int64_t)sp * tpi;
       ntok = min(tpi, partial_len - sp * tpi);
     }
-    if (k_read) rowbase = k_read + ((int64_t)r * ld + cand0) * row_bytes;
     __syncthreads();  // the previous item's reads of tk are done
     for (int i = tid; i < kFineMfmaTok * CPR; i += 256) {
       const int t = i / CPR, c = i % CPR;
@@ -2104,6 +2102,120 @@ __global__ void __launch_bounds__(256) fine_scan_mfma_kernel(
     const int t = 16 * wave + col;
     if (grp == 0 && t < ntok)
       atomicMax(&out[(int64_t)b * ld + cand0 + t], order_key(score_of<DT>(best, scale, round != 0)));
+  }
+}
+
+// Fine scan of a long query in one pass: every query row against tokens
+// held in registers.  The scans above keep a pass's query rows in LDS and
+// stream K, so a query of many positions reads K once per pass and each
+// wave's 16 tokens take a whole operand read from LDS per matrix
+// instruction (query of 200 positions over 131k candidates: 8 passes, 605
+// us, 310 TFLOP/s).  Here the roles are turned: block (x, r) takes
+// candidates [x * kFqTok, ...) of kv row r, wave w 16 * NT of them as the
+// NT B operands it keeps for the whole kernel (loaded once, straight from
+// memory: lane l holds dims 32 s + 8 (l / 16) .. + 7 of token l % 16), and
+// the query rows come through LDS in chunks of RC, double-buffered, the
+// next chunk's loads in flight while one is scored; one operand read feeds
+// NT matrix instructions.  Rows past the last repeat it, which changes no
+// maximum.  Bound by the matrix units: 2 * D operations per (token, row);
+// the query above takes 197 us, 950 TFLOP/s (an 8192^3 library product
+// reaches 1,225 on the same card).
+// Candidates are the union pages' tokens and then the partial page's, so
+// any page size fits the tiles.  The same instructions in the same order
+// over D as fine_scan_mfma_kernel: the same scores bit for bit.
+template <int KT> struct FqShape {
+  static constexpr int NT = KT <= 4 ? 4 : 2;   // token groups of 16 per wave (16 * NT * KT operand VGPRs / 4)
+  static constexpr int RC = KT <= 4 ? 64 : 32;  // query rows per LDS chunk
+  static constexpr int TOK = 4 * 16 * NT;       // candidates per block
+};
+
+template <int DT, int KT>
+__global__ void __launch_bounds__(256) fine_scan_query_kernel(
+    const int32_t *__restrict__ page_list, const int32_t *__restrict__ counters, int has_pages,
+    const uint64_t *__restrict__ ktab, int chunk_shift, int64_t page_bytes, const char *__restrict__ part_k,
+    int partial_len, int page_size, int hkv, const char *__restrict__ q, int64_t qs0, int64_t qs1, int64_t qs2, int hq,
+    int qlen, float scale, int round, uint32_t *__restrict__ out, int64_t ld, const char *__restrict__ k_read) {
+  static_assert(DT != DT_F32, "16-bit dtypes only");
+  using S = FqShape<KT>;
+  constexpr int NT = S::NT, RC = S::RC, D = 32 * KT, CPR = D / 8, ROW = D + 8;  // LDS rows padded by 16 bytes
+  constexpr int PJ = (RC * CPR + 255) / 256;  // chunk loads per thread
+  constexpr int64_t row_bytes = (int64_t)D * 2;
+  __shared__ __align__(16) uint16_t qs[2][RC * ROW];
+  const int r = blockIdx.y, b = r / hkv, kvh = r % hkv;
+  const int G = hq / hkv, GQ = G * qlen;
+  const int split = (has_pages ? counters[0] : 0) * page_size, n = split + partial_len;
+  const int c0 = blockIdx.x * S::TOK;
+  if (c0 >= n) return;  // block-uniform
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 15, grp = lane >> 4;
+  uint4 qreg[PJ];
+  auto load_q = [&](int j0) {
+#pragma unroll
+    for (int i = 0; i < PJ; ++i) {
+      const int at = tid + i * 256, c = at % CPR;
+      const int j = min(j0 + at / CPR, GQ - 1);
+      const int g = j / qlen, qp = j - g * qlen;
+      qreg[i] = load16(q + ((int64_t)b * qs0 + (int64_t)(kvh * G + g) * qs1 + (int64_t)qp * qs2 + c * 8) * 2);
+    }
+  };
+  load_q(0);
+  // This wave's tokens (those past the last candidate repeat it).
+  uint4 kb[NT][KT];
+#pragma unroll
+  for (int g = 0; g < NT; ++g) {
+    const int cand = min(c0 + (wave * NT + g) * 16 + col, n - 1);
+    const char *row;
+    if (k_read) {
+      row = k_read + ((int64_t)r * ld + cand) * row_bytes;
+    } else if (cand < split) {
+      const int v = cand / page_size, t = cand - v * page_size;
+      const int64_t page = page_list[v];
+      row = reinterpret_cast<const char *>(ktab[page >> chunk_shift]) +
+            (page & ((int64_t(1) << chunk_shift) - 1)) * page_bytes + ((int64_t)r * page_size + t) * row_bytes;
+    } else {
+      row = part_k + ((int64_t)r * page_size + (cand - split)) * row_bytes;
+    }
+#pragma unroll
+    for (int st = 0; st < KT; ++st) kb[g][st] = load16(row + (32 * st + 8 * grp) * 2);
+  }
+  float best[NT];
+#pragma unroll
+  for (int g = 0; g < NT; ++g) best[g] = -INFINITY;
+  int buf = 0;
+  for (int j0 = 0; j0 < GQ; j0 += RC, buf ^= 1) {
+    // A buffer is rewritten two chunks after its reads, which every wave
+    // has finished before the barrier in between.
+#pragma unroll
+    for (int i = 0; i < PJ; ++i) {
+      const int at = tid + i * 256;
+      if (PJ * 256 == RC * CPR || at < RC * CPR)
+        *reinterpret_cast<uint4 *>(&qs[buf][(at / CPR) * ROW + (at % CPR) * 8]) = qreg[i];
+    }
+    if (j0 + RC < GQ) load_q(j0 + RC);
+    __syncthreads();
+    const int nt = min(RC, GQ - j0);
+    for (int rt = 0; rt < nt; rt += 16) {
+      uint4 a[KT];
+#pragma unroll
+      for (int st = 0; st < KT; ++st)
+        a[st] = *reinterpret_cast<const uint4 *>(&qs[buf][(rt + col) * ROW + 32 * st + 8 * grp]);
+      f32x4_t acc[NT];
+#pragma unroll
+      for (int g = 0; g < NT; ++g) acc[g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int st = 0; st < KT; ++st)
+#pragma unroll
+        for (int g = 0; g < NT; ++g) acc[g] = mfma_16x16x32<DT>(a[st], kb[g][st], acc[g]);
+#pragma unroll
+      for (int g = 0; g < NT; ++g)
+        best[g] = fmaxf(best[g], fmaxf(fmaxf(acc[g][0], acc[g][1]), fmaxf(acc[g][2], acc[g][3])));
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < NT; ++g) {
+    const float m = half_wave_max(row_pair_max(best[g]));
+    const int cand = c0 + (wave * NT + g) * 16 + col;
+    if (grp == 0 && cand < n)
+      atomicMax(&out[(int64_t)b * ld + cand], order_key(score_of<DT>(m, scale, round != 0)));
   }
 }
 
@@ -2979,8 +3091,16 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
     // The select's page plan (one pass, so the bounds cover every query row).
     SelectPlan sp{};
     if (sel_plan) sp = SelectPlan{pr.ub, pr.lb, s->kr, a->out_width, pr.thr, pr.plan, pr.ctl};
-    for (int pass = 0; pass < passes && mfma; ++pass) {
-      const int Qp = std::min(Qb, Q - pass * Qb);
+    // A long query's union list (kFineMfmaRows query rows per kv row and up,
+    // no page plan) is scored in one pass by fine_scan_query_kernel.  Where
+    // K comes from host memory and is staged, the first pass's scan still
+    // streams it (whole rows a wave; it writes the staging copy) and the
+    // other positions read the copy.
+    // (Several passes imply a union list and more than kFineMfmaRows rows.)
+    const bool query_scan = mfma && union_src == UNION_LIST && !sel_plan && G * Q >= kFineMfmaRows;
+    const int first_q = mfma && (!query_scan || k_stage) ? std::min(Qb, Q) : 0;  // positions of the first scan
+    if (first_q > 0) {
+      const int Qp = first_q;
       const int gq16 = (G * Qp + 15) & ~15;
       const size_t lds = ((size_t)gq16 + kFineMfmaTok) * (D + 8) * 2 + (size_t)bwords * 4 + upage_bytes;
       s->prof_begin(KIV_STAGE_FINE_SCAN, st);
@@ -3003,11 +3123,38 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
                                  (const int32_t *)s->row_pages.ptr, rows * kc, bwords, (int32_t *)s->page_list.ptr,
                                  (int32_t *)s->counters.ptr, (const uint64_t *)s->k_tab.ptr, s->chunk_shift,
                                  s->page_bytes, (const char *)s->k_part.ptr, (int)s->partial_len, ps, tpi, hkv,
-                                 (const char *)a->q + pass * qstep, a->q_stride[0], a->q_stride[1],
-                                 a->q_stride[2], hq, Qp, a->scaling, round, (uint32_t *)s->fine_keys.ptr, ldc,
-                                 (const float *)coarse_stats, rows, N, a->pages_out, a->union_count_out,
-                                 a->stats_out, a->stats_accum, pass == 0 ? k_stage : nullptr,
-                                 pass == 0 ? nullptr : k_stage, sp);
+                                 (const char *)a->q, a->q_stride[0], a->q_stride[1], a->q_stride[2], hq, Qp,
+                                 a->scaling, round, (uint32_t *)s->fine_keys.ptr, ldc, (const float *)coarse_stats,
+                                 rows, N, a->pages_out, a->union_count_out, a->stats_out, a->stats_accum, k_stage, sp);
+              return (int)KIV_OK;
+            }
+          });
+        }
+      });
+      s->prof_end(KIV_STAGE_FINE_SCAN, st);
+      if (rc) return rc;
+      KIV_HIP(hipGetLastError());
+    }
+    if (query_scan && first_q < Q) {
+      s->prof_begin(KIV_STAGE_FINE_SCAN, st);
+      rc = with_dt(dt, [&](auto dtc) {
+        constexpr int DTV = decltype(dtc)::value;
+        if constexpr (DTV == DT_F32) {
+          return (int)KIV_ERR_UNSUPPORTED;
+        } else {
+          return with_kt(kt, [&](auto ktc) {
+            constexpr int KTV = decltype(ktc)::value;
+            if constexpr (KTV == 16) {
+              return (int)KIV_ERR_UNSUPPORTED;
+            } else {
+              const unsigned blocks = (unsigned)((cmax + FqShape<KTV>::TOK - 1) / FqShape<KTV>::TOK);
+              hipLaunchKernelGGL((fine_scan_query_kernel<DTV, KTV>), dim3(blocks, (unsigned)s->kr), dim3(256), 0, st,
+                                 (const int32_t *)s->page_list.ptr, (const int32_t *)s->counters.ptr, N > 0 ? 1 : 0,
+                                 (const uint64_t *)s->k_tab.ptr, s->chunk_shift, s->page_bytes,
+                                 (const char *)s->k_part.ptr, (int)s->partial_len, ps, hkv,
+                                 (const char *)a->q + (int64_t)first_q * a->q_stride[2] * eb, a->q_stride[0],
+                                 a->q_stride[1], a->q_stride[2], hq, Q - first_q, a->scaling, round,
+                                 (uint32_t *)s->fine_keys.ptr, ldc, (const char *)k_stage);
               return (int)KIV_OK;
             }
           });
