@@ -201,6 +201,15 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   return max(t[0], t[1]);
 }
 
+// Maximum over each row of 16 lanes; every lane of the row gets it.  All 64
+// lanes must be active.
+__device__ __forceinline__ uint32_t row_max_u32(uint32_t v) {
+  v = max(v, (uint32_t)dpp_i32<0xB1>((int)v));
+  v = max(v, (uint32_t)dpp_i32<0x4E>((int)v));
+  v = max(v, (uint32_t)dpp_i32<0x141>((int)v));
+  return max(v, (uint32_t)dpp_i32<0x140>((int)v));
+}
+
 // Number of set bits of a wave mask below the calling lane.
 __device__ __forceinline__ int lane_rank(uint64_t mask) {
   return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));

@@ -113,7 +113,8 @@ struct kiv_store {
   kiv::DevBuf page_list;     // [N] i32 union pages ascending
   kiv::DevBuf union_bits;    // [ceil(N/32)] u32 page bitmap of long row lists, zero between calls
   kiv::DevBuf counters;      // i32: [0] = U, the union size of the last coarse pass
-  kiv::DevBuf fine_keys;     // [B][ld] u32
+  kiv::DevBuf fine_keys;     // [B][ld] u32 (+ [B][ld / 16] group maxima), zero between calls
+  kiv::DevBuf fine_vals;     // the same of a scan that stores every key (decode with K in HBM)
   kiv::DevBuf sel_list;      // [B][list_ld] u64 top-P' candidates + [B] i32 counts
   kiv::DevBuf k_stage;       // [B*Hkv][ld][D] candidates' K rows (host tier)
   kiv::DevBuf prune;         // pruned fine scan: control, [B] thresholds, [N][kr] upper and lower bound keys

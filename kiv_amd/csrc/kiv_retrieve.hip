@@ -46,6 +46,7 @@ constexpr int kScanRowsPerSlice = 64;  // query rows per grid-z slice of the MFM
 constexpr int64_t kCoarseKeyBytes = int64_t(64) << 20;  // coarse keys of one pass of a long query
 constexpr int kSelThreads = 512;       // select block (8 waves)
 constexpr int kWideSelThreads = 1024;  // fine select block for rows of many candidates (16 waves)
+constexpr int64_t kWideSelKeys = 4 * 4 * kSelThreads;  // candidates past which a row's select is wide
 constexpr int kMaxWords = 4096;     // bitmap words ranked in LDS (131072 pages)
 constexpr int kCandCap = 2048;      // candidates a select keeps in LDS
 constexpr int kRankCap = 1024;      // candidates a coarse select ranks by counting in one block
@@ -369,8 +370,7 @@ template <int NT> struct MemKeys4 {
 // sum and the number of scored entries in nz: a zero key is an entry that
 // was not scored (a pruned fine scan leaves them) and is not summed.
 template <int NT, typename Src>
-__device__ int bound_candidates(const Src &src, int k, SelSh<NT> &sh, uint64_t *cand, float &mx, float &sum,
-                                int &nz) {
+__device__ uint32_t row_bound(const Src &src, int k, SelSh<NT> &sh, float &mx, float &sum, int &nz) {
   constexpr int W = NT / 64;
   const int tid = threadIdx.x, wave = tid >> 6;
   uint32_t m[4] = {0u, 0u, 0u, 0u};
@@ -411,6 +411,13 @@ __device__ int bound_candidates(const Src &src, int k, SelSh<NT> &sh, uint64_t *
     nz += sh.fcnt[w];
     bound = min(bound, sh.wave_bound[w]);
   }
+  return bound;
+}
+// The composites of keys >= bound into cand[] (at most cap); returns their
+// number.
+template <int NT, typename Src>
+__device__ int place_candidates(const Src &src, uint32_t bound, SelSh<NT> &sh, uint64_t *cand, int cap) {
+  const int tid = threadIdx.x;
   if constexpr (Src::kManySteps) {
     // Many register steps per thread: a first pass sums the steps' ballot
     // counts, one LDS atomic per wave reserves the wave's range, a second
@@ -429,17 +436,23 @@ __device__ int bound_candidates(const Src &src, int k, SelSh<NT> &sh, uint64_t *
         const uint64_t mask = __ballot(f);
         if (f) {
           const int pos = off + lane_rank(mask);
-          if (pos < kCandCap) cand[pos] = x;
+          if (pos < cap) cand[pos] = x;
         }
         off += __popcll(mask);
       });
     }
   } else {
     block_compact<NT>(src, [bound](uint64_t x) { return comp_key(x) >= bound; },
-                      [cand](int pos, uint64_t x) { cand[pos] = x; }, kCandCap, &sh.ncand);
+                      [cand](int pos, uint64_t x) { cand[pos] = x; }, cap, &sh.ncand);
   }
   __syncthreads();
   return sh.ncand;
+}
+template <int NT, typename Src>
+__device__ int bound_candidates(const Src &src, int k, SelSh<NT> &sh, uint64_t *cand, float &mx, float &sum,
+                                int &nz) {
+  const uint32_t bound = row_bound<NT>(src, k, sh, mx, sum, nz);
+  return place_candidates<NT>(src, bound, sh, cand, kCandCap);
 }
 
 // Calls ranked(x, r) for each of the top k composites of the C candidates
@@ -1150,6 +1163,12 @@ __global__ void __launch_bounds__(NT) coarse_select_tables_kernel(const uint32_t
 // (1024 blocks x ~2 KiB slices: 55 GB/s; 8 MiB in flight: 51 GB/s, 16 MiB:
 // 49 GB/s); HBM rows best in 32-token slices over 2048 blocks.
 constexpr int kFineUT = 4;  // tokens in flight per lane group
+// Group maxima (the wide fine select): with gmax set, a matrix-core scan
+// also leaves the largest key of every kGroupKeys consecutive candidates
+// ([B][ldg]; one 64-byte line of keys a group).  The vector scan does not:
+// its one more atomic a token costs more than the select gains (fp32 rows,
+// 16 heads over 47k candidates: scan 37 -> 60 us, select 21 -> 9).
+constexpr int kGroupKeys = 16;
 
 // Block (0, 0) of a fresh union: page_list / pages_out <- the union pages
 // ascending, counters[0] / union_out <- U, and the coarse telemetry.
@@ -2006,7 +2025,8 @@ __global__ void __launch_bounds__(256) fine_scan_mfma_kernel(
     int partial_len, int page_size, int tpi, int hkv, const char *__restrict__ q, int64_t qs0,
     int64_t qs1, int64_t qs2, int hq, int qlen, float scale, int round, uint32_t *__restrict__ out, int64_t ld,
     const float *__restrict__ coarse_stats, int rows, int n_pages, int32_t *pages_out, int32_t *union_out,
-    float *stats_out, double *stats_accum, char *__restrict__ k_stage, SelectPlan sp) {
+    float *stats_out, double *stats_accum, char *__restrict__ k_stage, SelectPlan sp, uint32_t *__restrict__ gmax,
+    int64_t ldg) {
   static_assert(DT != DT_F32, "16-bit dtypes only");
   constexpr int D = 32 * KT, CPR = D / 8, ROW = D + 8;  // LDS rows padded by 16 bytes
   extern __shared__ uint4 smem4[];
@@ -2100,8 +2120,163 @@ __global__ void __launch_bounds__(256) fine_scan_mfma_kernel(
     }
     best = half_wave_max(row_pair_max(best));
     const int t = 16 * wave + col;
-    if (grp == 0 && t < ntok)
-      atomicMax(&out[(int64_t)b * ld + cand0 + t], order_key(score_of<DT>(best, scale, round != 0)));
+    const uint32_t key = t < ntok ? order_key(score_of<DT>(best, scale, round != 0)) : 0u;
+    if (grp == 0 && t < ntok) atomicMax(&out[(int64_t)b * ld + cand0 + t], key);
+    if (gmax) {
+      const uint32_t top = row_max_u32(key);
+      if (lane == 0) atomicMax(&gmax[(int64_t)b * ldg + (cand0 + 16 * wave) / kGroupKeys], top);
+    }
+  }
+}
+
+// Fine scan of a decode step over K in HBM, without atomics: block (x, b)
+// takes tiles of 16 candidates of batch row b and every kv head of them, so
+// that a candidate's key, the maximum over the heads, is complete in the
+// block and is stored once (as is its group's maximum).  The block's four
+// waves are HW heads by 4 / HW tiles; a wave walks its heads h0, h0 + HW,
+// ..., the next head's rows in flight while one is scored, and the maxima
+// of the HW waves meet in LDS.  Pages are whole tiles, so a tile's K rows
+// of one head are one contiguous run, read 1 KiB an instruction and turned
+// into the B operand (lane l: dims 32 s + 8 (l / 16) .. + 7 of token l %
+// 16) through LDS of the wave's own, without a barrier; reading the operand
+// straight from memory touches 16 rows an instruction and was slower where
+// K comes from the caches.  Against fine_scan_mfma_kernel (one kv row a
+// block, K through LDS behind two barriers an item, an atomic per candidate
+// and head on keys that must start at zero): bound by HBM where K is large
+// (64 kv rows of head_dim 96, 403 MB of K: 102 -> 86 us, 4.7 TB/s; 21 MB:
+// 9.7 -> 9.4; 24 MB at 2 kv heads: 9.1 both, where the union's prologue and
+// the round trips are most of it).
+// Candidates are the union pages' tokens, then the partial page's; a tile's
+// places past the last candidate (rows of the partial page's buffer not yet
+// written) store zero keys.
+template <int DT, int KT>
+__global__ void __launch_bounds__(256) fine_scan_heads_kernel(
+    int union_src, const int32_t *__restrict__ row_pages, int row_pages_n, int words, int32_t *page_list,
+    int32_t *counters, const uint64_t *__restrict__ ktab, int nchunks, int chunk_shift, int64_t page_bytes,
+    const char *__restrict__ part_k, int partial_len, int page_size, int hkv, int hw, const char *__restrict__ q,
+    int64_t qs0, int64_t qs1, int64_t qs2, int hq, int qlen, float scale, int round, uint32_t *__restrict__ out,
+    int64_t ld, const float *__restrict__ coarse_stats, int rows, int n_pages, int32_t *pages_out, int32_t *union_out,
+    float *stats_out, double *stats_accum, SelectPlan sp, uint32_t *__restrict__ gmax, int64_t ldg) {
+  static_assert(DT != DT_F32, "16-bit dtypes only");
+  constexpr int D = 32 * KT, ROW = D + 8;  // LDS rows padded by 16 bytes
+  constexpr int64_t row_bytes = (int64_t)D * 2;
+  extern __shared__ uint4 smem4[];
+  __shared__ int scan_tmp[4];
+  __shared__ float part[2][4][16];
+  __shared__ __align__(16) uint16_t kt[4][16 * ROW];  // a wave's tile of K rows
+  const int b = blockIdx.y, G = hq / hkv, GQ = G * qlen;
+  uint32_t *ubits = reinterpret_cast<uint32_t *>(smem4);
+  int *upage = reinterpret_cast<int *>(ubits + words);  // row lists: the union pages
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int col = lane & 15, grp = lane >> 4;
+  const int h0 = wave % hw, tw = wave / hw, tiles_per_block = 4 / hw;  // hw: 1, 2 or 4
+  // The chunk bases, one a lane (read from memory past 64 chunks).
+  const bool tab_lanes = nchunks <= 64;
+  const uint64_t kt_lane = tab_lanes && lane < nchunks ? ktab[lane] : 0;
+  // Query rows 16 m .. + 15 of kv head kvh (rows past the last repeat it,
+  // which changes no maximum).
+  auto load_q = [&](int kvh, int m, uint4 (&qa)[KT]) {
+    const int j = min(16 * m + col, GQ - 1), g = j / qlen, qp = j - g * qlen;
+    const char *qr = q + ((int64_t)b * qs0 + (int64_t)(kvh * G + g) * qs1 + (int64_t)qp * qs2) * 2 + grp * 16;
+#pragma unroll
+    for (int st = 0; st < KT; ++st) qa[st] = load16(qr + st * 64);
+  };
+  uint4 qa[KT];
+  load_q(min(h0, hkv - 1), 0, qa);
+  int U = 0;
+  if (union_src == UNION_ROWS) {
+    U = rank_union<256>(row_pages, row_pages_n, words, ubits, upage, scan_tmp);
+    if (blockIdx.x == 0 && b == 0)
+      publish_union<DT>(upage, U, page_list, pages_out, counters, union_out, coarse_stats, rows, n_pages, round,
+                        stats_out, stats_accum);
+  } else if (union_src == UNION_LIST) {
+    U = counters[0];
+  }
+  auto page_of = [&](int v) -> int64_t { return union_src == UNION_ROWS ? upage[v] : page_list[v]; };
+  const int nscan = sp.plan ? (int)gridDim.x - 1 : (int)gridDim.x;
+  if ((int)blockIdx.x >= nscan) {
+    __shared__ SelSh<256> tsh;
+    select_plan<256>(sp, b, hkv, U, page_size, partial_len, page_of, tsh, scan_tmp);
+    return;
+  }
+  const int split = U * page_size, n = split + partial_len, tiles = (n + 15) >> 4;
+  const int64_t head_bytes = (int64_t)page_size * row_bytes;  // between a token's rows of two kv heads
+  const int hpw = (hkv + hw - 1) / hw;                        // head steps a wave
+  // K rows of a tile, kv head 0 of batch row b (wave-uniform).
+  auto tile_rows = [&](int tile) -> const char * {
+    const int cand = 16 * tile;
+    const int64_t r0 = (int64_t)b * hkv;
+    if (cand >= split) return part_k + (r0 * page_size + (cand - split)) * row_bytes;
+    const int v = cand / page_size, t = cand - v * page_size;
+    const int64_t page = (int64_t)uniform_u32((uint32_t)page_of(v));
+    const int chunk = (int)(page >> chunk_shift);
+    const uint64_t base = tab_lanes ? ((uint64_t)__builtin_amdgcn_readlane((uint32_t)(kt_lane >> 32), chunk) << 32) |
+                                          (uint32_t)__builtin_amdgcn_readlane((uint32_t)kt_lane, chunk)
+                                    : ktab[chunk];
+    return reinterpret_cast<const char *>(base) + (page & ((int64_t(1) << chunk_shift) - 1)) * page_bytes +
+           (r0 * page_size + t) * row_bytes;
+  };
+  const char *rows0 = nullptr;
+  auto load_k = [&](int step, uint4 (&x)[KT]) {  // head step of the tile at rows0 (past the last head: the last)
+    const char *at = rows0 + (int64_t)min(h0 + step * hw, hkv - 1) * head_bytes + lane * 16;
+#pragma unroll
+    for (int i = 0; i < KT; ++i) x[i] = load16(at + i * 1024);
+  };
+  uint16_t *mine = kt[wave];
+  int buf = 0;
+  uint4 kn[KT];
+  const int stride = nscan * tiles_per_block, t0 = blockIdx.x * tiles_per_block;
+  // The tile loop is block-uniform (its barrier); a wave whose tile is past
+  // the last works on the last one and stores nothing.
+  if (t0 < tiles) {
+    rows0 = tile_rows(min(t0 + tw, tiles - 1));
+    load_k(0, kn);
+  }
+  for (int tb = t0; tb < tiles; tb += stride, buf ^= 1) {
+    const int tile = tb + tw;
+    float best = -INFINITY;
+    for (int step = 0; step < hpw; ++step) {
+      // Piece i of lane l is chunk 64 i + l of the run.
+#pragma unroll
+      for (int i = 0; i < KT; ++i) {
+        const int f = 64 * i + lane;
+        *reinterpret_cast<uint4 *>(&mine[(f / (4 * KT)) * ROW + (f % (4 * KT)) * 8]) = kn[i];
+      }
+      // The next head's rows, or the next tile's first.
+      if (step + 1 < hpw) {
+        load_k(step + 1, kn);
+      } else if (tb + stride < tiles) {
+        rows0 = tile_rows(min(tb + stride + tw, tiles - 1));
+        load_k(0, kn);
+      }
+      uint4 kb[KT];
+#pragma unroll
+      for (int st = 0; st < KT; ++st) kb[st] = *reinterpret_cast<const uint4 *>(&mine[col * ROW + 32 * st + 8 * grp]);
+      const int kvh = min(h0 + step * hw, hkv - 1);
+      for (int m = 0; 16 * m < GQ; ++m) {
+        if (hpw > 1 || GQ > 16) load_q(kvh, m, qa);
+        f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int st = 0; st < KT; ++st) acc = mfma_16x16x32<DT>(qa[st], kb[st], acc);
+        best = fmaxf(best, fmaxf(fmaxf(acc[0], acc[1]), fmaxf(acc[2], acc[3])));
+      }
+    }
+    best = half_wave_max(row_pair_max(best));
+    if (hw > 1) {
+      // The buffer is rewritten two tiles later, past the next barrier.
+      if (lane < 16) part[buf][wave][lane] = best;
+      __syncthreads();
+      if (h0 == 0)
+        for (int w = 1; w < hw; ++w) best = fmaxf(best, part[buf][wave + w][col]);
+    }
+    if (h0 == 0 && tile < tiles) {
+      const uint32_t key = 16 * tile + col < n ? order_key(score_of<DT>(best, scale, round != 0)) : 0u;
+      if (lane < 16) out[(int64_t)b * ld + 16 * tile + col] = key;
+      if (gmax) {
+        const uint32_t top = row_max_u32(key);
+        if (lane == 0) gmax[(int64_t)b * ldg + tile] = top;
+      }
+    }
   }
 }
 
@@ -2134,7 +2309,8 @@ __global__ void __launch_bounds__(256) fine_scan_query_kernel(
     const int32_t *__restrict__ page_list, const int32_t *__restrict__ counters, int has_pages,
     const uint64_t *__restrict__ ktab, int chunk_shift, int64_t page_bytes, const char *__restrict__ part_k,
     int partial_len, int page_size, int hkv, const char *__restrict__ q, int64_t qs0, int64_t qs1, int64_t qs2, int hq,
-    int qlen, float scale, int round, uint32_t *__restrict__ out, int64_t ld, const char *__restrict__ k_read) {
+    int qlen, float scale, int round, uint32_t *__restrict__ out, int64_t ld, const char *__restrict__ k_read,
+    uint32_t *__restrict__ gmax, int64_t ldg) {
   static_assert(DT != DT_F32, "16-bit dtypes only");
   using S = FqShape<KT>;
   constexpr int NT = S::NT, RC = S::RC, D = 32 * KT, CPR = D / 8, ROW = D + 8;  // LDS rows padded by 16 bytes
@@ -2213,9 +2389,13 @@ __global__ void __launch_bounds__(256) fine_scan_query_kernel(
 #pragma unroll
   for (int g = 0; g < NT; ++g) {
     const float m = half_wave_max(row_pair_max(best[g]));
-    const int cand = c0 + (wave * NT + g) * 16 + col;
-    if (grp == 0 && cand < n)
-      atomicMax(&out[(int64_t)b * ld + cand], order_key(score_of<DT>(m, scale, round != 0)));
+    const int first = c0 + (wave * NT + g) * 16, cand = first + col;
+    const uint32_t key = cand < n ? order_key(score_of<DT>(m, scale, round != 0)) : 0u;
+    if (grp == 0 && cand < n) atomicMax(&out[(int64_t)b * ld + cand], key);
+    if (gmax) {
+      const uint32_t top = row_max_u32(key);
+      if (lane == 0 && first < n) atomicMax(&gmax[(int64_t)b * ldg + first / kGroupKeys], top);
+    }
   }
 }
 
@@ -2238,11 +2418,12 @@ __global__ void __launch_bounds__(256) fine_scan_query_kernel(
 // partial page, by the block's first NS threads (all of them, or the first
 // kSelThreads of a wide block, whose other waves have left: s_barrier waits
 // only for the waves still running).  Lists the candidates, clears the
-// keys (the whole row with zero_all) and writes the telemetry.
+// keys as `clear` says and writes the telemetry.
+enum { CLEAR_LISTED = 0, CLEAR_ROW = 1, CLEAR_NONE = 2 };
 template <int NS>
 __device__ __forceinline__ void select_listed_pages(uint32_t *row, const int *plist, int np, int page_size, int partial_len, int U,
-                                    int n, int k, int zero_all, SelSh<NS> &sh, uint64_t *cand, uint64_t *out,
-                                    int list_cap, float *fine_stats, int32_t *list_count, int b) {
+                                    int n, int k, int clear, SelSh<NS> &sh, uint64_t *cand, uint64_t *out,
+                                    int list_cap, float *fine_stats, int32_t *list_count, int b, int batch) {
   float mx, sum;
   int C, nz;
   const PageKeys<NS> pk{row, plist, np * page_size, np * page_size + partial_len, page_size,
@@ -2261,33 +2442,209 @@ __device__ __forceinline__ void select_listed_pages(uint32_t *row, const int *pl
     C = k;
   }
   __syncthreads();
-  if (zero_all) {  // a full scan wrote every key
+  if (clear == CLEAR_ROW) {  // a full scan wrote every key
     uint4 *row4 = reinterpret_cast<uint4 *>(row);
     for (int i = threadIdx.x; i < (n + 3) / 4; i += NS) row4[i] = make_uint4(0, 0, 0, 0);
-  } else {
+  } else if (clear == CLEAR_LISTED) {
     for (int e = threadIdx.x; e < pk.mall; e += NS) row[pk.index(e)] = 0u;
   }
   if (threadIdx.x == 0) {
     fine_stats[2 * b] = mx;
     fine_stats[2 * b + 1] = sum;
     list_count[b] = C;
-    list_count[gridDim.x + b] = nz;
+    list_count[batch + b] = nz;
   }
 }
 
+// The wide select (GR: rows that may hold more than 4 * 4 * kSelThreads
+// candidates, every candidate scored).  Reading the row through one block
+// is what bounds the plain select there: a compute unit takes the row's 64
+// KiB and up in, and every pass over its registers is a hundred ballots a
+// wave (20k keys 11.8 us, two rows of 33k 17, 46k 20, 131k 30; as below
+// 9.0, 12.5, 7.7 and 9.0 us).
+// The scan's group maxima (kGroupKeys candidates each) bound it with a
+// sixteenth of the reads: the k-th largest of the group maxima is at most
+// the row's k-th largest key (k groups hold a key at least as large), so
+// the block takes its bound B from the maxima and then reads the keys of
+// the groups that reach B alone.  Where those hold more than list_cap keys
+// >= B (clustered keys: the best candidates share groups), a second bound
+// over them, from the keys themselves, shortens the list.  A bound of 0, or
+// more groups or keys than fit, falls to the plain select.
+// The telemetry needs every score: blocks past the batch rows reduce one
+// segment of kSumKeys keys each (SegSum; the gather's telemetry block folds
+// them, nz = -1 says so), and keys and maxima that were folded with atomics
+// are cleared by blocks of the gather launch, a few KiB each, instead of by
+// this block (`keep` says that nothing is to be cleared: keys that
+// fine_scan_heads_kernel stored).
+constexpr int kSumKeys = 8192;       // keys per segment (summed or cleared by one block)
+constexpr int kGroupCap = 2048;      // groups the wide select lists
+constexpr int kGroupKeyCap = 6144;   // keys >= B it holds in LDS
+constexpr int kGroupChunks = 4;      // 16-byte chunks of group maxima per thread in registers
+struct SegSum {
+  float sum, max;
+  int32_t n, pad;
+};
+struct SelectGroups {
+  const uint32_t *gmax;
+  int64_t ldg;
+  SegSum *sums;  // [B][nseg]
+  int nseg, batch;
+};
+
+// Keys held in LDS as a select source (sub-slot: step & 3).
+template <int NT> struct LdsSlots {
+  static constexpr bool kManySteps = false;
+  const uint64_t *c;
+  int n;
+  template <typename F> __device__ void each_slot(F &&f) const {
+    int u = 0;
+    for (int i = threadIdx.x; i < n; i += NT, ++u) f(c[i], u & 3);
+  }
+  template <typename F> __device__ void each(F &&f) const {
+    each_slot([&](uint64_t x, int) { f(x); });
+  }
+};
+
+// Sum, maximum and number of the scored keys of one segment.
+template <int NT> __device__ void segment_sum(const uint32_t *row, int n, int seg, SegSum *out) {
+  __shared__ SegSum part[NT / 64];
+  const int first = seg * kSumKeys, tid = threadIdx.x;
+  const uint4 *row4 = reinterpret_cast<const uint4 *>(row + first);
+  const int n4 = max(0, min(kSumKeys, n - first) + 3) >> 2;  // keys past n are zero
+  float fs = 0.f;
+  uint32_t top = 0u;
+  int cnt = 0;
+#pragma unroll
+  for (int i = 0; i < kSumKeys / 4 / NT; ++i) {
+    const int c = tid + i * NT;
+    const uint4 x = c < n4 ? row4[c] : make_uint4(0, 0, 0, 0);
+    const uint32_t v[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      top = max(top, v[e]);
+      fs += v[e] ? key_to_float(v[e]) : 0.f;
+      cnt += v[e] != 0u;
+    }
+  }
+  fs = wave_sum(fs);
+  top = wave_max_u32(top);
+  cnt = wave_sum_i32(cnt);
+  if ((tid & 63) == 0) part[tid >> 6] = SegSum{fs, top ? key_to_float(top) : -INFINITY, cnt, 0};
+  __syncthreads();
+  if (tid != 0) return;
+  SegSum t = part[0];
+#pragma unroll
+  for (int w = 1; w < NT / 64; ++w) {
+    t.sum += part[w].sum;
+    t.max = fmaxf(t.max, part[w].max);
+    t.n += part[w].n;
+  }
+  *out = t;
+}
+
+// The wide select of one row: lists the candidates (see above) and returns
+// their number, or -1 when the plain select must run.
+template <int NT>
+__device__ int select_by_groups(const uint32_t *row, int n, int k, const uint32_t *gmax, SelSh<NT> &sh, int *gcnt,
+                                uint64_t *keys, int *glist, uint64_t *out, int list_cap) {
+  const int tid = threadIdx.x, ng = (n + kGroupKeys - 1) / kGroupKeys;
+  uint32_t bound;
+  if (ng <= 4 * kGroupChunks * NT) {
+    RegKeys4<NT, kGroupChunks> rk;
+    rk.load(gmax, ng);
+    bound = block_kth_bound<NT>(rk, k, sh);
+    if (bound == 0u) return -1;
+    block_compact<NT>(rk, [bound](uint64_t x) { return comp_key(x) >= bound; },
+                      [glist](int pos, uint64_t x) { glist[pos] = comp_index(x); }, kGroupCap, &gcnt[0]);
+  } else {
+    const MemKeys4<NT> mk{gmax, ng};
+    bound = block_kth_bound<NT>(mk, k, sh);
+    if (bound == 0u) return -1;
+    block_compact<NT>(mk, [bound](uint64_t x) { return comp_key(x) >= bound; },
+                      [glist](int pos, uint64_t x) { glist[pos] = comp_index(x); }, kGroupCap, &gcnt[0]);
+  }
+  __syncthreads();
+  const int groups = gcnt[0];
+  if (groups > kGroupCap) return -1;
+  // The listed groups' keys, 16 bytes a thread.
+  const uint4 *row4 = reinterpret_cast<const uint4 *>(row);
+  const int items = groups * (kGroupKeys / 4);
+  for (int base = 0; base < items; base += NT) {
+    const int it = base + tid;
+    const int c = it < items ? glist[it / (kGroupKeys / 4)] * (kGroupKeys / 4) + it % (kGroupKeys / 4) : 0;
+    const uint4 x = it < items ? row4[c] : make_uint4(0, 0, 0, 0);
+    const uint32_t v[4] = {x.x, x.y, x.z, x.w};
+    uint64_t m[4];
+    int total = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      m[e] = __ballot(v[e] >= bound);
+      total += __popcll(m[e]);
+    }
+    if (total) {
+      int off = 0;
+      if ((tid & 63) == 0) off = atomicAdd(&gcnt[1], total);
+      off = (int)uniform_u32((uint32_t)off);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int pos = off + lane_rank(m[e]);
+        if (v[e] >= bound && pos < kGroupKeyCap) keys[pos] = comp_of(v[e], 4 * c + e);
+        off += __popcll(m[e]);
+      }
+    }
+  }
+  __syncthreads();
+  const int C = gcnt[1];
+  if (C > kGroupKeyCap) return -1;
+  if (C <= list_cap) {
+    for (int i = tid; i < C; i += NT) out[i] = keys[i];
+    return C;
+  }
+  const LdsSlots<NT> ls{keys, C};
+  const uint32_t b2 = block_kth_bound<NT>(ls, k, sh);
+  block_compact<NT>(ls, [b2](uint64_t x) { return comp_key(x) >= b2; }, [out](int pos, uint64_t x) { out[pos] = x; },
+                    list_cap, &gcnt[2]);
+  __syncthreads();
+  if (gcnt[2] <= list_cap) return gcnt[2];
+  // Mass ties: exactly k.
+  const LdsComps<NT> lc{keys, C};
+  const uint64_t kth = block_kth<NT>(lc, k, sh);
+  block_compact<NT>(lc, [kth](uint64_t x) { return x >= kth; }, [out](int pos, uint64_t x) { out[pos] = x; }, k,
+                    &sh.nsel);
+  return k;
+}
+
 // V = 16-byte key chunks per thread kept in registers: rows of up to
-// 4 * V * NT keys are read once; longer rows are re-read.
-template <int V, int NT>
+// 4 * V * NT keys are read once; longer rows are re-read, as are the rows
+// of a wide select that falls to the plain one (V is not used there).  PL:
+// with the page bounds' path.
+template <int V, int NT, bool GR, bool PL>
 __global__ void __launch_bounds__(NT) fine_select_kernel(
     uint32_t *__restrict__ keys, int64_t ld, const int32_t *__restrict__ counters, int has_pages, int page_size,
     int partial_len, int width, float *__restrict__ fine_stats, uint64_t *__restrict__ list, int64_t list_ld,
     int32_t *__restrict__ list_count, int list_cap, const uint32_t *__restrict__ ub, int kr, int hkv,
     const uint32_t *__restrict__ thr, const int32_t *__restrict__ page_list, const int32_t *__restrict__ plan,
-    int zero_all, const int32_t *__restrict__ ctl) {
+    int zero_all, const int32_t *__restrict__ ctl, SelectGroups sg, int keep) {
   __shared__ SelSh<NT> sh;
   __shared__ SelSh<kSelThreads> sh_few;  // a wide block's few-page select
-  __shared__ uint64_t cand[kCandCap];
-  __shared__ int plist[kPageListCap];
+  // [cand][plist], or the wide select's [keys][groups] in the same place.
+  constexpr size_t kPlain = kCandCap * sizeof(uint64_t) + kPageListCap * sizeof(int);
+  constexpr size_t kWide = kGroupKeyCap * sizeof(uint64_t) + kGroupCap * sizeof(int);
+  __shared__ __align__(16) char pool[GR && kWide > kPlain ? kWide : kPlain];
+  __shared__ int gcnt[3];
+  uint64_t *cand = reinterpret_cast<uint64_t *>(pool);
+  int *plist = reinterpret_cast<int *>(cand + kCandCap);
+  const int U = has_pages ? counters[0] : 0;
+  const int n = U * page_size + partial_len;
+  const int batch = GR ? sg.batch : (int)gridDim.x;
+  if constexpr (GR) {
+    if ((int)blockIdx.x >= batch) {
+      const int i = blockIdx.x - batch, sb = i / sg.nseg, seg = i - sb * sg.nseg;
+      segment_sum<NT>(keys + (int64_t)sb * ld, n, seg, sg.sums + i);
+      return;
+    }
+    if (threadIdx.x < 3) gcnt[threadIdx.x] = 0;
+  }
   if (NT > kSelThreads && threadIdx.x == 0) {
     sh_few.cnt[0] = sh_few.cnt[1] = sh_few.cnt[2] = 0;
     sh_few.ncand = sh_few.nsel = 0;
@@ -2296,14 +2653,12 @@ __global__ void __launch_bounds__(NT) fine_select_kernel(
   }
   sel_init(sh);
   const int b = blockIdx.x;
-  const int U = has_pages ? counters[0] : 0;
-  const int n = U * page_size + partial_len;
   const int k = min(width, n);
   uint32_t *row = keys + (int64_t)b * ld;  // 256-byte aligned rows, zero past n
   uint64_t *out = list + (int64_t)b * list_ld;
   float mx, sum;
   int C, nz;
-  if (ub && *ctl <= 0) {  // not while pruning is paused (every key scored)
+  if (PL && ub && *ctl <= 0) {  // not while pruning is paused (every key scored)
     // Pruned fine scan: only the pages some kv row of b scanned (and the
     // partial page) hold nonzero keys; the others are not read.
     const uint32_t tb = thr[b];
@@ -2317,7 +2672,7 @@ __global__ void __launch_bounds__(NT) fine_select_kernel(
       np = planned;
       if ((int)threadIdx.x < min(np, kPageListCap)) plist[threadIdx.x] = first;
       for (int i = threadIdx.x + NT; i < min(np, kPageListCap); i += NT) plist[i] = pl[2 + i];
-      if (threadIdx.x == 0) list_count[2 * gridDim.x + b] = pl[1];
+      if (threadIdx.x == 0) list_count[2 * batch + b] = pl[1];
       __syncthreads();
     } else {
       int slices = 0;  // (page, kv row) slices the scan read, this thread's pages
@@ -2334,7 +2689,7 @@ __global__ void __launch_bounds__(NT) fine_select_kernel(
       if (threadIdx.x == 0) {
         int read = 0;
         for (int w = 0; w < NT / 64; ++w) read += sh.fcnt[w];
-        list_count[2 * gridDim.x + b] = read;
+        list_count[2 * batch + b] = read;
       }
       __syncthreads();  // fcnt is reused by the select below
     }
@@ -2342,21 +2697,35 @@ __global__ void __launch_bounds__(NT) fine_select_kernel(
     // (vector loads; the unscored keys are zero).  After a full scan's plan
     // "few" is at most a quarter (the whole row's register pass is fast).
     if (np <= kPageListCap && (zero_all ? 4 * np : 2 * np) <= U) {
+      const int clear = GR || keep ? CLEAR_NONE : zero_all ? CLEAR_ROW : CLEAR_LISTED;
       if constexpr (NT > kSelThreads) {
         // A few pages' keys: fewer waves merge their bounds faster, so the
         // waves past kSelThreads leave (a wave-uniform test).
         if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) >= kSelThreads / 64) return;
-        select_listed_pages<kSelThreads>(row, plist, np, page_size, partial_len, U, n, k, zero_all, sh_few, cand,
-                                         out, list_cap, fine_stats, list_count, b);
+        select_listed_pages<kSelThreads>(row, plist, np, page_size, partial_len, U, n, k, clear, sh_few, cand, out,
+                                         list_cap, fine_stats, list_count, b, batch);
       } else {
-        select_listed_pages<NT>(row, plist, np, page_size, partial_len, U, n, k, zero_all, sh, cand, out,
-                                list_cap, fine_stats, list_count, b);
+        select_listed_pages<NT>(row, plist, np, page_size, partial_len, U, n, k, clear, sh, cand, out, list_cap,
+                                fine_stats, list_count, b, batch);
       }
       return;
     }
   }
+  if constexpr (GR) {
+    __syncthreads();  // the pool's page list is done with
+    C = select_by_groups<NT>(row, n, k, sg.gmax + (int64_t)b * sg.ldg, sh, gcnt, reinterpret_cast<uint64_t *>(pool),
+                             reinterpret_cast<int *>(pool + kGroupKeyCap * sizeof(uint64_t)), out, list_cap);
+    if (C >= 0) {
+      if (threadIdx.x == 0) {
+        list_count[b] = C;
+        list_count[batch + b] = -1;
+      }
+      return;
+    }
+    __syncthreads();
+  }
   const MemKeys4<NT> mk{row, n};
-  if (n <= 4 * V * NT) {
+  if (!GR && n <= 4 * V * NT) {
     RegKeys4<NT, V> rk;
     rk.load(row, n);
     C = bound_candidates<NT>(rk, k, sh, cand, mx, sum, nz);
@@ -2369,14 +2738,16 @@ __global__ void __launch_bounds__(NT) fine_select_kernel(
     emit_topk_unranked<NT>(mk, cand, C, k, sh, [&](int pos, uint64_t x) { out[pos] = x; });
     C = k;
   }
-  __syncthreads();
-  uint4 *row4 = reinterpret_cast<uint4 *>(row);
-  for (int i = threadIdx.x; i < (n + 3) / 4; i += NT) row4[i] = make_uint4(0, 0, 0, 0);
+  if (!GR && !keep) {
+    __syncthreads();
+    uint4 *row4 = reinterpret_cast<uint4 *>(row);
+    for (int i = threadIdx.x; i < (n + 3) / 4; i += NT) row4[i] = make_uint4(0, 0, 0, 0);
+  }
   if (threadIdx.x == 0) {
     fine_stats[2 * b] = mx;
     fine_stats[2 * b + 1] = sum;
     list_count[b] = C;
-    list_count[gridDim.x + b] = nz;
+    list_count[batch + b] = nz;
   }
 }
 
@@ -2418,24 +2789,79 @@ struct GatherArgs {
   int round;
   float *stats_out;
   double *stats_accum;
+  // After a wide select: the segments' sums, and the keys and group maxima
+  // that the launch's last blocks clear.
+  const SegSum *sums;  // [B][nseg], or NULL
+  int nseg;
+  uint32_t *keys, *gmax;
+  int64_t keys_ld, gmax_ld;
 };
+
+// Blocks past the telemetry block, after a wide select: block i of a batch
+// row's nseg + 1 clears segment i of its keys, the last one its group
+// maxima, as far as candidates were scored.
+__device__ inline void clear_keys(const GatherArgs &ga, int i) {
+  const int b = i / (ga.nseg + 1), seg = i - b * (ga.nseg + 1);
+  const int n = (ga.has_pages ? ga.counters[0] : 0) * ga.page_size + ga.partial_len;
+  uint4 *at;
+  int n4;
+  if (seg < ga.nseg) {
+    at = reinterpret_cast<uint4 *>(ga.keys + (int64_t)b * ga.keys_ld + (int64_t)seg * kSumKeys);
+    n4 = (max(0, min(kSumKeys, n - seg * kSumKeys)) + 3) / 4;
+  } else {
+    at = reinterpret_cast<uint4 *>(ga.gmax + (int64_t)b * ga.gmax_ld);
+    n4 = ((n + kGroupKeys - 1) / kGroupKeys + 3) / 4;
+  }
+  for (int c = threadIdx.x; c < n4; c += 256) at[c] = make_uint4(0, 0, 0, 0);
+}
 
 // The fine telemetry (max and mean over the batch rows) and the pruning
 // control, run by one block of its own after the gather blocks: its global
 // reads then delay no copy.
 template <int DT> __device__ void gather_telemetry(const GatherArgs &ga) {
-  if (threadIdx.x != 0) return;
-  const int batch = ga.batch;
+  if (threadIdx.x >= 64) return;
+  // Every load that the results need is issued before any is used: this
+  // block's chain of round trips must not outlast the gather.
+  const int batch = ga.batch, lane = threadIdx.x;
   const int32_t *list_count = ga.list_count;
   const int U = ga.has_pages ? ga.counters[0] : 0;
+  const int c0 = ga.ctl ? ga.ctl[0] : 0;
+  const double a2 = ga.stats_accum ? ga.stats_accum[2] : 0.0, a3 = ga.stats_accum ? ga.stats_accum[3] : 0.0;
   float m = -INFINITY;
   double t = 0.0;
   int64_t scored = 0;  // every candidate, unless the fine scan was pruned
+  int64_t read = 0;
   for (int r = 0; r < batch; ++r) {
-    m = fmaxf(m, ga.fine_stats[2 * r]);
-    t += ga.fine_stats[2 * r + 1];
-    scored += list_count[batch + r];
+    int nz = list_count[batch + r];
+    float mr = ga.fine_stats[2 * r];
+    double sr = ga.fine_stats[2 * r + 1];
+    read += list_count[2 * batch + r];
+    if (ga.sums) {
+      // A wide select's segments, over the wave's lanes (nz -1: taken).
+      double ts = 0.0;
+      float ms = -INFINITY;
+      int cs = 0;
+      for (int i = lane; i < ga.nseg; i += 64) {
+        const SegSum x = ga.sums[(int64_t)r * ga.nseg + i];
+        ts += x.sum;
+        ms = fmaxf(ms, x.max);
+        cs += x.n;
+      }
+#pragma unroll
+      for (int o = 32; o >= 1; o >>= 1) ts += __shfl_xor(ts, o, 64);
+      ms = wave_max(ms);
+      cs = wave_sum_i32(cs);
+      if (nz < 0) {
+        nz = cs;
+        mr = ms;
+        sr = ts;
+      }
+    }
+    m = fmaxf(m, mr);
+    t += sr;
+    scored += nz;
   }
+  if (lane != 0) return;
   float mean = (float)(t / (double)scored);
   if (ga.round) mean = round_act<DT>(mean);
   if (ga.stats_out) {
@@ -2443,16 +2869,13 @@ template <int DT> __device__ void gather_telemetry(const GatherArgs &ga) {
     ga.stats_out[3] = mean;
   }
   if (ga.stats_accum) {
-    ga.stats_accum[2] += (double)m;
-    ga.stats_accum[3] += (double)mean;
+    ga.stats_accum[2] = a2 + (double)m;
+    ga.stats_accum[3] = a3 + (double)mean;
   }
   if (ga.ctl) {
     // Pruning pays when it skips: after a call that read more than three
     // quarters of the union's slices, the next kPruneRetry calls scan in
     // full; a paused call counts down.
-    int64_t read = 0;
-    for (int r = 0; r < batch; ++r) read += list_count[2 * batch + r];
-    const int c0 = ga.ctl[0];
     ga.ctl[0] = c0 > 0 ? c0 - 1 : (4 * read > 3 * (int64_t)U * ga.hkv * batch ? kPruneRetry : 0);
   }
 }
@@ -2540,29 +2963,33 @@ template <int DT> __device__ void gather_block(const GatherArgs &ga, int bx, int
   }
 }
 
-// Blocks [0, gx * B) gather (block i: entries of batch row i / gx), the
-// last one runs the telemetry.
+// The first block runs the telemetry, the next gx * B gather (block 1 + i:
+// entries of batch row i / gx), any after them clear keys.
 template <int DT> __global__ void __launch_bounds__(256) gather_kernel(GatherArgs ga, int gx) {
-  const int gather_blocks = gx * ga.batch;
-  if ((int)blockIdx.x < gather_blocks) gather_block<DT>(ga, blockIdx.x % gx, blockIdx.x / gx);
-  else gather_telemetry<DT>(ga);
+  const int i = (int)blockIdx.x - 1, gather_blocks = gx * ga.batch;
+  if (i < 0) gather_telemetry<DT>(ga);
+  else if (i < gather_blocks) gather_block<DT>(ga, i % gx, i / gx);
+  else clear_keys(ga, i - gather_blocks);
 }
 
 // The gather plus the hot window's attention splits (kiv_retrieve_attend):
-// blocks [0, gx * B) gather, the s_hot * R blocks after them each run one
-// hot split of one kv row, and the last block runs the telemetry.  The
-// splits do not depend on the retrieval, so they run alongside the gather
-// instead of after it.
+// the first block runs the telemetry, the next gx * B gather, the s_hot * R
+// blocks after them each run one hot split of one kv row, any after those
+// clear keys.  The splits do not depend on the retrieval, so they run
+// alongside the gather instead of after it.
 template <int DT, int KT>
 __global__ void __launch_bounds__(256) gather_attn_kernel(GatherArgs ga, AttnParams p, int gx, int s_hot) {
-  const int gather_blocks = gx * ga.batch;
-  if ((int)blockIdx.x < gather_blocks) {
-    gather_block<DT>(ga, blockIdx.x % gx, blockIdx.x / gx);
-    return;
+  const int i = (int)blockIdx.x - 1, gather_blocks = gx * ga.batch, splits = s_hot * ga.batch * ga.hkv;
+  if (i < 0) {
+    gather_telemetry<DT>(ga);
+  } else if (i < gather_blocks) {
+    gather_block<DT>(ga, i % gx, i / gx);
+  } else if (i < gather_blocks + splits) {
+    const int j = i - gather_blocks;
+    attn_mfma_split<DT, KT>(p, j % s_hot, j / s_hot);
+  } else {
+    clear_keys(ga, i - gather_blocks - splits);
   }
-  const int i = blockIdx.x - gather_blocks;
-  if (i < s_hot * ga.batch * ga.hkv) attn_mfma_split<DT, KT>(p, i % s_hot, i / s_hot);
-  else gather_telemetry<DT>(ga);
 }
 
 // Launches the select kernel kern_of(V) whose register chunks per thread V
@@ -3000,18 +3427,37 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
   // ---- fine: per-candidate max-over-heads score, top-P', gather
   const int64_t cmax = umax * ps + s->partial_len;
   const int64_t ldc = (cmax + 63) & ~int64_t(63);
-  if (s->fine_keys.bytes < (size_t)B * ldc * 4) {
-    if ((rc = s->fine_keys.ensure((size_t)B * ldc * 4, st, false))) return rc;
+  // A decode step over K in HBM: few query rows per kv head, pages of whole
+  // tiles.
+  const bool heads = fine_mfma && !host_tier && G * Q < kFineMfmaRows && ps % kGroupKeys == 0;
+  // The wide select (fine_select_kernel, GR): every candidate scored, rows
+  // that may hold more keys than a 512-thread block keeps in 4 chunks a
+  // thread, and group maxima that tile the pages.
+  const bool wide = cmax > kWideSelKeys && !prune;
+  const bool groups = wide && fine_mfma && ps % kGroupKeys == 0;
+  const int64_t ldg = groups ? (ldc / kGroupKeys + 63) & ~int64_t(63) : 0;
+  const int nseg = groups ? (int)((cmax + kSumKeys - 1) / kSumKeys) : 0;
+  // fine_scan_heads_kernel stores its keys, in a buffer of its own: the other
+  // scans fold theirs with atomics into a buffer that is zero between calls.
+  if (heads) {
+    if ((rc = s->fine_vals.ensure((size_t)B * (ldc + ldg) * 4, st, false))) return rc;
+  } else if (s->fine_keys.bytes < (size_t)B * (ldc + ldg) * 4) {
+    if ((rc = s->fine_keys.ensure((size_t)B * (ldc + ldg) * 4, st, false))) return rc;
     KIV_HIP(hipMemsetAsync(s->fine_keys.ptr, 0, s->fine_keys.bytes, st));
   }
   // Candidate lists of the fine select: [B][list_ld] composites, then [B]
-  // counts, [B] numbers of scored candidates and [B] slices read.
+  // counts, [B] numbers of scored candidates and [B] slices read, then the
+  // wide select's segment sums.
   const int list_cap = fine_list_cap(a->out_width);
   const int64_t lmax = std::min<int64_t>(cmax, std::max<int64_t>(list_cap, a->out_width));
   const int64_t list_ld = (std::max<int64_t>(list_cap, a->out_width) + 31) & ~int64_t(31);
-  if ((rc = s->sel_list.ensure((size_t)B * list_ld * 8 + (size_t)B * 12, st, false))) return rc;
+  const size_t sums_off = ((size_t)B * list_ld * 8 + (size_t)B * 12 + 255) & ~size_t(255);
+  if ((rc = s->sel_list.ensure(sums_off + (size_t)B * nseg * sizeof(SegSum), st, false))) return rc;
   uint64_t *list = (uint64_t *)s->sel_list.ptr;
   int32_t *list_count = (int32_t *)(list + (size_t)B * list_ld);
+  SegSum *sums = (SegSum *)((char *)s->sel_list.ptr + sums_off);
+  uint32_t *fkeys = (uint32_t *)(heads ? s->fine_vals.ptr : s->fine_keys.ptr);
+  uint32_t *gmax = groups ? fkeys + (size_t)B * ldc : nullptr;
   const int bwords = union_src == UNION_ROWS ? words : 0;
   // The fine scans' LDS list of the union pages (row lists: at most
   // min(rows * kc, N) pages).
@@ -3098,7 +3544,46 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
     // other positions read the copy.
     // (Several passes imply a union list and more than kFineMfmaRows rows.)
     const bool query_scan = mfma && union_src == UNION_LIST && !sel_plan && G * Q >= kFineMfmaRows;
-    const int first_q = mfma && (!query_scan || k_stage) ? std::min(Qb, Q) : 0;  // positions of the first scan
+    const int first_q = mfma && !heads && (!query_scan || k_stage) ? std::min(Qb, Q) : 0;  // positions of the first scan
+    if (heads) {
+      // Tiles of 16 candidates over the blocks that run at once: six a
+      // compute unit, four at head_dim 192 and 256 (by registers); more
+      // would only repeat the union's prologue.
+      const int hw = hkv >= 3 ? 4 : hkv;
+      const int64_t tile_blocks = ((cmax + 15) / 16 + 4 / hw - 1) / (4 / hw);
+      const unsigned nb_h = (unsigned)std::max<int64_t>(1, std::min<int64_t>(tile_blocks, ((kt > 4 ? 1024 : 1536) + B - 1) / B));
+      const size_t lds = (size_t)bwords * 4 + upage_bytes;
+      s->prof_begin(KIV_STAGE_FINE_SCAN, st);
+      rc = with_dt(dt, [&](auto dtc) {
+        constexpr int DTV = decltype(dtc)::value;
+        if constexpr (DTV == DT_F32) {
+          return (int)KIV_ERR_UNSUPPORTED;
+        } else {
+          return with_kt(kt, [&](auto ktc) {
+            constexpr int KTV = decltype(ktc)::value;
+            if constexpr (KTV == 16) {
+              return (int)KIV_ERR_UNSUPPORTED;
+            } else {
+              auto kern = fine_scan_heads_kernel<DTV, KTV>;
+              if (lds > 65536 - 2048)
+                KIV_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+              hipLaunchKernelGGL(kern, dim3(nb_h + (sp.plan ? 1u : 0u), (unsigned)B), dim3(256), lds, st, union_src,
+                                 (const int32_t *)s->row_pages.ptr, rows * kc, bwords, (int32_t *)s->page_list.ptr,
+                                 (int32_t *)s->counters.ptr, (const uint64_t *)s->k_tab.ptr, (int)s->k_chunks.size(),
+                                 s->chunk_shift, s->page_bytes, (const char *)s->k_part.ptr, (int)s->partial_len, ps,
+                                 hkv, hw,
+                                 (const char *)a->q, a->q_stride[0], a->q_stride[1], a->q_stride[2], hq, Q,
+                                 a->scaling, round, fkeys, ldc, (const float *)coarse_stats, rows, N, a->pages_out,
+                                 a->union_count_out, a->stats_out, a->stats_accum, sp, gmax, ldg);
+              return (int)KIV_OK;
+            }
+          });
+        }
+      });
+      s->prof_end(KIV_STAGE_FINE_SCAN, st);
+      if (rc) return rc;
+      KIV_HIP(hipGetLastError());
+    }
     if (first_q > 0) {
       const int Qp = first_q;
       const int gq16 = (G * Qp + 15) & ~15;
@@ -3124,8 +3609,9 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
                                  (int32_t *)s->counters.ptr, (const uint64_t *)s->k_tab.ptr, s->chunk_shift,
                                  s->page_bytes, (const char *)s->k_part.ptr, (int)s->partial_len, ps, tpi, hkv,
                                  (const char *)a->q, a->q_stride[0], a->q_stride[1], a->q_stride[2], hq, Qp,
-                                 a->scaling, round, (uint32_t *)s->fine_keys.ptr, ldc, (const float *)coarse_stats,
-                                 rows, N, a->pages_out, a->union_count_out, a->stats_out, a->stats_accum, k_stage, sp);
+                                 a->scaling, round, fkeys, ldc, (const float *)coarse_stats,
+                                 rows, N, a->pages_out, a->union_count_out, a->stats_out, a->stats_accum, k_stage, sp,
+                                 gmax, ldg);
               return (int)KIV_OK;
             }
           });
@@ -3154,7 +3640,7 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
                                  (const char *)s->k_part.ptr, (int)s->partial_len, ps, hkv,
                                  (const char *)a->q + (int64_t)first_q * a->q_stride[2] * eb, a->q_stride[0],
                                  a->q_stride[1], a->q_stride[2], hq, Q - first_q, a->scaling, round,
-                                 (uint32_t *)s->fine_keys.ptr, ldc, (const char *)k_stage);
+                                 fkeys, ldc, (const char *)k_stage, gmax, ldg);
               return (int)KIV_OK;
             }
           });
@@ -3182,7 +3668,7 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
                            (int32_t *)s->counters.ptr, (const uint64_t *)s->k_tab.ptr, s->chunk_shift,
                            s->page_bytes, (const char *)s->k_part.ptr, (int)s->partial_len, ps, tpi, hkv, D,
                            (const char *)a->q + pass * qstep, a->q_stride[0], a->q_stride[1], a->q_stride[2], hq,
-                           Qp, a->scaling, round, (uint32_t *)s->fine_keys.ptr, ldc, (const float *)coarse_stats,
+                           Qp, a->scaling, round, fkeys, ldc, (const float *)coarse_stats,
                            rows, N, a->pages_out, a->union_count_out, a->stats_out, a->stats_accum,
                            pass == 0 ? k_stage : nullptr, pass == 0 ? nullptr : k_stage, fp);
         KIV_HIP(hipGetLastError());
@@ -3197,20 +3683,28 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
   }
   {
     s->prof_begin(KIV_STAGE_FINE_SELECT, st);
-    // Rows of more than 8192 candidates take a block of 1024 threads (half
-    // the keys per thread, the same per-wave bound).
+    // Rows of more than kWideSelKeys candidates take a block of 1024 threads
+    // (half the keys per thread, the same per-wave bound), with the group
+    // maxima and the segments' blocks where the pages allow them.
+    const SelectGroups sg{gmax, ldg, sums, nseg, B};
     auto launch = [&](auto kern, int nt) {
-      hipLaunchKernelGGL(kern, dim3(B), dim3(nt), 0, st, (uint32_t *)s->fine_keys.ptr, ldc,
+      hipLaunchKernelGGL(kern, dim3((unsigned)(B + B * nseg)), dim3(nt), 0, st, fkeys, ldc,
                          (const int32_t *)s->counters.ptr, N > 0 ? 1 : 0, ps, (int)s->partial_len, a->out_width,
                          fine_stats, list, list_ld, list_count, list_cap, pr_ub, s->kr, hkv, pr_thr,
-                         (const int32_t *)s->page_list.ptr, (const int32_t *)pr.plan, sel_plan ? 1 : 0, pr.ctl);
+                         (const int32_t *)s->page_list.ptr, (const int32_t *)pr.plan, sel_plan ? 1 : 0, pr.ctl, sg,
+                         heads ? 1 : 0);
     };
-    if (cmax > 4 * 4 * kSelThreads && !prune)
-      with_select_chunks<kWideSelThreads>(cmax, [&](auto kern) { launch(kern, kWideSelThreads); },
-                                          [](auto vc) { return fine_select_kernel<decltype(vc)::value, kWideSelThreads>; });
+    if (groups)
+      launch(sel_plan ? fine_select_kernel<1, kWideSelThreads, true, true>
+                      : fine_select_kernel<1, kWideSelThreads, true, false>, kWideSelThreads);
+    else if (wide)
+      with_select_chunks<kWideSelThreads>(cmax, [&](auto kern) { launch(kern, kWideSelThreads); }, [](auto vc) {
+        return fine_select_kernel<decltype(vc)::value, kWideSelThreads, false, true>;
+      });
     else
-      with_select_chunks<kSelThreads>(cmax, [&](auto kern) { launch(kern, kSelThreads); },
-                                      [](auto vc) { return fine_select_kernel<decltype(vc)::value, kSelThreads>; });
+      with_select_chunks<kSelThreads>(cmax, [&](auto kern) { launch(kern, kSelThreads); }, [](auto vc) {
+        return fine_select_kernel<decltype(vc)::value, kSelThreads, false, true>;
+      });
     s->prof_end(KIV_STAGE_FINE_SELECT, st);
     KIV_HIP(hipGetLastError());
   }
@@ -3254,9 +3748,16 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
     ga.round = round;
     ga.stats_out = a->stats_out;
     ga.stats_accum = a->stats_accum;
+    ga.sums = groups ? sums : nullptr;
+    ga.nseg = nseg;
+    ga.keys = fkeys;
+    ga.gmax = gmax;
+    ga.keys_ld = ldc;
+    ga.gmax_ld = ldg;
+    const unsigned clears = groups && !heads ? (unsigned)(B * (nseg + 1)) : 0u;
     s->prof_begin(KIV_STAGE_GATHER, st);
     if (fa) {
-      const unsigned blocks = gx * (unsigned)B + (unsigned)(fa->s_hot * s->kr) + 1;
+      const unsigned blocks = gx * (unsigned)B + (unsigned)(fa->s_hot * s->kr) + 1 + clears;
       rc = with_dt(dt, [&](auto dtc) {
         constexpr int DTV = decltype(dtc)::value;
         if constexpr (DTV == DT_F32) {
@@ -3274,7 +3775,7 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
       });
     } else {
       rc = with_dt(dt, [&](auto dtc) {
-        hipLaunchKernelGGL((gather_kernel<decltype(dtc)::value>), dim3(gx * (unsigned)B + 1), dim3(256), 0, st, ga,
+        hipLaunchKernelGGL((gather_kernel<decltype(dtc)::value>), dim3(gx * (unsigned)B + 1 + clears), dim3(256), 0, st, ga,
                            (int)gx);
         return (int)KIV_OK;
       });

@@ -375,7 +375,7 @@ int64_t kiv_store::reserved_host_bytes() const {
 int64_t kiv_store::reserved_device_bytes() const {
   int64_t d = (int64_t)(summ.bytes + summ32.bytes + radius.bytes + k_tab.bytes + v_tab.bytes + k_part.bytes +
                         v_part.bytes + coarse_keys.bytes + row_stats.bytes + row_pages.bytes +
-                        page_list.bytes + union_bits.bytes + counters.bytes + fine_keys.bytes + sel_list.bytes + k_stage.bytes + prune.bytes +
+                        page_list.bytes + union_bits.bytes + counters.bytes + fine_keys.bytes + fine_vals.bytes + sel_list.bytes + k_stage.bytes + prune.bytes +
                         first_page.bytes);
   const int64_t chunk = pages_per_chunk * page_bytes;
   if (cfg.cold_tier != KIV_TIER_HOST) d += (int64_t)k_chunks.size() * chunk;
@@ -459,7 +459,8 @@ int kiv_store_destroy(kiv_store_t *s) {
   for (hipEvent_t e : s->prof_ev) (void)hipEventDestroy(e);
   DevBuf *bufs[] = {&s->summ, &s->summ32, &s->radius, &s->k_tab, &s->v_tab, &s->k_part, &s->v_part,
                     &s->coarse_keys, &s->row_stats, &s->row_pages, &s->page_list, &s->union_bits, &s->counters,
-                    &s->fine_keys, &s->sel_list, &s->k_stage, &s->prune};
+                    &s->fine_keys, &s->fine_vals, &s->sel_list, &s->k_stage, &s->prune,
+                    &s->first_page};
   for (DevBuf *b : bufs) b->release();
   delete s;
   return KIV_OK;

@@ -987,3 +987,75 @@ def test_long_query_edges(cuda, name, w, batch, positions, tier):
         q = data["q"].float().repeat(1, 1, positions, 1)
         q = (q + 0.2 * torch.randn(q.shape, generator=g)).to(w.dtype)
         check_retrieval(store, oracle, cfg, w, data, q, min_det_c=0.3)
+
+
+WIDE_SELECTS = [
+    # name, workload, batch, clustered query
+    # 3 kv heads on 4 waves, 17 query rows per head (two operand tiles), 16-token pages
+    ("hkv3_gq17_page16", Workload("ws1", 51, 3, 32, torch.float16, hot=16, cold=9000 + 15, top_pages=30, top_p=300,
+                                  segment=256, page_size=16), 1, False),
+    # 5 kv heads (two steps a wave, the last one short), two batch rows
+    ("hkv5_batch2_page32", Workload("ws2", 10, 5, 64, torch.bfloat16, hot=16, cold=12000 + 31, top_pages=60,
+                                    top_p=256, segment=512, page_size=32), 2, True),
+    # more keys asked for than a wave has group maxima: no bound, the plain select runs
+    ("hkv2_k_past_groups", Workload("ws3", 4, 2, 128, torch.bfloat16, hot=16, cold=9001, top_pages=70, top_p=1500,
+                                    segment=512), 1, False),
+    # the best candidates share groups: the second bound shortens the list
+    ("hkv1_d256_refined", Workload("ws4", 8, 1, 256, torch.bfloat16, hot=16, cold=30000 + 1, top_pages=64,
+                                   top_p=1024, segment=2048), 1, True),
+    # every tile of the last segment, and the row's very end
+    ("hkv4_d96_whole_pages", Workload("ws5", 16, 4, 96, torch.float16, hot=16, cold=128 * 128, top_pages=64,
+                                      top_p=64, segment=512), 1, False),
+]
+
+
+@pytest.mark.parametrize("name,w,batch,clustered", WIDE_SELECTS, ids=[c[0] for c in WIDE_SELECTS])
+def test_wide_select(cuda, name, w, batch, clustered):
+    """Decode over K in HBM whose rows may hold more than 8,192 candidates:
+    keys stored per tile, group maxima and the wide select, against the
+    oracle's bar, twice in a row with other queries (the telemetry too: its
+    mean comes from the segments' blocks)."""
+    data = generate(w, seed=23, batch=batch)
+    g = torch.Generator().manual_seed(24)
+    store, oracle, cfg = build(w, data, cuda, cold_tier="hbm")
+    for call in range(2):
+        q = data["q"].float() + 0.2 * torch.randn(data["q"].shape, generator=g)
+        if not clustered:
+            q = torch.randn(data["q"].shape, generator=g)
+        q = q.to(w.dtype)
+        info = {}
+        check_retrieval(store, oracle, cfg, w, data, q, min_det_c=0.0, info=info)
+        fine = store.telemetry_snapshot()["recent"][-1]
+        cand = exact.candidate_ids(np.array(info["union"], dtype=np.int64), w.page_size,
+                                   store.num_pages * w.page_size, store.cold_length % w.page_size)
+        lo, hi = score_interval(q.float().numpy(), data["cold_k"][:, :, torch.from_numpy(cand)].float().numpy(),
+                                w.scaling, DT[w.dtype], "activation")
+        # The fp32 sum of C scores, rounded to the dtype at the end: each
+        # partial sum's rounding is far below the dtype's half step.
+        step = 2.0 ** -8 if w.dtype == torch.bfloat16 else 2.0 ** -11
+        lo, hi = lo.max(axis=(1, 2)).mean(), hi.max(axis=(1, 2)).mean()
+        slack = step * max(abs(lo), abs(hi)) + 1e-4
+        assert lo - slack <= fine["mean_score"] <= hi + slack
+
+
+@pytest.mark.parametrize("equal", [1500, 4000, 9000])
+def test_wide_select_mass_ties(cuda, equal):
+    """`equal` tokens share the best score: the list (at most 1,024), the
+    keys held in LDS (6,144) and the row itself each run out in turn, and the
+    lowest candidates win."""
+    D, cold, P = 64, 20000, 256
+    cfg = KIVConfig(hot_budget=16, top_p=P, page_size=128, top_pages=200, cold_tier="hbm")
+    topo = ModelTopology.manual(global_layer_indices=(0,), num_query_heads=4, num_kv_heads=1, head_dim=D,
+                                num_hidden_layers=1)
+    store = ColdKVStore(cfg, topo, cuda)
+    k = torch.zeros(1, 1, cold, D)
+    first = 3001
+    k[:, :, first:first + equal, 0] = 1.0
+    v = torch.arange(cold, dtype=torch.float32)[None, None, :, None].expand(1, 1, cold, D) / 64
+    store.evict_from_hot(k.to(torch.bfloat16).to(cuda), v.to(torch.bfloat16).to(cuda))
+    q = torch.zeros(1, 4, 1, D)
+    q[..., 0] = 2.0
+    for _ in range(2):
+        store.retrieve_top_kv(q.to(torch.bfloat16).to(cuda), 1.0, cfg)
+        ids = store.telemetry_snapshot()["recent"][-1]["selected_token_indices"]
+        assert ids == list(range(first, first + P))
