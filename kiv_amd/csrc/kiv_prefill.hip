@@ -103,38 +103,30 @@ __device__ __forceinline__ float float_bias(const PrefillParams &p, int64_t o) {
   }
 }
 
-// Row groups of 16 query rows per wave: two up to head_dim 128 (each K and
-// V^T operand read from LDS then feeds two MFMAs, halving LDS and L2 traffic
-// per flop), one above (the accumulators would not fit twice).
+// Query rows per block: 32 a wave up to head_dim 128 (each K and V^T operand
+// read from LDS then feeds a 32x32 matrix instruction), 16 above (the
+// accumulators would not fit).
 template <int KT> struct PfShape {
-  static constexpr int RG = KT <= 4 ? 2 : 1;
-  static constexpr int ROWS = 64 * RG;  // query rows per block
+  static constexpr int ROWS = KT <= 4 ? 128 : 64;
 };
 constexpr int kPfLdsTiles = 4096;  // tile classes a block keeps in LDS (hot windows up to 256K keys)
 
 // One block's share of the work: its query rows, its key tiles and their
 // classes, and the staging of K and V tiles through registers into LDS (K
 // rows [64][D] padded by 16 bytes, V transposed [D][64] padded by 8 bytes).
-template <int DT, int KT, int MK> struct PfBlock {
-  static constexpr int D = 32 * KT, CPR = D / 8, RG = PfShape<KT>::RG, NT = kPfThreads, ROWS = PfShape<KT>::ROWS;
-  static constexpr int KROW = D + 8;        // K tile row stride in elements
-  static constexpr int VROW = kPfKeys + 4;  // V^T tile row stride in elements
-  static constexpr int KTILE = kPfKeys * KROW, VTILE = D * VROW;  // elements of one LDS tile
-  static constexpr int KJ = (kPfKeys * CPR + NT - 1) / NT;          // K chunks per thread
-  static constexpr int VJ = ((kPfKeys / 4) * CPR + NT - 1) / NT;    // V key quads per thread
+template <int DT, int KT, int MK> struct PfGeom {
+  static constexpr int D = 32 * KT, CPR = D / 8, NT = kPfThreads, ROWS = PfShape<KT>::ROWS;
   static_assert(ROWS % 64 == 0, "a block covers whole 64-row mask class entries");
 
   const PrefillParams &p;
   const uint8_t *tcls;  // LDS copy of this block's hot tile classes (mask tensors)
-  int b, h, kvh, z, tid, col, grp, q0, qlast, off, nct, nht, t_begin, t_end;
+  int b, h, kvh, z, tid, wave, lane, q0, qlast, off, nct, nht, t_begin, t_end;
   bool causal, cls_lds;
-  int qi[RG], qc[RG];  // the lane's query rows (rows past Q repeat row Q - 1's data)
   const uint8_t *cls_rows;
   int cls_n;
   const char *cold_kb, *cold_vb, *hot_kb, *hot_vb;
-  uint4 kreg[KJ], vreg[VJ][4];
 
-  __device__ __forceinline__ PfBlock(const PrefillParams &pp, uint8_t *tcls_lds) : p(pp), tcls(tcls_lds) {
+  __device__ __forceinline__ PfGeom(const PrefillParams &pp, uint8_t *tcls_lds) : p(pp), tcls(tcls_lds) {
     // One-dimensional grid, longest work first: row blocks from the last
     // (under the causal rule later rows see more tiles), then batch rows,
     // heads and key splits, so that the dispatcher hands out the block
@@ -147,15 +139,9 @@ template <int DT, int KT, int MK> struct PfBlock {
     h = bh - b * p.hq;
     kvh = h / (p.hq / p.hkv);
     tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
-    col = lane & 15;
-    grp = lane >> 4;
+    wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    lane = tid & 63;
     q0 = (nrb - 1 - rb) * ROWS;
-#pragma unroll
-    for (int g = 0; g < RG; ++g) {
-      qi[g] = q0 + 16 * (RG * wave + g) + col;
-      qc[g] = min(qi[g], p.qlen - 1);
-    }
     qlast = min(q0 + ROWS, p.qlen) - 1;
     off = p.hot_len - p.qlen;  // causal: hot column t visible to row i iff t <= i + off
     causal = p.mask_kind == KIV_MASK_CAUSAL;
@@ -221,6 +207,72 @@ template <int DT, int KT, int MK> struct PfBlock {
   }
   __device__ __forceinline__ int first_tile() const {
     return t_begin < t_end && tile_class(t_begin) != TILE_SKIP ? t_begin : next_tile(t_begin);
+  }
+
+  // Bias of four consecutive keys k4 .. k4 + 3 of a MIXED tile (its first
+  // key key0 of its segment, n keys left in it) for query row qrow, whose
+  // mask offset is row_mo: 0 or -inf, or the float mask's value (base 2).
+  __device__ __forceinline__ void bias4(bool cold, int key0, int n, int k4, int qrow, int64_t row_mo,
+                                        float (&bias)[4]) const {
+    const int64_t mo = row_mo + (int64_t)(key0 + k4) * p.ms3;
+    if (cold || MK == PF_ARITH) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bool vis = k4 + i < n && (cold || !causal || key0 + k4 + i <= qrow + off);
+        bias[i] = vis ? 0.f : -INFINITY;
+      }
+    } else if (MK == PF_BOOL) {
+      uint32_t bits = 0;
+      if (p.mask_vec4 && k4 + 4 <= n) {
+        bits = *reinterpret_cast<const uint32_t *>(p.mask + mo);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (k4 + i < n && p.mask[mo + (int64_t)i * p.ms3]) bits |= 0xffu << (8 * i);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) bias[i] = (bits >> (8 * i)) & 0xffu ? 0.f : -INFINITY;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) bias[i] = k4 + i < n ? float_bias(p, mo + (int64_t)i * p.ms3) : -INFINITY;
+    }
+  }
+  __device__ __forceinline__ int64_t row_mask_off(int qrow) const { return mask_off(p, b, h, qrow, 0); }
+
+  // Four consecutive output dims d .. d + 3 of query row qrow: normalised,
+  // or (with key splits) this split's unnormalised sums.
+  __device__ __forceinline__ int64_t split_row(int qrow) const {
+    return (int64_t)z * p.batch * p.qlen * p.hq + ((int64_t)b * p.qlen + qrow) * p.hq + h;
+  }
+  __device__ __forceinline__ char *out_row(int qrow) const {
+    return p.out + (((int64_t)b * p.qlen + qrow) * p.hq + h) * (int64_t)D * 2;
+  }
+};
+
+// Head dims above 128: a wave holds 16 query rows, tiles go to LDS through
+// registers (K rows padded by 16 bytes, V transposed).
+template <int DT, int KT, int MK> struct PfBlock : PfGeom<DT, KT, MK> {
+  using Geom = PfGeom<DT, KT, MK>;
+  using Geom::b, Geom::CPR, Geom::cold_kb, Geom::cold_vb, Geom::D, Geom::h, Geom::hot_kb, Geom::hot_vb, Geom::NT,
+      Geom::nct, Geom::p, Geom::tid, Geom::wave, Geom::lane, Geom::q0, Geom::z;
+  static constexpr int RG = 1;
+  static constexpr int KROW = D + 8;        // K tile row stride in elements
+  static constexpr int VROW = kPfKeys + 4;  // V^T tile row stride in elements
+  static constexpr int KTILE = kPfKeys * KROW, VTILE = D * VROW;  // elements of one LDS tile
+  static constexpr int KJ = (kPfKeys * CPR + NT - 1) / NT;          // K chunks per thread
+  static constexpr int VJ = ((kPfKeys / 4) * CPR + NT - 1) / NT;    // V key quads per thread
+  int col, grp;
+  int qi[RG], qc[RG];  // the lane's query rows (rows past Q repeat row Q - 1's data)
+  uint4 kreg[KJ], vreg[VJ][4];
+
+  __device__ __forceinline__ PfBlock(const PrefillParams &pp, uint8_t *tcls_lds) : Geom(pp, tcls_lds) {
+    col = lane & 15;
+    grp = lane >> 4;
+#pragma unroll
+    for (int g = 0; g < RG; ++g) {
+      qi[g] = q0 + 16 * (RG * wave + g) + col;
+      qc[g] = min(qi[g], p.qlen - 1);
+    }
   }
 
   // Loads tile t's K chunks (V key quads) into registers through a buffer
@@ -299,42 +351,17 @@ template <int DT, int KT, int MK> struct PfBlock {
   __device__ __forceinline__ void add_bias(f32x4_t (&s)[RG][4], int t) const {
     const bool cold = t < nct;
     const int key0 = (cold ? t : t - nct) * kPfKeys, n = (cold ? p.cold_len : p.hot_len) - key0;
-    // Mask element offsets: a per-lane part per row group plus a uniform part.
-    int64_t lane_mo[RG];
 #pragma unroll
-    for (int g = 0; g < RG; ++g) lane_mo[g] = (int64_t)qc[g] * p.ms2 + (int64_t)(4 * grp) * p.ms3;
-    const int64_t blk_mo = (int64_t)b * p.ms0 + (int64_t)h * p.ms1 + (int64_t)key0 * p.ms3;
-#pragma unroll
-    for (int g = 0; g < RG; ++g)
+    for (int g = 0; g < RG; ++g) {
+      const int64_t row_mo = this->row_mask_off(qc[g]);
 #pragma unroll
       for (int sub = 0; sub < 4; ++sub) {
-        const int k4 = 16 * sub + 4 * grp;  // first of the lane's four keys in the tile
-        const int64_t mo = blk_mo + (int64_t)(16 * sub) * p.ms3 + lane_mo[g];
         float bias[4];
-        if (cold || MK == PF_ARITH) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const bool vis = k4 + i < n && (cold || !causal || key0 + k4 + i <= qc[g] + off);
-            bias[i] = vis ? 0.f : -INFINITY;
-          }
-        } else if (MK == PF_BOOL) {
-          uint32_t bits = 0;
-          if (p.mask_vec4 && k4 + 4 <= n) {
-            bits = *reinterpret_cast<const uint32_t *>(p.mask + mo);
-          } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              if (k4 + i < n && p.mask[mo + (int64_t)i * p.ms3]) bits |= 0xffu << (8 * i);
-          }
-#pragma unroll
-          for (int i = 0; i < 4; ++i) bias[i] = (bits >> (8 * i)) & 0xffu ? 0.f : -INFINITY;
-        } else {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) bias[i] = k4 + i < n ? float_bias(p, mo + (int64_t)i * p.ms3) : -INFINITY;
-        }
+        this->bias4(cold, key0, n, 16 * sub + 4 * grp, qc[g], row_mo, bias);
 #pragma unroll
         for (int i = 0; i < 4; ++i) s[g][sub][i] = fmaf(s[g][sub][i], p.scale_log2, bias[i]);
       }
+    }
   }
 
   // The block's rows: normalised output, or (with key splits) this split's
@@ -342,12 +369,11 @@ template <int DT, int KT, int MK> struct PfBlock {
   __device__ __forceinline__ void finish(const f32x4_t (&o)[RG][D / 16], const float (&m_run)[RG],
                                          const float (&l_lane)[RG]) const {
     if (p.nsplit > 1) {
-      const int64_t nrows = (int64_t)p.batch * p.qlen * p.hq;
 #pragma unroll
       for (int g = 0; g < RG; ++g) {
         const float l_row = half_wave_sum(row_pair_sum(l_lane[g]));
         if (qi[g] >= p.qlen) continue;
-        const int64_t sr = (int64_t)z * nrows + ((int64_t)b * p.qlen + qi[g]) * p.hq + h;
+        const int64_t sr = this->split_row(qi[g]);
         float *po = p.ws_o + sr * D;
 #pragma unroll
         for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<f32x4_t *>(po + 16 * dt + 4 * grp) = o[g][dt];
@@ -364,7 +390,7 @@ template <int DT, int KT, int MK> struct PfBlock {
       if (qi[g] >= p.qlen) continue;
       // A row with no visible key (fully masked) gets zeros.
       const float inv = l_row > 0.f ? 1.f / l_row : 0.f;
-      char *orow = p.out + (((int64_t)b * p.qlen + qi[g]) * p.hq + h) * (int64_t)D * 2;
+      char *orow = this->out_row(qi[g]);
 #pragma unroll
       for (int dt = 0; dt < D / 16; ++dt)
         *reinterpret_cast<uint2 *>(orow + (16 * dt + 4 * grp) * 2) = make_uint2(
@@ -587,8 +613,288 @@ __global__ void __launch_bounds__(kPfThreads) mask_tiles_kernel(PrefillParams p)
   }
 }
 
-// One tile at a time, every step in order: store the tile to LDS, scores,
-// softmax, PV.
+// ---------------------------------------------------------------------------
+// Head dims up to 128: 32 query rows a wave on v_mfma_f32_32x32x16.
+//
+// K and V tiles go from memory straight to LDS (buffer loads of 16 bytes a
+// lane into 1 KiB of LDS an instruction), both as rows, double-buffered: a
+// tile has the whole computation of the one before it to arrive, and a wave
+// passes one barrier a tile.  LDS rows hold CP 16-byte chunks (head_dim 96
+// is padded to 16 chunks); the chunks of a row are permuted so that every
+// operand read spreads over the banks (K by row, so that 16 rows' same chunk
+// lie in 16 different places; V by key, so that four keys' 64-byte pieces
+// do), which the loading lanes do by fetching the permuted chunk.
+//  - S^T = K Q^T: lane l gives row l % 32 of a 32-key sub-tile of K (A) and
+//    its own query row l % 32 (B, in registers for the whole kernel), dims
+//    16 st + 8 (l / 32) .. + 7 of step st, and receives keys
+//    8 (i / 4) + 4 (l / 32) + i % 4 (i < 16) of the sub-tile for its row.
+//  - O^T += V^T P^T, 16 keys a step: the B operand is the lane's own
+//    probabilities 8 j .. 8 j + 7 of a sub-tile (keys 16 j + 4 (l / 32) + i
+//    for i < 4, 16 j + 8 + 4 (l / 32) + i - 4 for i >= 4), the A operand the
+//    same keys of dim l % 32, from two transposing LDS reads
+//    (ds_read_b64_tr_b16: each 16 lanes read 4 keys x 16 dims and lane n
+//    receives the 4 keys of dim n).
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+template <int DT> __device__ __forceinline__ f32x16_t mfma_32x32x16(const uint4 &a, const uint4 &b, f32x16_t c) {
+  if constexpr (DT == DT_BF16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b),
+                                                    c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c,
+                                                   0, 0, 0);
+}
+constexpr int kWaitVm0 = 0x0f70;  // s_waitcnt vmcnt(0), the other counters unconstrained
+typedef __attribute__((address_space(3))) void lds_void_t;
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) i16x4_t lds_i16x4_t;
+
+template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
+  using Geom = PfGeom<DT, KT, MK>;
+  using Geom::b, Geom::CPR, Geom::cold_kb, Geom::cold_vb, Geom::D, Geom::h, Geom::hot_kb, Geom::hot_vb, Geom::nct,
+      Geom::p, Geom::wave, Geom::lane, Geom::q0;
+  static constexpr int CP = CPR <= 4 ? 4 : CPR <= 8 ? 8 : 16;  // chunks per LDS row
+  static constexpr int RPI = 64 / CP;                          // rows per load instruction
+  static constexpr int NJ = CP / 4;                            // load instructions per wave for a tile of K (of V)
+  static constexpr int TILE = kPfKeys * CP * 8;                // elements of a tile in LDS
+  static constexpr int KS = D / 16, ND = D / 32;               // score steps, output dim tiles
+  int row, hf;         // the lane's query row (column of both products) and half
+  int qi, qc;          // its query position; the last one for rows past Q
+  int lrow, kc, vc;    // loads: the lane's row of the wave's first instruction, its K and V chunk bytes
+  int kaddr, vaddr[ND];  // operand reads: byte offsets of the lane within a K / V tile
+
+  __device__ __forceinline__ PfBlock32(const PrefillParams &pp, uint8_t *tcls_lds) : Geom(pp, tcls_lds) {
+    row = lane & 31;
+    hf = lane >> 5;
+    qi = q0 + 32 * wave + row;
+    qc = min(qi, p.qlen - 1);
+    // Row r holds K chunk c at c ^ xk(r), xk(r) = r / (16 / CP) mod CP, and
+    // V chunk c at c ^ 4 xv(r), xv(r) = r mod 4 (16 chunks) or r / 2 mod 2
+    // (8) or 0 (4): the same for every load instruction of a lane, whose
+    // rows are 4 RPI apart.
+    lrow = wave * RPI + lane / CP;
+    const int pc = lane % CP;
+    kc = min(pc ^ ((lrow / (16 / CP)) & (CP - 1)), CPR - 1) * 16;
+    vc = min(pc ^ (4 * xv(lrow)), CPR - 1) * 16;
+    kaddr = row * CP * 16 + ((hf ^ ((row / (16 / CP)) & (CP - 1))) << 4);
+    const int j16 = lane & 15, q = j16 >> 2;  // the transposing read: key q of four, dims 4 (j16 % 4) ..
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) {
+      const int c = 4 * (dt ^ xv(q)) + 2 * ((lane >> 4) & 1) + ((j16 & 3) >> 1);
+      vaddr[dt] = (4 * hf + q) * CP * 16 + c * 16 + (j16 & 1) * 8;
+    }
+  }
+  static __device__ __forceinline__ int xv(int r) { return CP == 16 ? r & 3 : CP == 8 ? (r >> 1) & 1 : 0; }
+
+  // Starts tile t's loads into LDS (rows past the segment's end repeat its
+  // last row; their scores get a -inf bias, as such a tile is MIXED).
+  __device__ __forceinline__ void load_tile(int t, uint16_t *ks, uint16_t *vs) const {
+    const bool cold = t < nct;
+    const int key0 = (cold ? t : t - nct) * kPfKeys, last = (cold ? p.cold_len : p.hot_len) - key0 - 1;
+    const uint32_t krs = cold ? D * 2 : (uint32_t)p.hks2 * 2, vrs = cold ? D * 2 : (uint32_t)p.hvs2 * 2;
+    const auto rk = tile_rsrc((cold ? cold_kb : hot_kb) + (int64_t)key0 * krs, 0xffffffffu);
+    const auto rv = tile_rsrc((cold ? cold_vb : hot_vb) + (int64_t)key0 * vrs, 0xffffffffu);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const uint32_t r = (uint32_t)min(lrow + j * 4 * RPI, last);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_void_t *)(ks + (j * 4 + wave) * 512), 16,
+                                               (int)(r * krs + (uint32_t)kc), 0, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const uint32_t r = (uint32_t)min(lrow + j * 4 * RPI, last);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_void_t *)(vs + (j * 4 + wave) * 512), 16,
+                                               (int)(r * vrs + (uint32_t)vc), 0, 0, 0);
+    }
+  }
+
+  __device__ __forceinline__ void load_q(uint4 (&qx)[KS]) const {
+    const char *qrow = p.q + ((int64_t)b * p.qs0 + (int64_t)h * p.qs1 + (int64_t)qc * p.qs2) * 2 + 16 * hf;
+#pragma unroll
+    for (int st = 0; st < KS; ++st) qx[st] = load16(qrow + 32 * st);
+  }
+
+  // MIXED tile t: hidden keys' dot products become -inf (the others stay as
+  // in a FULL tile, bit for bit); with a float mask the scores become
+  // s * scaling * log2 e + bias (base 2).
+  __device__ __forceinline__ void add_bias(f32x16_t (&s)[2], int t) const {
+    const bool cold = t < nct;
+    const int key0 = (cold ? t : t - nct) * kPfKeys, n = (cold ? p.cold_len : p.hot_len) - key0;
+    const int64_t row_mo = this->row_mask_off(qc);
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        float bias[4];
+        this->bias4(cold, key0, n, 32 * sub + 8 * u + 4 * hf, qc, row_mo, bias);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          s[sub][4 * u + i] = MK == PF_FLOAT ? fmaf(s[sub][4 * u + i], p.scale_log2, bias[i]) : s[sub][4 * u + i] + bias[i];
+      }
+  }
+
+  // The rows' outputs (dims 32 dt + 8 u + 4 hf .. + 3 of the lane's row), or
+  // with key splits the unnormalised sums, running max and row sum.
+  __device__ __forceinline__ void finish(const f32x16_t (&o)[ND], float m_run, float l_lane) const {
+    const float l_row = half_wave_sum(l_lane);
+    if (qi >= p.qlen) return;
+    if (p.nsplit > 1) {
+      const int64_t sr = this->split_row(qi);
+      float *po = p.ws_o + sr * D;
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          *reinterpret_cast<f32x4_t *>(po + 32 * dt + 8 * u + 4 * hf) =
+              f32x4_t{o[dt][4 * u], o[dt][4 * u + 1], o[dt][4 * u + 2], o[dt][4 * u + 3]};
+      if (hf == 0) {
+        p.ws_m[sr] = m_run;
+        p.ws_l[sr] = l_row;
+      }
+      return;
+    }
+    // A row with no visible key (fully masked) gets zeros.
+    const float inv = l_row > 0.f ? 1.f / l_row : 0.f;
+    char *orow = this->out_row(qi);
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt)
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        *reinterpret_cast<uint2 *>(orow + (32 * dt + 8 * u + 4 * hf) * 2) =
+            make_uint2(pack2<DT>(o[dt][4 * u] * inv, o[dt][4 * u + 1] * inv),
+                       pack2<DT>(o[dt][4 * u + 2] * inv, o[dt][4 * u + 3] * inv));
+  }
+
+  // One tile, its rows in ks / vs.
+  __device__ __forceinline__ void tile(int t, int cls, const uint16_t *ks, const uint16_t *vs, const uint4 (&qx)[KS],
+                                       f32x16_t (&o)[ND], float &m_run, float &l_lane) const {
+    const char *kb = reinterpret_cast<const char *>(ks), *vb = reinterpret_cast<const char *>(vs);
+    f32x16_t s[2] = {};
+#pragma unroll
+    for (int st = 0; st < KS; ++st)
+#pragma unroll
+      for (int sub = 0; sub < 2; ++sub) {
+        const uint4 a = *reinterpret_cast<const uint4 *>(kb + (kaddr ^ (st << 5)) + sub * 32 * CP * 16);
+        s[sub] = mfma_32x32x16<DT>(a, qx[st], s[sub]);
+      }
+    // Issue order: kAhead operand reads in flight, then one per instruction.
+    constexpr int NR = 2 * KS, kAhead = NR < 6 ? NR : 6;
+    __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
+#pragma unroll
+    for (int i = 0; i < NR - kAhead; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
+    // The first PV step's V operands, in flight under the softmax.
+    uint4 va[2][ND];
+    load_v(vb, 0, va[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    // Scores in base-2 units are cc * s, cc = scaling * log2 e folded into
+    // the exponent (1 where a float mask's bias was added).
+    float cc = p.scale_log2;
+    if (cls == TILE_MIXED) {
+      add_bias(s, t);
+      if (MK == PF_FLOAT) cc = 1.f;
+    }
+    // The running max is raised (and the sums rescaled) only on a tile where
+    // a lane's maximum exceeds it by more than 2^kRescaleSlack; the row's
+    // maximum, over its two lanes, is formed on such tiles alone.
+    float x = s[0][0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) x = fmaxf(x, s[0][i]);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x = fmaxf(x, s[1][i]);
+    if (__ballot(x * cc > m_run + kRescaleSlack)) {
+      const float mt = half_wave_max(x) * cc;
+      const float m_new = mt > m_run + kRescaleSlack ? mt : m_run;
+      const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
+      l_lane *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt) o[dt] *= alpha;
+      m_run = m_new;
+    }
+    // Probabilities 2^(cc s - m), rounded to the dtype as operands; a row
+    // that has seen no key keeps m = -inf, its probabilities are 0.
+    // Four steps of 16 keys: a step's matrix instructions issue among the
+    // next step's exponentials, and its V operands were read a step before.
+    const float m_neg = m_run == -INFINITY ? 0.f : -m_run;
+    auto probs = [&](int k) {
+      float e[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) e[i] = __builtin_amdgcn_exp2f(fmaf(s[k >> 1][8 * (k & 1) + i], cc, m_neg));
+#pragma unroll
+      for (int i = 0; i < 8; ++i) l_lane += e[i];
+      return make_uint4(pack2<DT>(e[0], e[1]), pack2<DT>(e[2], e[3]), pack2<DT>(e[4], e[5]), pack2<DT>(e[6], e[7]));
+    };
+    uint4 pb = probs(0);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (k < 3) load_v(vb, k + 1, va[(k + 1) & 1]);
+      uint4 pn = pb;
+      if (k < 3) pn = probs(k + 1);
+#pragma unroll
+      for (int dt = 0; dt < ND; ++dt) o[dt] = mfma_32x32x16<DT>(va[k & 1][dt], pb, o[dt]);
+      if (k < 3) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 * ND, 0);
+#pragma unroll
+        for (int dt = 0; dt < ND; ++dt) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x402, 28 / ND, 0);
+        }
+      }
+      pb = pn;
+    }
+  }
+  // V^T operands of PV step k (keys 16 k .. + 15 of the tile).
+  __device__ __forceinline__ void load_v(const char *vb, int k, uint4 (&a)[ND]) const {
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) {
+      const char *at = vb + vaddr[dt] + 16 * k * CP * 16;
+      const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t *)at));
+      const uint2 hi =
+          __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t *)(at + 8 * CP * 16)));
+      a[dt] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+    }
+  }
+};
+
+template <int DT, int KT, int MK>
+__global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
+prefill_attn32_kernel(PrefillParams p) {
+  using Blk = PfBlock32<DT, KT, MK>;
+  // Two buffers as objects of their own: the compiler then knows that a
+  // tile's operand reads do not depend on the other buffer's loads.
+  __shared__ __align__(1024) uint16_t k0[Blk::TILE], k1[Blk::TILE], v0[Blk::TILE], v1[Blk::TILE];
+  __shared__ uint8_t tcls[MK == PF_ARITH ? 1 : kPfLdsTiles];
+  Blk blk(p, tcls);
+  int t = blk.first_tile();
+  if (t < blk.t_end) blk.load_tile(t, k0, v0);
+  uint4 qx[Blk::KS];
+  blk.load_q(qx);
+  f32x16_t o[Blk::ND] = {};
+  float m_run = -INFINITY, l_lane = 0.f;  // l_lane: this lane's share of the row sum
+  // The tile's loads have arrived (each wave waits for its own, then the
+  // barrier), and every wave is done with the buffer the next ones fill.
+  auto step = [&](uint16_t *ks, uint16_t *vs, uint16_t *kn, uint16_t *vn) {
+    const int cls = blk.tile_class(t), tn = blk.next_tile(t);
+    __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (tn < blk.t_end) blk.load_tile(tn, kn, vn);
+    blk.tile(t, cls, ks, vs, qx, o, m_run, l_lane);
+    t = tn;
+  };
+  while (t < blk.t_end) {
+    step(k0, v0, k1, v1);
+    if (t >= blk.t_end) break;
+    step(k1, v1, k0, v0);
+  }
+  blk.finish(o, m_run, l_lane);
+}
+
+// Head dims above 128, one tile at a time, every step in order: store the
+// tile to LDS, scores, softmax, PV.
 template <int DT, int KT, int MK>
 __global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
 prefill_attn_kernel(PrefillParams p) {
@@ -826,7 +1132,10 @@ int kiv_prefill_attention(const kiv_attention_args_t *a, kiv_stream_t stream) {
       const dim3 grid((unsigned)nblocks);
       auto launch = [&](auto dtc, auto mkc) {
         constexpr int DTV = decltype(dtc)::value, MKV = decltype(mkc)::value;
-        hipLaunchKernelGGL((prefill_attn_kernel<DTV, KTV, MKV>), grid, dim3(kPfThreads), 0, st, p);
+        if constexpr (KTV <= 4)
+          hipLaunchKernelGGL((prefill_attn32_kernel<DTV, KTV, MKV>), grid, dim3(kPfThreads), 0, st, p);
+        else
+          hipLaunchKernelGGL((prefill_attn_kernel<DTV, KTV, MKV>), grid, dim3(kPfThreads), 0, st, p);
       };
       using std::integral_constant;
       auto by_mode = [&](auto dtc) {
