@@ -12,14 +12,23 @@
 // own rounding, u * sum_k p_k |v_k|.
 //
 // Blocks of 256 threads own 128 query rows of one q head (64 above head_dim
-// 128): wave w holds row groups of 16 rows.  The grid is one-dimensional in
-// longest-first order (row blocks from the last, which under the causal rule
-// see the most keys), and long rows are split over key ranges whose partial
-// rows a combine kernel merges; the host picks the split count by
-// simulating the longest-first schedule over the GPU's block slots.  Keys
-// come in tiles of 64: first the retrieved keys, then the hot keys (a tile
-// never mixes the two, so hot tiles line up with the mask's column tiles).
-// Per tile:
+// 128).  Keys come in tiles of 64: first the retrieved keys, then the hot
+// keys (a tile never mixes the two, so hot tiles line up with the mask's
+// column tiles).  Online softmax in base 2; the running maximum is raised,
+// and the accumulators rescaled, only when a score exceeds it by more than
+// 2^8, so probabilities stay below 256 and most tiles skip the rescale and
+// the cross-lane maxima.
+//
+// Head dims up to 128 (prefill_attn32_kernel, below): 32 query rows a wave,
+// the work dealt to the GPU's block slots in equal shares (PfShares).  The
+// model's chunk, 4096 x 8192 keys of 12 heads under a boolean mask: 230.6 ->
+// 185.0 us a call, 155 GFLOP; the attention kernel about 160 us, matrix
+// cores busy 43% of its cycles (28% before), bound by the issue of the
+// softmax beside the matrix instructions with two waves a SIMD.
+//
+// Head dims above 128 (prefill_attn_kernel): wave w holds 16 query rows.
+// The grid is one-dimensional in longest-first order and long rows are split
+// over key ranges whose partial rows a combine kernel merges.  Per tile:
 //  - K rows ([64][D], rows padded by 16 bytes) and V transposed ([D][64],
 //    rows padded by 8 bytes) go to LDS from registers that were loaded
 //    (buffer loads bounded to the segment) while the previous tile was
@@ -28,17 +37,12 @@
 //    16-key sub-tile of K (A) and its own query row l % 16 (B, held in
 //    registers for the whole kernel), dims 32 s + 8 (l / 16) .. + 7 of
 //    step s, and receives keys 4 (l / 16) + i of the sub-tile for its row;
-//  - online softmax in base 2 per query row: the lane's 16 scores, and the
-//    row maximum across the four lanes that share the row (l, l ^ 16,
-//    l ^ 32, l ^ 48) on the tiles that raise it.  The running maximum is
-//    raised, and the accumulators rescaled, only when a score exceeds it by
-//    more than 2^8, so probabilities stay below 256 and most tiles skip the
-//    rescale and the cross-lane maxima;
 //  - O^T += V^T P^T with v_mfma_f32_16x16x32 over 32 keys: the B operand is
 //    exactly the lane's probabilities of two sub-tiles (k index 8 g + i is
 //    key 4 g + i of the first sub-tile for i < 4, of the second for i >= 4),
 //    the A operand the same keys of one dim from the V^T tile.  All O^T
 //    entries of a lane belong to its query row.
+//
 // Tile classes: SKIP (no row of the block sees a key of the tile), FULL
 // (every key present and visible with zero bias: no per-element work) and
 // MIXED.  The causal rule and the tile edges give them arithmetically; for
@@ -61,6 +65,33 @@ constexpr float kRescaleSlack = 8.f;  // base-2 headroom before the running max 
 enum { TILE_SKIP = 0, TILE_FULL = 1, TILE_MIXED = 2 };
 enum { PF_ARITH = 0, PF_BOOL = 1, PF_FLOAT = 2 };  // how MIXED tiles get their bias
 
+// Shares of the work of head dims up to 128.  A unit is a block of kPfUnitRows
+// query rows of one (b, q head); units are numbered heads first (unit = bh *
+// nrb + rb) and a unit's weight is its tiles: the retrieved keys' and the hot
+// keys' up to its last row's diagonal (every hot tile without a mask; a mask
+// tensor is taken to be causal, which only balances the shares).
+// blocks > 0: block i takes the weights [start(i), start(i + 1)), equal to
+// within one tile, through as many units as they span; a unit cut by a
+// share's end is merged from partial rows by prefill_merge_kernel: partial
+// 2 i is block i's first fragment, 2 i + 1 its last.  (Key splits of equal
+// tile ranges left 27% of the block slots' time empty on the model's chunk,
+// where a range may hold no visible tile; see prefill_attn32_kernel.)
+// blocks == 0: block i is one whole unit, longest first.
+struct PfShares {
+  int blocks, per, rem;   // start(i) = i * per + min(i, rem)
+  int nrb, head, a, step; // row blocks; weight of one (b, q head); weight of row block rb < nrb - 1: a + step * rb
+  int tiles;              // tiles of a unit (the last row block's weight)
+  __host__ __device__ int start(int i) const { return i * per + (i < rem ? i : rem); }
+  __host__ __device__ int block_of(int x) const {
+    const int cut = rem * (per + 1);
+    return x < cut ? x / (per + 1) : rem + (x - cut) / per;
+  }
+  // Weight of the row blocks before rb.
+  __host__ __device__ int before(int rb) const { return rb * a + step * (rb * (rb - 1) / 2); }
+  __host__ __device__ int weight(int rb) const { return rb + 1 == nrb ? tiles : a + step * rb; }
+};
+constexpr int kPfUnitRows = 128;
+
 struct PrefillParams {
   const char *q;
   int64_t qs0, qs1, qs2;
@@ -81,6 +112,7 @@ struct PrefillParams {
   // rows and (running max, row sum) here and prefill_combine_kernel merges.
   int nsplit;
   float *ws_m, *ws_l, *ws_o;  // [nsplit][B*Q*Hq], [nsplit][B*Q*Hq], [nsplit][B*Q*Hq][D]
+  PfShares sh;                // head dims up to 128: the blocks' shares (then ws_* are per partial, see there)
 };
 
 // Two fp32 values rounded to the dtype (hardware conversion, nearest even),
@@ -119,53 +151,42 @@ template <int DT, int KT, int MK> struct PfGeom {
   static_assert(ROWS % 64 == 0, "a block covers whole 64-row mask class entries");
 
   const PrefillParams &p;
-  const uint8_t *tcls;  // LDS copy of this block's hot tile classes (mask tensors)
   int b, h, kvh, z, tid, wave, lane, q0, qlast, off, nct, nht, t_begin, t_end;
-  bool causal, cls_lds;
+  bool causal;
   const uint8_t *cls_rows;
   int cls_n;
   const char *cold_kb, *cold_vb, *hot_kb, *hot_vb;
 
-  __device__ __forceinline__ PfGeom(const PrefillParams &pp, uint8_t *tcls_lds) : p(pp), tcls(tcls_lds) {
-    // One-dimensional grid, longest work first: row blocks from the last
-    // (under the causal rule later rows see more tiles), then batch rows,
-    // heads and key splits, so that the dispatcher hands out the block
-    // slots longest-first and the launch ends with short blocks.
-    const int per_rb = p.batch * p.hq * p.nsplit, lin = blockIdx.x;
-    const int nrb = gridDim.x / per_rb, rb = lin / per_rb, rem = lin - rb * per_rb;
-    const int bh = rem / p.nsplit;
-    z = rem - bh * p.nsplit;
-    b = bh / p.hq;
-    h = bh - b * p.hq;
-    kvh = h / (p.hq / p.hkv);
+
+  __device__ __forceinline__ explicit PfGeom(const PrefillParams &pp) : p(pp) {
+    z = 0;
     tid = threadIdx.x;
     wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     lane = tid & 63;
-    q0 = (nrb - 1 - rb) * ROWS;
-    qlast = min(q0 + ROWS, p.qlen) - 1;
     off = p.hot_len - p.qlen;  // causal: hot column t visible to row i iff t <= i + off
     causal = p.mask_kind == KIV_MASK_CAUSAL;
     nct = (p.cold_len + kPfKeys - 1) / kPfKeys;
     nht = (p.hot_len + kPfKeys - 1) / kPfKeys;
-    // This block's share of the tiles (all of them without key splits).
-    const int ntiles = nct + nht;
-    t_end = (int)((int64_t)(z + 1) * ntiles / p.nsplit);
-    t_begin = (int)((int64_t)z * ntiles / p.nsplit);
+  }
+
+  // Row block rb of (b, q head) bh, its tiles [t0, t1).
+  __device__ __forceinline__ void set_unit(int bh, int rb, int t0, int t1) {
+    b = bh / p.hq;
+    h = bh - b * p.hq;
+    kvh = h / (p.hq / p.hkv);
+    q0 = rb * ROWS;
+    qlast = min(q0 + ROWS, p.qlen) - 1;
+    t_begin = t0;
+    t_end = t1;
     // Mask tensors: the classes of this block's rows (the 64-row entries it
-    // spans, combined), in LDS when they fit.
+    // spans, to be combined).
     cls_rows = nullptr;
     cls_n = 0;
-    cls_lds = false;
     if constexpr (MK != PF_ARITH) {
       const int mb = p.mask_b == 1 ? 0 : b, mh = p.mask_h == 1 ? 0 : h;
       const int nqb = (p.qlen + 63) / 64, r0 = q0 / 64;
       cls_n = min(ROWS / 64, nqb - r0);
       cls_rows = p.tiles + ((int64_t)(mb * p.mask_h + mh) * nqb + r0) * nht;
-      cls_lds = nht <= kPfLdsTiles;
-      if (cls_lds) {
-        for (int k = tid; k < nht; k += NT) tcls_lds[k] = (uint8_t)combine(k);
-        __syncthreads();
-      }
     }
     cold_kb = p.cold_k + ((int64_t)b * p.hkv + kvh) * p.cold_len * (int64_t)D * 2;
     cold_vb = p.cold_v + ((int64_t)b * p.hkv + kvh) * p.cold_len * (int64_t)D * 2;
@@ -181,32 +202,18 @@ template <int DT, int KT, int MK> struct PfGeom {
     }
     return c;
   }
-  // Class of tile t for this block (uniform over the block).
-  __device__ __forceinline__ int tile_class(int t) const {
+  // Class of tile t for this block (mask tensors: read from memory).
+  __device__ __forceinline__ int tile_class_of(int t) const {
     if (t < nct) return (t + 1) * kPfKeys <= p.cold_len ? TILE_FULL : TILE_MIXED;
-    const int key0 = (t - nct) * kPfKeys;
     if constexpr (MK == PF_ARITH) {
+      const int key0 = (t - nct) * kPfKeys;
       const bool whole = key0 + kPfKeys <= p.hot_len;
       if (!causal) return whole ? TILE_FULL : TILE_MIXED;
       if (key0 > qlast + off) return TILE_SKIP;
       return whole && key0 + kPfKeys - 1 <= q0 + off ? TILE_FULL : TILE_MIXED;
     } else {
-      return __builtin_amdgcn_readfirstlane(cls_lds ? (int)tcls[t - nct] : combine(t - nct));
+      return combine(t - nct);
     }
-  }
-  // The first tile after t that is not skipped, or t_end.
-  __device__ __forceinline__ int next_tile(int t) const {
-    for (++t; t < t_end; ++t) {
-      if constexpr (MK == PF_ARITH) {
-        // The causal rule hides every tile after the first hidden one.
-        if (causal && t >= nct && (t - nct) * kPfKeys > qlast + off) return t_end;
-      }
-      if (tile_class(t) != TILE_SKIP) return t;
-    }
-    return t_end;
-  }
-  __device__ __forceinline__ int first_tile() const {
-    return t_begin < t_end && tile_class(t_begin) != TILE_SKIP ? t_begin : next_tile(t_begin);
   }
 
   // Bias of four consecutive keys k4 .. k4 + 3 of a MIXED tile (its first
@@ -254,18 +261,56 @@ template <int DT, int KT, int MK> struct PfGeom {
 template <int DT, int KT, int MK> struct PfBlock : PfGeom<DT, KT, MK> {
   using Geom = PfGeom<DT, KT, MK>;
   using Geom::b, Geom::CPR, Geom::cold_kb, Geom::cold_vb, Geom::D, Geom::h, Geom::hot_kb, Geom::hot_vb, Geom::NT,
-      Geom::nct, Geom::p, Geom::tid, Geom::wave, Geom::lane, Geom::q0, Geom::z;
+      Geom::nct, Geom::p, Geom::t_begin, Geom::t_end, Geom::tid, Geom::wave, Geom::lane, Geom::q0, Geom::z;
   static constexpr int RG = 1;
   static constexpr int KROW = D + 8;        // K tile row stride in elements
   static constexpr int VROW = kPfKeys + 4;  // V^T tile row stride in elements
   static constexpr int KTILE = kPfKeys * KROW, VTILE = D * VROW;  // elements of one LDS tile
   static constexpr int KJ = (kPfKeys * CPR + NT - 1) / NT;          // K chunks per thread
   static constexpr int VJ = ((kPfKeys / 4) * CPR + NT - 1) / NT;    // V key quads per thread
+  const uint8_t *tcls;  // LDS copy of this block's hot tile classes (mask tensors)
+  bool cls_lds;
   int col, grp;
   int qi[RG], qc[RG];  // the lane's query rows (rows past Q repeat row Q - 1's data)
   uint4 kreg[KJ], vreg[VJ][4];
 
-  __device__ __forceinline__ PfBlock(const PrefillParams &pp, uint8_t *tcls_lds) : Geom(pp, tcls_lds) {
+  // Class of tile t, uniform over the block.
+  __device__ __forceinline__ int tile_class(int t) const {
+    if (MK == PF_ARITH || t < nct) return this->tile_class_of(t);
+    return __builtin_amdgcn_readfirstlane(cls_lds ? (int)tcls[t - nct] : this->combine(t - nct));
+  }
+  // The first tile after t that is not skipped, or t_end.
+  __device__ __forceinline__ int next_tile(int t) const {
+    for (++t; t < t_end; ++t) {
+      if constexpr (MK == PF_ARITH) {
+        // The causal rule hides every tile after the first hidden one.
+        if (this->causal && t >= nct && (t - nct) * kPfKeys > this->qlast + this->off) return t_end;
+      }
+      if (tile_class(t) != TILE_SKIP) return t;
+    }
+    return t_end;
+  }
+  __device__ __forceinline__ int first_tile() const {
+    return t_begin < t_end && tile_class(t_begin) != TILE_SKIP ? t_begin : next_tile(t_begin);
+  }
+
+  __device__ __forceinline__ PfBlock(const PrefillParams &pp, uint8_t *tcls_lds) : Geom(pp), tcls(tcls_lds) {
+    // One-dimensional grid, longest work first: row blocks from the last
+    // (under the causal rule later rows see more tiles), then batch rows,
+    // heads and key splits, so that the dispatcher hands out the block
+    // slots longest-first and the launch ends with short blocks.
+    const int per_rb = p.batch * p.hq * p.nsplit, lin = blockIdx.x;
+    const int nrb = gridDim.x / per_rb, rb = lin / per_rb, rem = lin - rb * per_rb;
+    const int bh = rem / p.nsplit;
+    z = rem - bh * p.nsplit;
+    // This block's share of the tiles (all of them without key splits).
+    const int ntiles = nct + this->nht;
+    this->set_unit(bh, nrb - 1 - rb, (int)((int64_t)z * ntiles / p.nsplit), (int)((int64_t)(z + 1) * ntiles / p.nsplit));
+    cls_lds = MK != PF_ARITH && this->nht <= kPfLdsTiles;
+    if (cls_lds) {
+      for (int k = tid; k < this->nht; k += NT) tcls_lds[k] = (uint8_t)this->combine(k);
+      __syncthreads();
+    }
     col = lane & 15;
     grp = lane >> 4;
 #pragma unroll
@@ -643,7 +688,8 @@ template <int DT> __device__ __forceinline__ f32x16_t mfma_32x32x16(const uint4 
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c,
                                                    0, 0, 0);
 }
-constexpr int kWaitVm0 = 0x0f70;  // s_waitcnt vmcnt(0), the other counters unconstrained
+constexpr int kWaitVm0 = 0x0f70;    // s_waitcnt vmcnt(0), the other counters unconstrained
+constexpr int kWaitLgkm0 = 0xc07f;  // s_waitcnt lgkmcnt(0)
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) i16x4_t lds_i16x4_t;
@@ -651,7 +697,7 @@ typedef __attribute__((address_space(3))) i16x4_t lds_i16x4_t;
 template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
   using Geom = PfGeom<DT, KT, MK>;
   using Geom::b, Geom::CPR, Geom::cold_kb, Geom::cold_vb, Geom::D, Geom::h, Geom::hot_kb, Geom::hot_vb, Geom::nct,
-      Geom::p, Geom::wave, Geom::lane, Geom::q0;
+      Geom::p, Geom::t_begin, Geom::t_end, Geom::wave, Geom::lane, Geom::q0;
   static constexpr int CP = CPR <= 4 ? 4 : CPR <= 8 ? 8 : 16;  // chunks per LDS row
   static constexpr int RPI = 64 / CP;                          // rows per load instruction
   static constexpr int NJ = CP / 4;                            // load instructions per wave for a tile of K (of V)
@@ -662,11 +708,12 @@ template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
   int lrow, kc, vc;    // loads: the lane's row of the wave's first instruction, its K and V chunk bytes
   int kaddr, vaddr[ND];  // operand reads: byte offsets of the lane within a K / V tile
 
-  __device__ __forceinline__ PfBlock32(const PrefillParams &pp, uint8_t *tcls_lds) : Geom(pp, tcls_lds) {
+  int wbase;             // tiles wbase .. + 63 as bits: not skipped, and mixed
+  uint64_t wseen, wmixed;
+
+  __device__ __forceinline__ explicit PfBlock32(const PrefillParams &pp) : Geom(pp) {
     row = lane & 31;
     hf = lane >> 5;
-    qi = q0 + 32 * wave + row;
-    qc = min(qi, p.qlen - 1);
     // Row r holds K chunk c at c ^ xk(r), xk(r) = r / (16 / CP) mod CP, and
     // V chunk c at c ^ 4 xv(r), xv(r) = r mod 4 (16 chunks) or r / 2 mod 2
     // (8) or 0 (4): the same for every load instruction of a lane, whose
@@ -683,6 +730,38 @@ template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
       vaddr[dt] = (4 * hf + q) * CP * 16 + c * 16 + (j16 & 1) * 8;
     }
   }
+  __device__ __forceinline__ void set_unit(int bh, int rb, int t0, int t1) {
+    Geom::set_unit(bh, rb, t0, t1);
+    qi = q0 + 32 * wave + row;
+    qc = min(qi, p.qlen - 1);
+    window(t0);
+  }
+  // The classes of 64 tiles in scalar registers, a tile a lane: the loop
+  // finds its next tile with scalar bit operations.
+  __device__ __forceinline__ void window(int base) {
+    wbase = base;
+    const int t = base + lane, cls = t < t_end ? this->tile_class_of(t) : (int)TILE_SKIP;
+    wseen = __ballot(cls != TILE_SKIP);
+    wmixed = __ballot(cls == TILE_MIXED);
+  }
+  // The first tile from t on that is not skipped (its class in cls), or t_end.
+  __device__ __forceinline__ int find_tile(int t, int &cls) {
+    while (t < t_end) {
+      if (t >= wbase + 64) window(t);
+      const uint64_t m = wseen >> (t - wbase);
+      if (m) {
+        t += __builtin_ctzll(m);
+        cls = (wmixed >> (t - wbase)) & 1 ? TILE_MIXED : TILE_FULL;
+        return t;
+      }
+      t = wbase + 64;
+      if constexpr (MK == PF_ARITH) {
+        // The causal rule hides every tile after the first hidden one.
+        if (this->causal && t >= nct && (t - nct) * kPfKeys > this->qlast + this->off) return t_end;
+      }
+    }
+    return t_end;
+  }
   static __device__ __forceinline__ int xv(int r) { return CP == 16 ? r & 3 : CP == 8 ? (r >> 1) & 1 : 0; }
 
   // Starts tile t's loads into LDS (rows past the segment's end repeat its
@@ -693,18 +772,24 @@ template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
     const uint32_t krs = cold ? D * 2 : (uint32_t)p.hks2 * 2, vrs = cold ? D * 2 : (uint32_t)p.hvs2 * 2;
     const auto rk = tile_rsrc((cold ? cold_kb : hot_kb) + (int64_t)key0 * krs, 0xffffffffu);
     const auto rv = tile_rsrc((cold ? cold_vb : hot_vb) + (int64_t)key0 * vrs, 0xffffffffu);
+    auto load = [&](__amdgpu_buffer_rsrc_t rs, uint16_t *to, int j, uint32_t voff, uint32_t soff) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void_t *)(to + (j * 4 + wave) * 512), 16, (int)voff, (int)soff,
+                                               0, 0);
+    };
+    if (last >= kPfKeys - 1) {
+      // A whole tile: one lane offset each, the instructions' rows in the
+      // scalar offset.
+      const uint32_t ko = (uint32_t)lrow * krs + (uint32_t)kc, vo = (uint32_t)lrow * vrs + (uint32_t)vc;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const uint32_t r = (uint32_t)min(lrow + j * 4 * RPI, last);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_void_t *)(ks + (j * 4 + wave) * 512), 16,
-                                               (int)(r * krs + (uint32_t)kc), 0, 0, 0);
+      for (int j = 0; j < NJ; ++j) load(rk, ks, j, ko, (uint32_t)(j * 4 * RPI) * krs);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) load(rv, vs, j, vo, (uint32_t)(j * 4 * RPI) * vrs);
+      return;
     }
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const uint32_t r = (uint32_t)min(lrow + j * 4 * RPI, last);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_void_t *)(vs + (j * 4 + wave) * 512), 16,
-                                               (int)(r * vrs + (uint32_t)vc), 0, 0, 0);
-    }
+    for (int j = 0; j < NJ; ++j) load(rk, ks, j, (uint32_t)min(lrow + j * 4 * RPI, last) * krs + (uint32_t)kc, 0);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) load(rv, vs, j, (uint32_t)min(lrow + j * 4 * RPI, last) * vrs + (uint32_t)vc, 0);
   }
 
   __device__ __forceinline__ void load_q(uint4 (&qx)[KS]) const {
@@ -713,9 +798,50 @@ template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
     for (int st = 0; st < KS; ++st) qx[st] = load16(qrow + 32 * st);
   }
 
-  // MIXED tile t: hidden keys' dot products become -inf (the others stay as
-  // in a FULL tile, bit for bit); with a float mask the scores become
-  // s * scaling * log2 e + bias (base 2).
+  // Visible keys of MIXED tile t as bits, 64 a query row of the block, into
+  // vis[ROWS][2] (thread tid: row tid / 2, keys 32 (tid % 2) .. + 31).  Read
+  // by every lane of the row in hide(); the registers of the mask's elements
+  // are then not live beside the tile's operands.
+  __device__ __forceinline__ void visible_bits(int t, uint32_t *vis) const {
+    const bool cold = t < nct;
+    const int key0 = (cold ? t : t - nct) * kPfKeys, n = (cold ? p.cold_len : p.hot_len) - key0;
+    const int tid = this->tid, half = tid & 1, qr = min(q0 + (tid >> 1), p.qlen - 1);
+    int seen = n;  // keys [0, seen) of the tile can be visible
+    if (!cold && this->causal) seen = min(seen, qr + this->off - key0 + 1);
+    const int cnt = min(max(seen - 32 * half, 0), 32);
+    uint32_t bits = cnt == 32 ? ~0u : (1u << cnt) - 1u;
+    if (MK == PF_BOOL && !cold && cnt > 0) {
+      const char *m = p.mask + mask_off(p, b, h, qr, key0 + 32 * half);
+      uint32_t on = 0;
+      if (p.mask_vec4 && cnt == 32) {
+        uint32_t w[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) w[u] = *reinterpret_cast<const uint32_t *>(m + 4 * u);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) on |= (w[u] >> (8 * i)) & 0xffu ? 1u << (4 * u + i) : 0u;
+      } else {
+        for (int i = 0; i < cnt; ++i) on |= m[(int64_t)i * p.ms3] ? 1u << i : 0u;
+      }
+      bits &= on;
+    }
+    vis[tid] = bits;
+  }
+  // Hidden keys' dot products become -inf; the others stay as in a FULL
+  // tile, bit for bit.
+  __device__ __forceinline__ void hide(f32x16_t (&s)[2], const uint32_t *vis) const {
+    const uint2 w = *reinterpret_cast<const uint2 *>(vis + 2 * (32 * wave + row));
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub) {
+      const uint32_t v = (sub ? w.y : w.x) >> (4 * hf);  // bit 8 u + i: key 8 u + 4 hf + i
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (!(v & (1u << (8 * (i >> 2) + (i & 3))))) s[sub][i] = -INFINITY;
+    }
+  }
+  // MIXED tile t under a float mask: scores become s * scaling * log2 e +
+  // bias (base 2).
   __device__ __forceinline__ void add_bias(f32x16_t (&s)[2], int t) const {
     const bool cold = t < nct;
     const int key0 = (cold ? t : t - nct) * kPfKeys, n = (cold ? p.cold_len : p.hot_len) - key0;
@@ -724,21 +850,21 @@ template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
     for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
+        __builtin_amdgcn_sched_barrier(0);  // four keys at a time: few registers
         float bias[4];
         this->bias4(cold, key0, n, 32 * sub + 8 * u + 4 * hf, qc, row_mo, bias);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          s[sub][4 * u + i] = MK == PF_FLOAT ? fmaf(s[sub][4 * u + i], p.scale_log2, bias[i]) : s[sub][4 * u + i] + bias[i];
+        for (int i = 0; i < 4; ++i) s[sub][4 * u + i] = fmaf(s[sub][4 * u + i], p.scale_log2, bias[i]);
       }
   }
 
   // The rows' outputs (dims 32 dt + 8 u + 4 hf .. + 3 of the lane's row), or
-  // with key splits the unnormalised sums, running max and row sum.
-  __device__ __forceinline__ void finish(const f32x16_t (&o)[ND], float m_run, float l_lane) const {
+  // (partial >= 0) the unnormalised sums, running max and row sum.
+  __device__ __forceinline__ void finish(const f32x16_t (&o)[ND], float m_run, float l_lane, int partial) const {
     const float l_row = half_wave_sum(l_lane);
     if (qi >= p.qlen) return;
-    if (p.nsplit > 1) {
-      const int64_t sr = this->split_row(qi);
+    if (partial >= 0) {
+      const int64_t sr = (int64_t)partial * kPfUnitRows + 32 * wave + row;
       float *po = p.ws_o + sr * D;
 #pragma unroll
       for (int dt = 0; dt < ND; ++dt)
@@ -765,26 +891,26 @@ template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
   }
 
   // One tile, its rows in ks / vs.
-  __device__ __forceinline__ void tile(int t, int cls, const uint16_t *ks, const uint16_t *vs, const uint4 (&qx)[KS],
-                                       f32x16_t (&o)[ND], float &m_run, float &l_lane) const {
+  __device__ __forceinline__ void tile(int t, int cls, const uint16_t *ks, const uint16_t *vs, const uint32_t *vis,
+                                       const uint4 (&qx)[KS], f32x16_t (&o)[ND], float &m_run, float &l_lane) const {
     const char *kb = reinterpret_cast<const char *>(ks), *vb = reinterpret_cast<const char *>(vs);
     f32x16_t s[2] = {};
-#pragma unroll
-    for (int st = 0; st < KS; ++st)
-#pragma unroll
-      for (int sub = 0; sub < 2; ++sub) {
-        const uint4 a = *reinterpret_cast<const uint4 *>(kb + (kaddr ^ (st << 5)) + sub * 32 * CP * 16);
-        s[sub] = mfma_32x32x16<DT>(a, qx[st], s[sub]);
-      }
-    // Issue order: kAhead operand reads in flight, then one per instruction.
+    // Operand i (step i / 2, sub-tile i % 2): kAhead reads in flight, one more
+    // issued behind each matrix instruction, in that order.
     constexpr int NR = 2 * KS, kAhead = NR < 6 ? NR : 6;
-    __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
+    auto k_op = [&](int i) {
+      return *reinterpret_cast<const uint4 *>(kb + (kaddr ^ ((i >> 1) << 5)) + (i & 1) * 32 * CP * 16);
+    };
+    uint4 ka[NR];
 #pragma unroll
-    for (int i = 0; i < NR - kAhead; ++i) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    for (int i = 0; i < kAhead; ++i) ka[i] = k_op(i);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      s[i & 1] = mfma_32x32x16<DT>(ka[i], qx[i >> 1], s[i & 1]);
+      if (i + kAhead < NR) ka[i + kAhead] = k_op(i + kAhead);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
     // The first PV step's V operands, in flight under the softmax.
     uint4 va[2][ND];
     load_v(vb, 0, va[0]);
@@ -793,8 +919,12 @@ template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
     // the exponent (1 where a float mask's bias was added).
     float cc = p.scale_log2;
     if (cls == TILE_MIXED) {
-      add_bias(s, t);
-      if (MK == PF_FLOAT) cc = 1.f;
+      if constexpr (MK == PF_FLOAT) {
+        add_bias(s, t);
+        cc = 1.f;
+      } else {
+        hide(s, vis);
+      }
     }
     // The running max is raised (and the sums rescaled) only on a tile where
     // a lane's maximum exceeds it by more than 2^kRescaleSlack; the row's
@@ -866,31 +996,111 @@ prefill_attn32_kernel(PrefillParams p) {
   // Two buffers as objects of their own: the compiler then knows that a
   // tile's operand reads do not depend on the other buffer's loads.
   __shared__ __align__(1024) uint16_t k0[Blk::TILE], k1[Blk::TILE], v0[Blk::TILE], v1[Blk::TILE];
-  __shared__ uint8_t tcls[MK == PF_ARITH ? 1 : kPfLdsTiles];
-  Blk blk(p, tcls);
-  int t = blk.first_tile();
-  if (t < blk.t_end) blk.load_tile(t, k0, v0);
-  uint4 qx[Blk::KS];
-  blk.load_q(qx);
-  f32x16_t o[Blk::ND] = {};
-  float m_run = -INFINITY, l_lane = 0.f;  // l_lane: this lane's share of the row sum
-  // The tile's loads have arrived (each wave waits for its own, then the
-  // barrier), and every wave is done with the buffer the next ones fill.
-  auto step = [&](uint16_t *ks, uint16_t *vs, uint16_t *kn, uint16_t *vn) {
-    const int cls = blk.tile_class(t), tn = blk.next_tile(t);
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (tn < blk.t_end) blk.load_tile(tn, kn, vn);
-    blk.tile(t, cls, ks, vs, qx, o, m_run, l_lane);
-    t = tn;
-  };
-  while (t < blk.t_end) {
-    step(k0, v0, k1, v1);
-    if (t >= blk.t_end) break;
-    step(k1, v1, k0, v0);
+  __shared__ uint32_t vis0[2 * Blk::ROWS], vis1[2 * Blk::ROWS];
+  Blk blk(p);
+  const PfShares &sh = p.sh;
+  // This block's units: a share's range of weights [w, w_end), or one unit.
+  int bh, rb, w, w_end, id = 0;
+  if (sh.blocks > 0) {
+    // Blocks are dealt to the eight dies in turn: a die takes consecutive
+    // shares, which read the same heads' keys through its L2.
+    id = (sh.blocks & 7) ? (int)blockIdx.x : (int)(blockIdx.x & 7) * (sh.blocks >> 3) + (int)(blockIdx.x >> 3);
+    w = sh.start(id);
+    w_end = sh.start(id + 1);
+    bh = w / sh.head;
+    const int rest = w - bh * sh.head;
+    rb = 0;  // the last row block that starts at or before it
+    for (int hi = sh.nrb - 1; rb < hi;) {
+      const int mid = (rb + hi + 1) >> 1;
+      if (sh.before(mid) <= rest) rb = mid;
+      else hi = mid - 1;
+    }
+  } else {
+    const int nbh = p.batch * p.hq, i = (int)blockIdx.x / nbh;
+    bh = (int)blockIdx.x - i * nbh;
+    rb = sh.nrb - 1 - i;  // longest first
+    w = bh * sh.head + sh.before(rb);
+    w_end = w + sh.weight(rb);
   }
-  blk.finish(o, m_run, l_lane);
+  const int w0 = w;
+  while (w < w_end) {
+    const int us = bh * sh.head + sh.before(rb), ue = us + sh.weight(rb);
+    // A fragment that reaches the unit's end also takes the tiles past its
+    // weight (hidden ones, unless a mask tensor is not causal).
+    blk.set_unit(bh, rb, w - us, w_end >= ue ? sh.tiles : w_end - us);
+    const int partial = w == us && w_end >= ue ? -1 : 2 * id + (w == w0 ? 0 : 1);
+    int cls = TILE_FULL, t = blk.find_tile(blk.t_begin, cls);
+    if (t < blk.t_end) blk.load_tile(t, k0, v0);
+    uint4 qx[Blk::KS];
+    blk.load_q(qx);
+    f32x16_t o[Blk::ND] = {};
+    float m_run = -INFINITY, l_lane = 0.f;  // l_lane: this lane's share of the row sum
+    // The tile's loads have arrived (each wave waits for its own, then the
+    // barrier), and every wave is done with the buffer the next ones fill.
+    auto step = [&](uint16_t *ks, uint16_t *vs, uint16_t *kn, uint16_t *vn, uint32_t *vis) {
+      int cls_n = TILE_FULL;
+      const int tn = blk.find_tile(t + 1, cls_n);
+      if (MK != PF_FLOAT && cls == TILE_MIXED) {
+        blk.visible_bits(t, vis);
+        __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+      }
+      __builtin_amdgcn_s_waitcnt(kWaitVm0);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (tn < blk.t_end) blk.load_tile(tn, kn, vn);
+      blk.tile(t, cls, ks, vs, vis, qx, o, m_run, l_lane);
+      t = tn;
+      cls = cls_n;
+    };
+    while (t < blk.t_end) {
+      step(k0, v0, k1, v1, vis0);
+      if (t >= blk.t_end) break;
+      step(k1, v1, k0, v0, vis1);
+    }
+    blk.finish(o, m_run, l_lane, partial);
+    w = ue;
+    if (++rb == sh.nrb) {
+      rb = 0;
+      ++bh;
+    }
+    if (w < w_end) __syncthreads();  // the next unit's first loads reuse the LDS
+  }
+}
+
+// Merges the units that the shares cut: out = sum_i 2^(m_i - M) o_i / sum_i
+// 2^(m_i - M) l_i over a unit's partials, M their largest running max.
+// Grid (pieces of rows, units): D / 4 threads per output row, 4 dims each;
+// blocks of whole units leave at once.  A row that saw no key gets zeros.
+template <int DT>
+__global__ void __launch_bounds__(kPfThreads) prefill_merge_kernel(PrefillParams p, int D) {
+  const PfShares &sh = p.sh;
+  const int bh = blockIdx.y / sh.nrb, rb = blockIdx.y - bh * sh.nrb;
+  const int us = bh * sh.head + sh.before(rb), ue = us + sh.weight(rb);
+  const int i0 = sh.block_of(us), i1 = sh.block_of(ue - 1);
+  if (i0 == i1) return;
+  const int tpr = D / 4, rows_per_block = kPfThreads / tpr;
+  const int r = blockIdx.x * rows_per_block + threadIdx.x / tpr, d0 = 4 * (threadIdx.x % tpr);
+  const int qi = rb * kPfUnitRows + r;
+  if ((int)threadIdx.x >= rows_per_block * tpr || r >= kPfUnitRows || qi >= p.qlen) return;
+  // Block i0's last fragment, or its first where its share starts with the unit.
+  auto at = [&](int i) { return (int64_t)(2 * i + (i == i0 && sh.start(i0) < us ? 1 : 0)) * kPfUnitRows + r; };
+  float M = -INFINITY;
+  for (int i = i0; i <= i1; ++i) M = fmaxf(M, p.ws_m[at(i)]);
+  float L = 0.f;
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  if (M != -INFINITY) {
+    for (int i = i0; i <= i1; ++i) {
+      const float m = p.ws_m[at(i)];
+      if (m == -INFINITY) continue;
+      const float w = __builtin_amdgcn_exp2f(m - M);
+      L += w * p.ws_l[at(i)];
+      acc += w * *reinterpret_cast<const f32x4_t *>(p.ws_o + at(i) * D + d0);
+    }
+  }
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const int b = bh / p.hq, h = bh - b * p.hq;
+  *reinterpret_cast<uint2 *>(p.out + ((((int64_t)b * p.qlen + qi) * p.hq + h) * D + d0) * 2) =
+      make_uint2(pack2<DT>(acc[0] * inv, acc[1] * inv), pack2<DT>(acc[2] * inv, acc[3] * inv));
 }
 
 // Head dims above 128, one tile at a time, every step in order: store the
@@ -949,7 +1159,7 @@ prefill_attn_kernel(PrefillParams p) {
   blk.finish(o, m_run, l_lane);
 }
 
-// Merges the key splits: out = sum_s 2^(m_s - M) o_s / sum_s 2^(m_s - M) l_s
+// Head dims above 128: merges the key splits, out = sum_s 2^(m_s - M) o_s / sum_s 2^(m_s - M) l_s
 // with M the largest running max.  D / 4 threads per output row, 4 dims
 // each; a row that saw no key in any split gets zeros.
 template <int DT>
@@ -980,12 +1190,11 @@ __global__ void __launch_bounds__(kPfThreads) prefill_combine_kernel(PrefillPara
 
 static int64_t div_up(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-// Key splits: enough (row block, batch row * head, split) units for about
-// two rounds of the GPU's block slots, at least two key tiles per split, at
-// most 8.  With the longest-first order a second round fills the slots the
-// short row blocks free; more splits only add partial rows to write and
-// merge (on the model's chunk, 4096 x 8192 keys with 12 heads: 3 splits 571,
-// 4 splits 523, 2 splits 537 TFLOP/s).
+// Key splits of head dims above 128: enough (row block, batch row * head,
+// split) units for about two rounds of the GPU's block slots, at least two
+// key tiles per split, at most 8.  With the longest-first order a second
+// round fills the slots the short row blocks free; more splits only add
+// partial rows to write and merge.
 static int prefill_splits(int Q, int rows, int BH, int cold_len, int hot_len, int slots) {
   const int64_t units = div_up(Q, rows) * BH, tiles = div_up(cold_len, kPfKeys) + div_up(hot_len, kPfKeys);
   if (units >= 2 * (int64_t)slots) return 1;
@@ -996,25 +1205,58 @@ static int prefill_splits(int Q, int rows, int BH, int cold_len, int hot_len, in
 // Block slots of the attention kernel: two blocks per compute unit.
 static int prefill_slots() { return 2 * device_cu_count(); }
 
+// Blocks that share the units of a head dim up to 128 (0: a block per unit):
+// the GPU's slots while the units are fewer than two rounds of them, but no
+// more than leave a block kPfShareTiles tiles (a share's partial rows cost
+// about that much to write and merge).
+constexpr int kPfShareTiles = 8;
+static int prefill_share_blocks(int Q, int BH, int cold_len, int hot_len, int slots) {
+  const int64_t units = div_up(Q, kPfUnitRows) * BH, tiles = div_up(cold_len, kPfKeys) + div_up(hot_len, kPfKeys);
+  if (units >= 2 * (int64_t)slots || units * tiles > INT32_MAX / 4 || tiles <= kPfShareTiles) return 0;
+  return (int)std::min<int64_t>(slots, std::max<int64_t>(units, units * tiles / kPfShareTiles));
+}
+
+static PfShares prefill_shares(int Q, int BH, int cold_len, int hot_len, bool masked, int blocks) {
+  PfShares s;
+  const int nct = (int)div_up(cold_len, kPfKeys), nht = (int)div_up(hot_len, kPfKeys), off = hot_len - Q;
+  s.nrb = (int)div_up(Q, kPfUnitRows);
+  s.tiles = nct + nht;
+  s.blocks = blocks;
+  if (masked && off >= 0) {
+    // Row block rb's last row sees hot columns up to 128 (rb + 1) - 1 + off.
+    s.a = nct + kPfUnitRows / kPfKeys + (int)div_up(off, kPfKeys);
+    s.step = kPfUnitRows / kPfKeys;
+  } else {
+    s.a = s.tiles;
+    s.step = 0;
+  }
+  s.head = s.before(s.nrb - 1) + s.tiles;
+  const int total = s.head * BH;
+  s.per = blocks > 0 ? total / blocks : 0;
+  s.rem = blocks > 0 ? total - s.per * blocks : 0;
+  return s;
+}
+
 struct PrefillWorkspace {
   size_t tiles_bytes, m_off, l_off, o_off, total;
-  int nsplit;
+  int nsplit, blocks;
 };
 
 static PrefillWorkspace prefill_workspace(int B, int hq, int D, int Q, int cold_len, int hot_len, int mask_b,
-                                          int mask_h, int nsplit) {
+                                          int mask_h) {
   PrefillWorkspace w;
-  w.nsplit = nsplit;
+  const bool shares = D <= 128;
+  w.nsplit = shares ? 1 : prefill_splits(Q, 64, B * hq, cold_len, hot_len, prefill_slots());
+  w.blocks = shares ? prefill_share_blocks(Q, B * hq, cold_len, hot_len, prefill_slots()) : 0;
   w.tiles_bytes = hot_len > 0 ? (size_t)mask_b * mask_h * div_up(Q, kPfRows) * div_up(hot_len, kPfKeys) : 0;
-  const size_t nrows = (size_t)B * Q * hq;
+  // Partial rows: every row of each split, or two units a share.
+  const size_t nrows = shares ? (size_t)2 * w.blocks * kPfUnitRows : w.nsplit > 1 ? (size_t)B * Q * hq * w.nsplit : 0;
   w.m_off = (w.tiles_bytes + 255) & ~size_t(255);
-  w.l_off = w.m_off + ((nrows * w.nsplit * 4 + 255) & ~size_t(255));
-  w.o_off = w.l_off + ((nrows * w.nsplit * 4 + 255) & ~size_t(255));
-  w.total = w.nsplit > 1 ? w.o_off + nrows * w.nsplit * D * 4 : w.tiles_bytes;
+  w.l_off = w.m_off + ((nrows * 4 + 255) & ~size_t(255));
+  w.o_off = w.l_off + ((nrows * 4 + 255) & ~size_t(255));
+  w.total = nrows > 0 ? w.o_off + nrows * D * 4 : w.tiles_bytes;
   return w;
 }
-
-static int prefill_rows(int D) { return D <= 128 ? 128 : 64; }  // query rows per block (PfShape)
 
 }  // namespace kiv
 
@@ -1025,8 +1267,7 @@ extern "C" {
 size_t kiv_prefill_workspace_size(int32_t batch, int32_t num_q_heads, int32_t head_dim, int32_t q_len,
                                   int32_t cold_len, int32_t hot_len) {
   if (batch < 1 || num_q_heads < 1 || head_dim < 1 || q_len < 1 || cold_len < 0 || hot_len < 0) return 0;
-  const int ns = prefill_splits(q_len, prefill_rows(head_dim), batch * num_q_heads, cold_len, hot_len, prefill_slots());
-  return prefill_workspace(batch, num_q_heads, head_dim, q_len, cold_len, hot_len, batch, num_q_heads, ns).total;
+  return prefill_workspace(batch, num_q_heads, head_dim, q_len, cold_len, hot_len, batch, num_q_heads).total;
 }
 
 int kiv_prefill_attention(const kiv_attention_args_t *a, kiv_stream_t stream) {
@@ -1101,15 +1342,15 @@ int kiv_prefill_attention(const kiv_attention_args_t *a, kiv_stream_t stream) {
   p.out = (char *)a->out;
   hipStream_t st = (hipStream_t)stream;
   const int mode = mk == KIV_MASK_BOOL ? PF_BOOL : (mk == KIV_MASK_NONE || mk == KIV_MASK_CAUSAL) ? PF_ARITH : PF_FLOAT;
-  const int nsplit = prefill_splits(Q, prefill_rows(D), B * hq, a->cold_len, a->hot_len, prefill_slots());
   const PrefillWorkspace w = prefill_workspace(B, hq, D, Q, a->cold_len, a->hot_len,
-                                               mode != PF_ARITH ? p.mask_b : 0, mode != PF_ARITH ? p.mask_h : 0, nsplit);
+                                               mode != PF_ARITH ? p.mask_b : 0, mode != PF_ARITH ? p.mask_h : 0);
   p.nsplit = w.nsplit;
+  p.sh = prefill_shares(Q, B * hq, a->cold_len, a->hot_len, mk != KIV_MASK_NONE, w.blocks);
   p.ws_m = p.ws_l = p.ws_o = nullptr;
   if (w.total > 0 && (!a->workspace || a->workspace_bytes < w.total || ((uintptr_t)a->workspace & 255)))
     return fail(KIV_ERR_INVALID, "%s: needs a 256-byte aligned workspace of %zu bytes (kiv_prefill_workspace_size)",
                 who, w.total);
-  if (w.nsplit > 1) {
+  if (w.nsplit > 1 || w.blocks > 0) {
     char *ws = (char *)a->workspace;
     p.ws_m = (float *)(ws + w.m_off);
     p.ws_l = (float *)(ws + w.l_off);
@@ -1127,7 +1368,7 @@ int kiv_prefill_attention(const kiv_attention_args_t *a, kiv_stream_t stream) {
     if constexpr (KTV == 16) {
       return (int)fail(KIV_ERR_UNSUPPORTED, "%s: head_dim 512 unsupported", who);
     } else {
-      const int64_t nblocks = div_up(Q, PfShape<KTV>::ROWS) * B * hq * p.nsplit;
+      const int64_t nblocks = w.blocks > 0 ? w.blocks : div_up(Q, PfShape<KTV>::ROWS) * B * hq * p.nsplit;
       if (nblocks > INT32_MAX) return (int)fail(KIV_ERR_UNSUPPORTED, "%s: too many query rows", who);
       const dim3 grid((unsigned)nblocks);
       auto launch = [&](auto dtc, auto mkc) {
@@ -1152,6 +1393,14 @@ int kiv_prefill_attention(const kiv_attention_args_t *a, kiv_stream_t stream) {
           hipLaunchKernelGGL(prefill_combine_kernel<DT_BF16>, cgrid, dim3(kPfThreads), 0, st, p, D);
         else
           hipLaunchKernelGGL(prefill_combine_kernel<DT_F16>, cgrid, dim3(kPfThreads), 0, st, p, D);
+      }
+      if (w.blocks > 0) {
+        const int rows_per_block = kPfThreads / (D / 4);
+        const dim3 mgrid((unsigned)div_up(std::min(Q, kPfUnitRows), rows_per_block), (unsigned)(p.sh.nrb * B * hq));
+        if (dt == KIV_DTYPE_BF16)
+          hipLaunchKernelGGL(prefill_merge_kernel<DT_BF16>, mgrid, dim3(kPfThreads), 0, st, p, D);
+        else
+          hipLaunchKernelGGL(prefill_merge_kernel<DT_F16>, mgrid, dim3(kPfThreads), 0, st, p, D);
       }
       return (int)KIV_OK;
     }

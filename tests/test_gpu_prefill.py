@@ -95,6 +95,14 @@ CASES = [
     ("short_query_key_splits", 1, 8, 2, 128, 40, 300, 1500, torch.bfloat16, "bool"),
     ("short_causal_key_splits_d64", 1, 4, 4, 64, 70, 0, 900, torch.float16, "causal"),
     ("d256_key_splits_batch", 2, 4, 1, 256, 20, 64, 500, torch.bfloat16, "none"),
+    # shares of the work that cut units anywhere: row blocks of unequal weight, a last one of one
+    # row, padded LDS rows (head_dim 96), retrieved tiles, masks that show tiles past the diagonal
+    ("share_cuts_causal_d96", 1, 4, 2, 96, 513, 0, 1537, torch.bfloat16, "causal"),
+    ("share_cuts_retrieved_bool_d32", 2, 4, 1, 32, 257, 70, 700, torch.float16, "bool"),
+    ("share_cuts_float_d128", 1, 3, 3, 128, 130, 65, 1100, torch.float16, "float"),
+    ("one_row_many_tiles_d64", 1, 8, 1, 64, 1, 1000, 3000, torch.bfloat16, "none"),
+    # two rounds of units: a block per unit, no shares
+    ("block_per_unit_d32", 2, 128, 8, 32, 512, 0, 520, torch.float16, "causal"),
 ]
 
 
