@@ -115,6 +115,31 @@ struct PrefillParams {
   PfShares sh;                // head dims up to 128: the blocks' shares (then ws_* are per partial, see there)
 };
 
+// N bytes at p, of any alignment (mask rows start anywhere: a hot window of
+// T columns puts consecutive rows T elements apart); the compiler emits one
+// vector load where the target allows it.
+template <typename T> __device__ __forceinline__ T load_any(const char *p) {
+  T v;
+  __builtin_memcpy(&v, p, sizeof(T));
+  return v;
+}
+// Four consecutive float-mask elements from element o on (base 2).
+__device__ __forceinline__ void float_bias4(const PrefillParams &p, int64_t o, float (&bias)[4]) {
+  if (p.mask_kind == KIV_MASK_F32) {
+    const uint4 v = load_any<uint4>(p.mask + 4 * o);
+    bias[0] = __uint_as_float(v.x) * kLog2e;
+    bias[1] = __uint_as_float(v.y) * kLog2e;
+    bias[2] = __uint_as_float(v.z) * kLog2e;
+    bias[3] = __uint_as_float(v.w) * kLog2e;
+    return;
+  }
+  const uint2 v = load_any<uint2>(p.mask + 2 * o);
+  const uint32_t w[4] = {v.x & 0xffffu, v.x >> 16, v.y & 0xffffu, v.y >> 16};
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    bias[i] = (p.mask_kind == KIV_MASK_F16 ? f16_bits_to_f32(w[i]) : bf16_bits_to_f32(w[i])) * kLog2e;
+}
+
 // Two fp32 values rounded to the dtype (hardware conversion, nearest even),
 // packed low-first.
 template <int DT> __device__ __forceinline__ uint32_t pack2(float a, float b) {
@@ -239,6 +264,8 @@ template <int DT, int KT, int MK> struct PfGeom {
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) bias[i] = (bits >> (8 * i)) & 0xffu ? 0.f : -INFINITY;
+    } else if (p.ms3 == 1 && n >= kPfKeys) {
+      float_bias4(p, mo, bias);
     } else {
 #pragma unroll
       for (int i = 0; i < 4; ++i) bias[i] = k4 + i < n ? float_bias(p, mo + (int64_t)i * p.ms3) : -INFINITY;
@@ -608,12 +635,12 @@ __global__ void __launch_bounds__(kPfThreads) mask_tiles_kernel(PrefillParams p)
   };
   if (row < p.qlen) {
     const int64_t o = mask_off(p, mb, mh, row, 0);
-    if (p.mask_kind == KIV_MASK_BOOL && p.ms3 == 1 && !(((uintptr_t)p.mask + o) & 15)) {
+    if (p.mask_kind == KIV_MASK_BOOL && p.ms3 == 1) {
       uint4 v[TPB];
 #pragma unroll
       for (int j = 0; j < TPB; ++j) {
         const int c0 = (kt0 + j) * kPfKeys + cq;
-        v[j] = c0 + 16 <= p.hot_len ? load16(p.mask + o + c0) : make_uint4(0, 0, 0, 0);
+        v[j] = c0 + 16 <= p.hot_len ? load_any<uint4>(p.mask + o + c0) : make_uint4(0, 0, 0, 0);
       }
 #pragma unroll
       for (int j = 0; j < TPB; ++j) {
@@ -629,6 +656,26 @@ __global__ void __launch_bounds__(kPfThreads) mask_tiles_kernel(PrefillParams p)
               any[j] |= vis;
               all[j] &= vis;
             }
+        } else {
+          scalar(o, c0, any[j], all[j]);
+        }
+      }
+    } else if (p.mask_kind != KIV_MASK_BOOL && p.ms3 == 1) {
+#pragma unroll
+      for (int j = 0; j < TPB; ++j) {
+        const int c0 = (kt0 + j) * kPfKeys + cq;
+        if (kt0 + j >= nkt) continue;
+        if (c0 + 16 <= p.hot_len) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            float v[4];
+            float_bias4(p, o + c0 + 4 * u, v);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              any[j] |= v[e] != -INFINITY;
+              all[j] &= v[e] == 0.f;
+            }
+          }
         } else {
           scalar(o, c0, any[j], all[j]);
         }
@@ -813,10 +860,9 @@ template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
     if (MK == PF_BOOL && !cold && cnt > 0) {
       const char *m = p.mask + mask_off(p, b, h, qr, key0 + 32 * half);
       uint32_t on = 0;
-      if (p.mask_vec4 && cnt == 32) {
-        uint32_t w[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) w[u] = *reinterpret_cast<const uint32_t *>(m + 4 * u);
+      if (p.ms3 == 1 && cnt == 32) {
+        const uint4 lo = load_any<uint4>(m), hi = load_any<uint4>(m + 16);
+        const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
         for (int u = 0; u < 8; ++u)
 #pragma unroll
@@ -850,7 +896,6 @@ template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
     for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        __builtin_amdgcn_sched_barrier(0);  // four keys at a time: few registers
         float bias[4];
         this->bias4(cold, key0, n, 32 * sub + 8 * u + 4 * hf, qc, row_mo, bias);
 #pragma unroll
@@ -1206,14 +1251,19 @@ static int prefill_splits(int Q, int rows, int BH, int cold_len, int hot_len, in
 static int prefill_slots() { return 2 * device_cu_count(); }
 
 // Blocks that share the units of a head dim up to 128 (0: a block per unit):
-// the GPU's slots while the units are fewer than two rounds of them, but no
-// more than leave a block kPfShareTiles tiles (a share's partial rows cost
-// about that much to write and merge).
+// the GPU's slots (two a compute unit) while the units are fewer than two
+// rounds of them, but no more than leave a block kPfShareTiles tiles, whose
+// partial rows cost about that much to write and merge (200 positions of 28
+// heads over 2,304 keys: 512 blocks of 4 tiles 24.6 + 14.6 us, 259 of 8 24.9
+// + 9.0); work that would then leave compute units idle is dealt to all of
+// them, down to two tiles a block.
 constexpr int kPfShareTiles = 8;
 static int prefill_share_blocks(int Q, int BH, int cold_len, int hot_len, int slots) {
   const int64_t units = div_up(Q, kPfUnitRows) * BH, tiles = div_up(cold_len, kPfKeys) + div_up(hot_len, kPfKeys);
-  if (units >= 2 * (int64_t)slots || units * tiles > INT32_MAX / 4 || tiles <= kPfShareTiles) return 0;
-  return (int)std::min<int64_t>(slots, std::max<int64_t>(units, units * tiles / kPfShareTiles));
+  if (units >= 2 * (int64_t)slots || units * tiles > INT32_MAX / 4 || tiles < 4) return 0;
+  const int64_t all = units * tiles, few = std::min<int64_t>(slots / 2, all / 2);
+  const int64_t blocks = std::min<int64_t>(slots, std::max<int64_t>(few, all / kPfShareTiles));
+  return (int)std::max<int64_t>(blocks, std::min<int64_t>(units, slots));
 }
 
 static PfShares prefill_shares(int Q, int BH, int cold_len, int hot_len, bool masked, int blocks) {
