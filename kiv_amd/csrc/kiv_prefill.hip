@@ -22,7 +22,7 @@
 // Head dims up to 128 (prefill_attn32_kernel, below): 32 query rows a wave,
 // the work dealt to the GPU's block slots in equal shares (PfShares).  The
 // model's chunk, 4096 x 8192 keys of 12 heads under a boolean mask: 230.6 ->
-// 185.0 us a call, 155 GFLOP; the attention kernel about 160 us, matrix
+// 183.8 us a call, 155 GFLOP; the attention kernel about 160 us, matrix
 // cores busy 43% of its cycles (28% before), bound by the issue of the
 // softmax beside the matrix instructions with two waves a SIMD.
 //
@@ -1116,6 +1116,7 @@ prefill_attn32_kernel(PrefillParams p) {
 // 2^(m_i - M) l_i over a unit's partials, M their largest running max.
 // Grid (pieces of rows, units): D / 4 threads per output row, 4 dims each;
 // blocks of whole units leave at once.  A row that saw no key gets zeros.
+constexpr int kMergeBatch = 4;
 template <int DT>
 __global__ void __launch_bounds__(kPfThreads) prefill_merge_kernel(PrefillParams p, int D) {
   const PfShares &sh = p.sh;
@@ -1129,18 +1130,36 @@ __global__ void __launch_bounds__(kPfThreads) prefill_merge_kernel(PrefillParams
   if ((int)threadIdx.x >= rows_per_block * tpr || r >= kPfUnitRows || qi >= p.qlen) return;
   // Block i0's last fragment, or its first where its share starts with the unit.
   auto at = [&](int i) { return (int64_t)(2 * i + (i == i0 && sh.start(i0) < us ? 1 : 0)) * kPfUnitRows + r; };
-  float M = -INFINITY;
-  for (int i = i0; i <= i1; ++i) M = fmaxf(M, p.ws_m[at(i)]);
-  float L = 0.f;
+  // kMergeBatch partials' loads in flight together, folded by their largest
+  // max (a unit of 9 partials, 28 x 16 rows: 10.6 us reading one at a time,
+  // 4.0 in batches).
+  float M = -INFINITY, L = 0.f;
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-  if (M != -INFINITY) {
-    for (int i = i0; i <= i1; ++i) {
-      const float m = p.ws_m[at(i)];
-      if (m == -INFINITY) continue;
-      const float w = __builtin_amdgcn_exp2f(m - M);
-      L += w * p.ws_l[at(i)];
-      acc += w * *reinterpret_cast<const f32x4_t *>(p.ws_o + at(i) * D + d0);
+  for (int f = i0; f <= i1; f += kMergeBatch) {
+    float ms[kMergeBatch], ls[kMergeBatch];
+    f32x4_t os[kMergeBatch];
+#pragma unroll
+    for (int u = 0; u < kMergeBatch; ++u) {
+      const bool in = f + u <= i1;
+      const int64_t x = at(in ? f + u : f);
+      ms[u] = in ? p.ws_m[x] : -INFINITY;
+      ls[u] = in ? p.ws_l[x] : 0.f;
+      os[u] = in ? *reinterpret_cast<const f32x4_t *>(p.ws_o + x * D + d0) : f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
+    float m = M;
+#pragma unroll
+    for (int u = 0; u < kMergeBatch; ++u) m = fmaxf(m, ms[u]);
+    if (m == -INFINITY) continue;
+    const float w0 = M == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(M - m);
+    L *= w0;
+    acc *= w0;
+#pragma unroll
+    for (int u = 0; u < kMergeBatch; ++u) {
+      const float w = ms[u] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms[u] - m);
+      L = fmaf(w, ls[u], L);
+      acc += w * os[u];
+    }
+    M = m;
   }
   const float inv = L > 0.f ? 1.f / L : 0.f;
   const int b = bh / p.hq, h = bh - b * p.hq;
