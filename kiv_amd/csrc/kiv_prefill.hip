@@ -108,7 +108,7 @@ struct PrefillParams {
   int batch, hq, hkv, qlen;
   float scale_log2;  // scaling * log2(e)
   char *out;
-  // Key splits (grid z): with nsplit > 1 each split writes its unnormalised
+  // Key splits (head dims above 128): with nsplit > 1 each split writes its unnormalised
   // rows and (running max, row sum) here and prefill_combine_kernel merges.
   int nsplit;
   float *ws_m, *ws_l, *ws_o;  // [nsplit][B*Q*Hq], [nsplit][B*Q*Hq], [nsplit][B*Q*Hq][D]
