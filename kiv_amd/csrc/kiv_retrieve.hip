@@ -3538,13 +3538,15 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
     SelectPlan sp{};
     if (sel_plan) sp = SelectPlan{pr.ub, pr.lb, s->kr, a->out_width, pr.thr, pr.plan, pr.ctl};
     // A long query's union list (kFineMfmaRows query rows per kv row and up,
-    // no page plan) is scored in one pass by fine_scan_query_kernel.  Where
-    // K comes from host memory and is staged, the first pass's scan still
-    // streams it (whole rows a wave; it writes the staging copy) and the
-    // other positions read the copy.
-    // (Several passes imply a union list and more than kFineMfmaRows rows.)
-    const bool query_scan = mfma && union_src == UNION_LIST && !sel_plan && G * Q >= kFineMfmaRows;
+    // no page plan), or several passes over a partial page alone (no union
+    // then), are scored in one pass by fine_scan_query_kernel.  Where K comes
+    // from host memory and is staged, the first pass's scan still streams it
+    // (whole rows a wave; it writes the staging copy) and the other positions
+    // read the copy.
+    const bool query_scan = mfma && !sel_plan && G * Q >= kFineMfmaRows && (union_src == UNION_LIST || passes > 1);
     const int first_q = mfma && !heads && (!query_scan || k_stage) ? std::min(Qb, Q) : 0;  // positions of the first scan
+    if (mfma && !heads && !query_scan && first_q < Q)
+      return fail(KIV_ERR_UNSUPPORTED, "kiv_retrieve: %d of %d query positions have no fine scan", Q - first_q, Q);
     if (heads) {
       // Tiles of 16 candidates over the blocks that run at once: six a
       // compute unit, four at head_dim 192 and 256 (by registers); more

@@ -989,6 +989,42 @@ def test_long_query_edges(cuda, name, w, batch, positions, tier):
         check_retrieval(store, oracle, cfg, w, data, q, min_det_c=0.3)
 
 
+PARTIAL_ONLY = [
+    # name, workload, batch, positions: several passes of query positions (Qb
+    # = 27, 24 and 96 here) over a cold tier that is one partial page
+    ("gqa7_d128", Workload("po1", 28, 4, 128, torch.bfloat16, hot=16, cold=100, top_pages=4, top_p=32, segment=1),
+     1, 40),
+    # more candidates than a block of the query scan takes, two batch rows
+    ("gqa4_d256_page256", Workload("po2", 8, 2, 256, torch.float16, hot=16, cold=201, top_pages=4, top_p=64,
+                                   segment=1, page_size=256), 2, 37),
+    ("mha_d64_one_position_past", Workload("po3", 12, 3, 64, torch.bfloat16, hot=16, cold=117, top_pages=4, top_p=5,
+                                           segment=1), 1, 97),
+]
+
+
+@pytest.mark.parametrize("tier", ["host", "hbm", "split"])
+@pytest.mark.parametrize("name,w,batch,positions", PARTIAL_ONLY, ids=[c[0] for c in PARTIAL_ONLY])
+def test_long_query_over_a_partial_page(cuda, name, w, batch, positions, tier):
+    """A long query over a store with no finished page: the tokens that the
+    positions past the first pass ask for are the best ones (keys drawn one by
+    one: a key's product with itself is far above any other).  Twice, the
+    second query asking for other tokens with lower scores (keys left behind
+    would win)."""
+    data = generate(w, seed=51, batch=batch)
+    g = torch.Generator().manual_seed(52)
+    store, oracle, cfg = build(w, data, cuda, cold_tier=tier)
+    assert store.num_pages == 0
+    asked = max(1, positions - 48 * 1024 // (w.groups * w.head_dim * 2))  # positions past the first pass
+    for call in range(2):
+        q = 0.01 * torch.randn(batch, w.num_q_heads, positions, w.head_dim, generator=g)
+        tokens = torch.randperm(w.cold, generator=g)[:min(asked, w.top_p)]
+        rows = data["cold_k"].float()[:, :, tokens].repeat_interleave(w.groups, dim=1)
+        q[:, :, positions - tokens.numel():] += (1.0 - 0.4 * call) * rows
+        _, _, sel = check_retrieval(store, oracle, cfg, w, data, q.to(w.dtype))
+        for b in range(batch):
+            assert set(tokens.tolist()) <= set(sel[b].tolist())
+
+
 WIDE_SELECTS = [
     # name, workload, batch, clustered query
     # 3 kv heads on 4 waves, 17 query rows per head (two operand tiles), 16-token pages
