@@ -735,8 +735,7 @@ template <int DT> __device__ __forceinline__ f32x16_t mfma_32x32x16(const uint4 
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c,
                                                    0, 0, 0);
 }
-constexpr int kWaitVm0 = 0x0f70;    // s_waitcnt vmcnt(0), the other counters unconstrained
-constexpr int kWaitLgkm0 = 0xc07f;  // s_waitcnt lgkmcnt(0)
+constexpr int kWaitMem = 0x0070;  // s_waitcnt vmcnt(0) lgkmcnt(0)
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) i16x4_t lds_i16x4_t;
@@ -1081,15 +1080,16 @@ prefill_attn32_kernel(PrefillParams p) {
     f32x16_t o[Blk::ND] = {};
     float m_run = -INFINITY, l_lane = 0.f;  // l_lane: this lane's share of the row sum
     // The tile's loads have arrived (each wave waits for its own, then the
-    // barrier), and every wave is done with the buffer the next ones fill.
+    // barrier), and every wave is done with the buffer the next ones fill:
+    // its reads of the tile before are issued ahead of the wait, which no
+    // memory access is moved across, and the wait covers them too.
     auto step = [&](uint16_t *ks, uint16_t *vs, uint16_t *kn, uint16_t *vn, uint32_t *vis) {
       int cls_n = TILE_FULL;
       const int tn = blk.find_tile(t + 1, cls_n);
-      if (MK != PF_FLOAT && cls == TILE_MIXED) {
-        blk.visible_bits(t, vis);
-        __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
-      }
-      __builtin_amdgcn_s_waitcnt(kWaitVm0);
+      if (MK != PF_FLOAT && cls == TILE_MIXED) blk.visible_bits(t, vis);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_waitcnt(kWaitMem);
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       if (tn < blk.t_end) blk.load_tile(tn, kn, vn);
