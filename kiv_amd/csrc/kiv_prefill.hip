@@ -54,43 +54,16 @@
 #include "kiv_common.h"
 #include "kiv_dispatch.h"
 #include "kiv_internal.h"
+#include "kiv_prefill_shares.h"
 
 namespace kiv {
 
 constexpr int kPfThreads = 256;
 constexpr int kPfRows = 64;  // query rows per mask tile class entry
-constexpr int kPfKeys = 64;  // keys per tile
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kRescaleSlack = 8.f;  // base-2 headroom before the running max moves
 enum { TILE_SKIP = 0, TILE_FULL = 1, TILE_MIXED = 2 };
 enum { PF_ARITH = 0, PF_BOOL = 1, PF_FLOAT = 2 };  // how MIXED tiles get their bias
-
-// Shares of the work of head dims up to 128.  A unit is a block of kPfUnitRows
-// query rows of one (b, q head); units are numbered heads first (unit = bh *
-// nrb + rb) and a unit's weight is its tiles: the retrieved keys' and the hot
-// keys' up to its last row's diagonal (every hot tile without a mask; a mask
-// tensor is taken to be causal, which only balances the shares).
-// blocks > 0: block i takes the weights [start(i), start(i + 1)), equal to
-// within one tile, through as many units as they span; a unit cut by a
-// share's end is merged from partial rows by prefill_merge_kernel: partial
-// 2 i is block i's first fragment, 2 i + 1 its last.  (Key splits of equal
-// tile ranges left 27% of the block slots' time empty on the model's chunk,
-// where a range may hold no visible tile; see prefill_attn32_kernel.)
-// blocks == 0: block i is one whole unit, longest first.
-struct PfShares {
-  int blocks, per, rem;   // start(i) = i * per + min(i, rem)
-  int nrb, head, a, step; // row blocks; weight of one (b, q head); weight of row block rb < nrb - 1: a + step * rb
-  int tiles;              // tiles of a unit (the last row block's weight)
-  __host__ __device__ int start(int i) const { return i * per + (i < rem ? i : rem); }
-  __host__ __device__ int block_of(int x) const {
-    const int cut = rem * (per + 1);
-    return x < cut ? x / (per + 1) : rem + (x - cut) / per;
-  }
-  // Weight of the row blocks before rb.
-  __host__ __device__ int before(int rb) const { return rb * a + step * (rb * (rb - 1) / 2); }
-  __host__ __device__ int weight(int rb) const { return rb + 1 == nrb ? tiles : a + step * rb; }
-};
-constexpr int kPfUnitRows = 128;
 
 struct PrefillParams {
   const char *q;
@@ -1044,31 +1017,14 @@ prefill_attn32_kernel(PrefillParams p) {
   Blk blk(p);
   const PfShares &sh = p.sh;
   // This block's units: a share's range of weights [w, w_end), or one unit.
-  int bh, rb, w, w_end, id = 0;
-  if (sh.blocks > 0) {
-    // Blocks are dealt to the eight dies in turn: a die takes consecutive
-    // shares, which read the same heads' keys through its L2.
-    id = (sh.blocks & 7) ? (int)blockIdx.x : (int)(blockIdx.x & 7) * (sh.blocks >> 3) + (int)(blockIdx.x >> 3);
-    w = sh.start(id);
-    w_end = sh.start(id + 1);
-    bh = w / sh.head;
-    const int rest = w - bh * sh.head;
-    rb = 0;  // the last row block that starts at or before it
-    for (int hi = sh.nrb - 1; rb < hi;) {
-      const int mid = (rb + hi + 1) >> 1;
-      if (sh.before(mid) <= rest) rb = mid;
-      else hi = mid - 1;
-    }
-  } else {
-    const int nbh = p.batch * p.hq, i = (int)blockIdx.x / nbh;
-    bh = (int)blockIdx.x - i * nbh;
-    rb = sh.nrb - 1 - i;  // longest first
-    w = bh * sh.head + sh.before(rb);
-    w_end = w + sh.weight(rb);
-  }
+  // Blocks are dealt to the eight dies in turn: a die takes consecutive
+  // shares, which read the same heads' keys through its L2.
+  int bh, rb, w, w_end, id = (int)blockIdx.x;
+  if (sh.blocks > 0 && !(sh.blocks & 7)) id = (id & 7) * (sh.blocks >> 3) + (id >> 3);
+  sh.first(id, p.batch * p.hq, bh, rb, w, w_end);
   const int w0 = w;
   while (w < w_end) {
-    const int us = bh * sh.head + sh.before(rb), ue = us + sh.weight(rb);
+    const int us = sh.unit_start(bh, rb), ue = us + sh.weight(rb);
     // A fragment that reaches the unit's end also takes the tiles past its
     // weight (hidden ones, unless a mask tensor is not causal).
     blk.set_unit(bh, rb, w - us, w_end >= ue ? sh.tiles : w_end - us);
@@ -1121,7 +1077,7 @@ template <int DT>
 __global__ void __launch_bounds__(kPfThreads) prefill_merge_kernel(PrefillParams p, int D) {
   const PfShares &sh = p.sh;
   const int bh = blockIdx.y / sh.nrb, rb = blockIdx.y - bh * sh.nrb;
-  const int us = bh * sh.head + sh.before(rb), ue = us + sh.weight(rb);
+  const int us = sh.unit_start(bh, rb), ue = us + sh.weight(rb);
   const int i0 = sh.block_of(us), i1 = sh.block_of(ue - 1);
   if (i0 == i1) return;
   const int tpr = D / 4, rows_per_block = kPfThreads / tpr;
@@ -1252,7 +1208,7 @@ __global__ void __launch_bounds__(kPfThreads) prefill_combine_kernel(PrefillPara
       make_uint2(pack2<DT>(acc[0] * inv, acc[1] * inv), pack2<DT>(acc[2] * inv, acc[3] * inv));
 }
 
-static int64_t div_up(int64_t a, int64_t b) { return (a + b - 1) / b; }
+static int64_t div_up(int64_t a, int64_t b) { return pf_div_up(a, b); }
 
 // Key splits of head dims above 128: enough (row block, batch row * head,
 // split) units for about two rounds of the GPU's block slots, at least two
@@ -1268,43 +1224,6 @@ static int prefill_splits(int Q, int rows, int BH, int cold_len, int hot_len, in
 
 // Block slots of the attention kernel: two blocks per compute unit.
 static int prefill_slots() { return 2 * device_cu_count(); }
-
-// Blocks that share the units of a head dim up to 128 (0: a block per unit):
-// the GPU's slots (two a compute unit) while the units are fewer than two
-// rounds of them, but no more than leave a block kPfShareTiles tiles, whose
-// partial rows cost about that much to write and merge (200 positions of 28
-// heads over 2,304 keys: 512 blocks of 4 tiles 24.6 + 14.6 us, 259 of 8 24.9
-// + 9.0); work that would then leave compute units idle is dealt to all of
-// them, down to two tiles a block.
-constexpr int kPfShareTiles = 8;
-static int prefill_share_blocks(int Q, int BH, int cold_len, int hot_len, int slots) {
-  const int64_t units = div_up(Q, kPfUnitRows) * BH, tiles = div_up(cold_len, kPfKeys) + div_up(hot_len, kPfKeys);
-  if (units >= 2 * (int64_t)slots || units * tiles > INT32_MAX / 4 || tiles < 4) return 0;
-  const int64_t all = units * tiles, few = std::min<int64_t>(slots / 2, all / 2);
-  const int64_t blocks = std::min<int64_t>(slots, std::max<int64_t>(few, all / kPfShareTiles));
-  return (int)std::max<int64_t>(blocks, std::min<int64_t>(units, slots));
-}
-
-static PfShares prefill_shares(int Q, int BH, int cold_len, int hot_len, bool masked, int blocks) {
-  PfShares s;
-  const int nct = (int)div_up(cold_len, kPfKeys), nht = (int)div_up(hot_len, kPfKeys), off = hot_len - Q;
-  s.nrb = (int)div_up(Q, kPfUnitRows);
-  s.tiles = nct + nht;
-  s.blocks = blocks;
-  if (masked && off >= 0) {
-    // Row block rb's last row sees hot columns up to 128 (rb + 1) - 1 + off.
-    s.a = nct + kPfUnitRows / kPfKeys + (int)div_up(off, kPfKeys);
-    s.step = kPfUnitRows / kPfKeys;
-  } else {
-    s.a = s.tiles;
-    s.step = 0;
-  }
-  s.head = s.before(s.nrb - 1) + s.tiles;
-  const int total = s.head * BH;
-  s.per = blocks > 0 ? total / blocks : 0;
-  s.rem = blocks > 0 ? total - s.per * blocks : 0;
-  return s;
-}
 
 struct PrefillWorkspace {
   size_t tiles_bytes, m_off, l_off, o_off, total;
