@@ -210,6 +210,18 @@ __device__ __forceinline__ uint32_t row_max_u32(uint32_t v) {
   return max(v, (uint32_t)dpp_i32<0x140>((int)v));
 }
 
+// Inclusive sum over the lanes up to the calling one.  All 64 lanes must be
+// active.
+__device__ __forceinline__ int wave_incl_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // row_shr 1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast 15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast 31 into rows 2 and 3
+  return v;
+}
+
 // Number of set bits of a wave mask below the calling lane.
 __device__ __forceinline__ int lane_rank(uint64_t mask) {
   return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));

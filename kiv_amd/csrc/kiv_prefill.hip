@@ -86,6 +86,12 @@ struct PrefillParams {
   int nsplit;
   float *ws_m, *ws_l, *ws_o;  // [nsplit][B*Q*Hq], [nsplit][B*Q*Hq], [nsplit][B*Q*Hq][D]
   PfShares sh;                // head dims up to 128: the blocks' shares (then ws_* are per partial, see there)
+  int2 *cuts;  // with shares, per unit: 2 * its first block + (not that block's first fragment), its last block
+  // Mask tensors under shares: a bit per hot tile that a 64-row entry sees,
+  // [Bm][Hm][2 * row blocks][1 << seen_shift] words, zero past the last tile
+  // and row.
+  uint32_t *seen;
+  int seen_shift;
 };
 
 // N bytes at p, of any alignment (mask rows start anywhere: a hot window of
@@ -155,7 +161,6 @@ template <int DT, int KT, int MK> struct PfGeom {
   int cls_n;
   const char *cold_kb, *cold_vb, *hot_kb, *hot_vb;
 
-
   __device__ __forceinline__ explicit PfGeom(const PrefillParams &pp) : p(pp) {
     z = 0;
     tid = threadIdx.x;
@@ -183,8 +188,9 @@ template <int DT, int KT, int MK> struct PfGeom {
     if constexpr (MK != PF_ARITH) {
       const int mb = p.mask_b == 1 ? 0 : b, mh = p.mask_h == 1 ? 0 : h;
       const int nqb = (p.qlen + 63) / 64, r0 = q0 / 64;
+      const int64_t entry = (int64_t)(mb * p.mask_h + mh) * nqb + r0;
       cls_n = min(ROWS / 64, nqb - r0);
-      cls_rows = p.tiles + ((int64_t)(mb * p.mask_h + mh) * nqb + r0) * nht;
+      cls_rows = p.tiles + entry * nht;
     }
     cold_kb = p.cold_k + ((int64_t)b * p.hkv + kvh) * p.cold_len * (int64_t)D * 2;
     cold_vb = p.cold_v + ((int64_t)b * p.hkv + kvh) * p.cold_len * (int64_t)D * 2;
@@ -666,15 +672,29 @@ __global__ void __launch_bounds__(kPfThreads) mask_tiles_kernel(PrefillParams p)
     }
   }
   __syncthreads();
+  if (wave != 0) return;
+  const int nqb = (p.qlen + kPfRows - 1) / kPfRows;
+  const int64_t entry = (int64_t)bh * nqb + qb;
+  int an = 0, al = 1;
   if (tid < TPB && kt0 + tid < nkt) {
-    int an = 0, al = 1;
 #pragma unroll
     for (int w = 0; w < W; ++w) {
       an |= wany[tid][w];
       al &= wall[tid][w];
     }
-    const int nqb = (p.qlen + kPfRows - 1) / kPfRows;
-    p.tiles[((int64_t)bh * nqb + qb) * nkt + kt0 + tid] = (uint8_t)(!an ? TILE_SKIP : al ? TILE_FULL : TILE_MIXED);
+    p.tiles[entry * nkt + kt0 + tid] = (uint8_t)(!an ? TILE_SKIP : al ? TILE_FULL : TILE_MIXED);
+  }
+  if (p.seen) {
+    // This block's byte of the row's bits; the last blocks also write the
+    // zeros after the row and a missing second row of the row block.
+    static_assert(TPB == 8, "a block's tiles are one byte of bits");
+    const uint64_t seen = __ballot(an);
+    const int bytes = 4 << p.seen_shift, last = blockIdx.x == gridDim.x - 1 ? bytes : (int)blockIdx.x + 1;
+    uint8_t *row = reinterpret_cast<uint8_t *>(p.seen) + ((int64_t)bh * 2 * p.sh.nrb + qb) * bytes;
+    for (int at = (int)blockIdx.x + tid; at < last; at += 64) {
+      row[at] = at == (int)blockIdx.x ? (uint8_t)seen : 0;
+      if (qb == nqb - 1 && !(qb & 1)) row[bytes + at] = 0;
+    }
   }
 }
 
@@ -753,7 +773,6 @@ template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
     Geom::set_unit(bh, rb, t0, t1);
     qi = q0 + 32 * wave + row;
     qc = min(qi, p.qlen - 1);
-    window(t0);
   }
   // The classes of 64 tiles in scalar registers, a tile a lane: the loop
   // finds its next tile with scalar bit operations.
@@ -762,6 +781,33 @@ template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
     const int t = base + lane, cls = t < t_end ? this->tile_class_of(t) : (int)TILE_SKIP;
     wseen = __ballot(cls != TILE_SKIP);
     wmixed = __ballot(cls == TILE_MIXED);
+  }
+  // Mask tensors: word base + lane of the unit's bits of visible hot tiles.
+  __device__ __forceinline__ uint32_t seen_bits(int base) const {
+    const int mb = p.mask_b == 1 ? 0 : b, mh = p.mask_h == 1 ? 0 : h, at = base + lane;
+    const uint32_t *row =
+        p.seen + (((int64_t)(mb * p.mask_h + mh) * p.sh.nrb * 2 + q0 / 64) << p.seen_shift) + at;
+    return at < 1 << p.seen_shift ? row[0] | row[1 << p.seen_shift] : 0u;
+  }
+  // The tile that v visible tiles of the unit precede (the retrieved keys'
+  // tiles are all visible), or all tiles past the last; bits: seen_bits(0).
+  __device__ __forceinline__ int locate(int v, uint32_t bits) const {
+    if (v < nct) return v;
+    v -= nct;
+    for (int base = 0; base < 1 << p.seen_shift; base += 64) {
+      if (base > 0) bits = seen_bits(base);
+      const int upto = wave_incl_scan(__popc(bits));  // visible tiles up to this lane's word
+      const uint64_t past = __ballot(upto > v);
+      if (past) {
+        const int l = __builtin_ctzll(past);
+        uint32_t word = (uint32_t)__builtin_amdgcn_readlane((int)bits, l);
+        int skip = v - (__builtin_amdgcn_readlane(upto, l) - __popc(word));
+        for (; skip > 0; --skip) word &= word - 1;
+        return nct + 32 * (base + l) + __builtin_ctz(word);
+      }
+      v -= __builtin_amdgcn_readlane(upto, 63);
+    }
+    return nct + this->nht;
   }
   // The first tile from t on that is not skipped (its class in cls), or t_end.
   __device__ __forceinline__ int find_tile(int t, int &cls) {
@@ -1006,6 +1052,137 @@ template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
   }
 };
 
+// Blocks are dealt to the eight dies in turn: a die takes consecutive
+// shares, which read the same heads' keys through its L2.
+__device__ __forceinline__ int die_order(int blocks) {
+  const int i = (int)blockIdx.x;
+  return blocks > 0 && !(blocks & 7) ? (i & 7) * (blocks >> 3) + (i >> 3) : i;
+}
+
+// Mask tensors: the weights of the units from the bits of their visible
+// tiles, kept as prefix sums over the mask's own (batch, head) planes: pre[u]
+// before row block u % nrb of plane u / nrb.  The heads that share a plane
+// repeat it.  A unit that sees no tile weighs one, so that a block writes its
+// rows.  (Shares by the causal rule's weights whatever the mask, where the
+// block that reached a unit's end took all the tiles past the diagonal: 4096
+// positions of 12 heads over 8192 keys, all visible 291 us a call, 240 by the
+// table; columns from the diagonal on 181 -> 110; documents of 512 tokens 61
+// -> 43.  The table costs a block about 3 us, mostly its code's first run, and
+// the test for the causal tiles about 1.)
+struct PfTable {
+  const PrefillParams &p;
+  const int *pre;
+  const int own, rep;  // own row blocks; heads that repeat a plane
+  __device__ __forceinline__ int at(int i) const { return __builtin_amdgcn_readfirstlane(pre[i]); }
+  __device__ __forceinline__ int first_own(int b, int h) const {
+    return ((p.mask_b == 1 ? 0 : b) * p.mask_h + (p.mask_h == 1 ? 0 : h)) * p.sh.nrb;
+  }
+  // Weights before batch row b.
+  __device__ __forceinline__ int batch_start(int b) const {
+    return p.mask_b == 1 ? b * rep * at(own) : rep * at(b * p.mask_h * p.sh.nrb);
+  }
+  __device__ __forceinline__ int total() const { return (p.mask_b == 1 ? p.batch : 1) * rep * at(own); }
+  // Weights [us, ue) of unit (bh, rb).
+  __device__ __forceinline__ void unit(int bh, int rb, int &us, int &ue) const {
+    const int b = bh / p.hq, h = bh - b * p.hq, o = first_own(b, h);
+    const int before = p.mask_h == 1 ? h * (at(o + p.sh.nrb) - at(o)) - at(o)
+                                     : -at(p.mask_b == 1 ? 0 : b * p.mask_h * p.sh.nrb);
+    us = batch_start(b) + before + at(o + rb);
+    ue = batch_start(b) + before + at(o + rb + 1);
+  }
+  // Of own row blocks [o, o + n): the last that starts at or before x.
+  __device__ __forceinline__ int find(int o, int n, int x) const {
+    const int lane = threadIdx.x & 63;
+    int i = 0;
+    for (int base = 0; base < n; base += 64) {
+      const uint64_t m = __ballot(base + lane < n && pre[o + min(base + lane, n - 1)] <= x);
+      i += __popcll(m);
+      if (m != ~uint64_t(0)) break;
+    }
+    return o + i - 1;
+  }
+  // The unit that weight w < total() falls in.
+  __device__ __forceinline__ void unit_of(int w, int &bh, int &rb) const {
+    const int nrb = p.sh.nrb;
+    int b = 0;
+    if (p.mask_b == 1) {
+      b = w / (rep * at(own));
+    } else {
+      while (b + 1 < p.batch && batch_start(b + 1) <= w) ++b;
+    }
+    const int o = first_own(b, 0);
+    int r = w - batch_start(b);
+    if (p.mask_h == 1) {
+      const int plane = at(o + nrb) - at(o), h = r / plane;
+      rb = find(o, nrb, at(o) + r - h * plane) - o;
+      bh = b * p.hq + h;
+    } else {
+      const int u = find(o, p.hq * nrb, at(o) + r) - o, h = u / nrb;
+      rb = u - h * nrb;
+      bh = b * p.hq + h;
+    }
+  }
+};
+
+// Whether every row block of a mask tensor sees just the tiles that the causal
+// rule's weights count (p.sh): the shares need no table then.  Called by the
+// whole block.
+__device__ __forceinline__ bool sees_causal_tiles(const PrefillParams &p, int own) {
+  __shared__ int other[kPfThreads / 64];
+  const int nct = (p.cold_len + kPfKeys - 1) / kPfKeys, nrb = p.sh.nrb, words = 1 << p.seen_shift;
+  bool differs = false;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < own << p.seen_shift; i += kPfThreads) {
+    const int u = i >> p.seen_shift, at = i & (words - 1);
+    const uint32_t *row = p.seen + ((int64_t)u << (p.seen_shift + 1)) + at;
+    const int n = p.sh.weight(own == nrb ? u : u % nrb) - nct - 32 * at;  // tiles from the word's first on
+    differs |= (row[0] | row[words]) != (n >= 32 ? ~0u : n <= 0 ? 0u : (1u << n) - 1u);
+  }
+  const uint64_t any = __ballot(differs);
+  if ((threadIdx.x & 63) == 0) other[threadIdx.x >> 6] = any != 0;
+  __syncthreads();
+  int all = 0;
+#pragma unroll
+  for (int i = 0; i < kPfThreads / 64; ++i) all |= other[i];
+  return __builtin_amdgcn_readfirstlane(all) == 0;
+}
+
+// Fills pre[0 .. own] by the whole block.
+__device__ __forceinline__ void fill_table(const PrefillParams &p, int *pre, int own) {
+  __shared__ int wsum[kPfThreads / 64];
+  const int tid = threadIdx.x, wave = tid >> 6;
+  const int nct = (p.cold_len + kPfKeys - 1) / kPfKeys;
+  // 1 << ls lanes a unit, a word of its two rows each at a time.
+  const int ls = min(p.seen_shift, 6), sub = tid & ((1 << ls) - 1);
+  for (int u = tid >> ls; u < own; u += kPfThreads >> ls) {
+    const uint32_t *row = p.seen + ((int64_t)u << (p.seen_shift + 1));
+    int n = 0;
+    for (int i = sub; i < 1 << p.seen_shift; i += 64) n += __popc(row[i] | row[i + (1 << p.seen_shift)]);
+    for (int o = 1; o < 1 << ls; o <<= 1) n += __shfl_xor(n, o, 64);
+    if (sub == 0) pre[u] = max(1, nct + n);
+  }
+  __syncthreads();
+  constexpr int PT = kPfMaxUnits / kPfThreads;  // row blocks a thread
+  int x[PT], mine = 0;
+#pragma unroll
+  for (int j = 0; j < PT; ++j) {
+    x[j] = PT * tid + j < own ? pre[PT * tid + j] : 0;
+    mine += x[j];
+  }
+  const int upto = wave_incl_scan(mine);
+  if ((tid & 63) == 63) wsum[wave] = upto;
+  __syncthreads();
+  int at = upto - mine;
+#pragma unroll
+  for (int i = 0; i < kPfThreads / 64 - 1; ++i) at += i < wave ? wsum[i] : 0;
+#pragma unroll
+  for (int j = 0; j < PT; ++j) {
+    if (PT * tid + j <= own) pre[PT * tid + j] = at;
+    at += x[j];
+  }
+  __syncthreads();
+}
+
 template <int DT, int KT, int MK>
 __global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
 prefill_attn32_kernel(PrefillParams p) {
@@ -1014,21 +1191,54 @@ prefill_attn32_kernel(PrefillParams p) {
   // tile's operand reads do not depend on the other buffer's loads.
   __shared__ __align__(1024) uint16_t k0[Blk::TILE], k1[Blk::TILE], v0[Blk::TILE], v1[Blk::TILE];
   __shared__ uint32_t vis0[2 * Blk::ROWS], vis1[2 * Blk::ROWS];
-  Blk blk(p);
-  const PfShares &sh = p.sh;
+  // Mask tensors: the units' weights (else arithmetic, see PfShares).
+  constexpr bool kTable = MK != PF_ARITH;
+  __shared__ int pre[kTable ? kPfMaxUnits : 1];
+  const PfTable tab{p, pre, p.mask_b * p.mask_h * p.sh.nrb, p.mask_h == 1 ? p.hq : 1};
+  bool table = false;
+  if constexpr (kTable) table = p.sh.blocks > 0 && !sees_causal_tiles(p, tab.own);
   // This block's units: a share's range of weights [w, w_end), or one unit.
-  // Blocks are dealt to the eight dies in turn: a die takes consecutive
-  // shares, which read the same heads' keys through its L2.
-  int bh, rb, w, w_end, id = (int)blockIdx.x;
-  if (sh.blocks > 0 && !(sh.blocks & 7)) id = (id & 7) * (sh.blocks >> 3) + (id >> 3);
-  sh.first(id, p.batch * p.hq, bh, rb, w, w_end);
+  int bh, rb, w, w_end, id;
+  if (table) {
+    PfShares sh = p.sh;
+    fill_table(p, pre, tab.own);
+    const int total = tab.total(), units = p.batch * p.hq * sh.nrb;
+    sh.deal(total, (int)pf_min(sh.blocks, share_blocks_of(total, units, sh.slots)));
+    if ((int)blockIdx.x >= sh.blocks) return;
+    id = die_order(sh.blocks);
+    w = sh.start(id);
+    w_end = sh.start(id + 1);
+    tab.unit_of(w, bh, rb);
+  } else {
+    id = die_order(p.sh.blocks);
+    p.sh.first(id, p.batch * p.hq, bh, rb, w, w_end);
+  }
+  Blk blk(p);
   const int w0 = w;
   while (w < w_end) {
-    const int us = sh.unit_start(bh, rb), ue = us + sh.weight(rb);
-    // A fragment that reaches the unit's end also takes the tiles past its
-    // weight (hidden ones, unless a mask tensor is not causal).
-    blk.set_unit(bh, rb, w - us, w_end >= ue ? sh.tiles : w_end - us);
-    const int partial = w == us && w_end >= ue ? -1 : 2 * id + (w == w0 ? 0 : 1);
+    int us, ue;
+    if (table) {
+      tab.unit(bh, rb, us, ue);
+    } else {
+      us = p.sh.unit_start(bh, rb);
+      ue = us + p.sh.weight(rb);
+    }
+    const bool ends = w_end >= ue;
+    const int frag = 2 * id + (w == w0 ? 0 : 1), partial = w == us && ends ? -1 : frag;
+    if (p.cuts && threadIdx.x == 0) {
+      int2 &cut = p.cuts[bh * p.sh.nrb + rb];
+      if (w == us) cut.x = frag;
+      if (ends) cut.y = id;
+    }
+    // Under a table a fragment is the unit's visible tiles [w - us, w_end - us);
+    // else all are visible up to there.
+    blk.set_unit(bh, rb, w - us, ends ? p.sh.tiles : w_end - us);
+    if (table) {
+      const uint32_t bits = blk.seen_bits(0);
+      if (w > us) blk.t_begin = blk.locate(w - us, bits);
+      if (!ends) blk.t_end = blk.locate(w_end - us, bits);
+    }
+    blk.window(blk.t_begin);
     int cls = TILE_FULL, t = blk.find_tile(blk.t_begin, cls);
     if (t < blk.t_end) blk.load_tile(t, k0, v0);
     uint4 qx[Blk::KS];
@@ -1060,7 +1270,7 @@ prefill_attn32_kernel(PrefillParams p) {
     }
     blk.finish(o, m_run, l_lane, partial);
     w = ue;
-    if (++rb == sh.nrb) {
+    if (++rb == p.sh.nrb) {
       rb = 0;
       ++bh;
     }
@@ -1075,17 +1285,15 @@ prefill_attn32_kernel(PrefillParams p) {
 constexpr int kMergeBatch = 4;
 template <int DT>
 __global__ void __launch_bounds__(kPfThreads) prefill_merge_kernel(PrefillParams p, int D) {
-  const PfShares &sh = p.sh;
-  const int bh = blockIdx.y / sh.nrb, rb = blockIdx.y - bh * sh.nrb;
-  const int us = sh.unit_start(bh, rb), ue = us + sh.weight(rb);
-  const int i0 = sh.block_of(us), i1 = sh.block_of(ue - 1);
+  const int nrb = p.sh.nrb, bh = blockIdx.y / nrb, rb = blockIdx.y - bh * nrb;
+  const int2 cut = p.cuts[blockIdx.y];
+  const int i0 = cut.x >> 1, i1 = cut.y;
   if (i0 == i1) return;
   const int tpr = D / 4, rows_per_block = kPfThreads / tpr;
   const int r = blockIdx.x * rows_per_block + threadIdx.x / tpr, d0 = 4 * (threadIdx.x % tpr);
   const int qi = rb * kPfUnitRows + r;
   if ((int)threadIdx.x >= rows_per_block * tpr || r >= kPfUnitRows || qi >= p.qlen) return;
-  // Block i0's last fragment, or its first where its share starts with the unit.
-  auto at = [&](int i) { return (int64_t)(2 * i + (i == i0 && sh.start(i0) < us ? 1 : 0)) * kPfUnitRows + r; };
+  auto at = [&](int i) { return (int64_t)(i == i0 ? cut.x : 2 * i) * kPfUnitRows + r; };
   // kMergeBatch partials' loads in flight together, folded by their largest
   // max (a unit of 9 partials, 28 x 16 rows: 10.6 us reading one at a time,
   // 4.0 in batches).
@@ -1226,8 +1434,8 @@ static int prefill_splits(int Q, int rows, int BH, int cold_len, int hot_len, in
 static int prefill_slots() { return 2 * device_cu_count(); }
 
 struct PrefillWorkspace {
-  size_t tiles_bytes, m_off, l_off, o_off, total;
-  int nsplit, blocks;
+  size_t tiles_bytes, seen_off, cuts_off, m_off, l_off, o_off, total;
+  int nsplit, blocks, seen_shift;
 };
 
 static PrefillWorkspace prefill_workspace(int B, int hq, int D, int Q, int cold_len, int hot_len, int mask_b,
@@ -1239,7 +1447,14 @@ static PrefillWorkspace prefill_workspace(int B, int hq, int D, int Q, int cold_
   w.tiles_bytes = hot_len > 0 ? (size_t)mask_b * mask_h * div_up(Q, kPfRows) * div_up(hot_len, kPfKeys) : 0;
   // Partial rows: every row of each split, or two units a share.
   const size_t nrows = shares ? (size_t)2 * w.blocks * kPfUnitRows : w.nsplit > 1 ? (size_t)B * Q * hq * w.nsplit : 0;
-  w.m_off = (w.tiles_bytes + 255) & ~size_t(255);
+  // With shares: the bits of a mask tensor's visible tiles and the units' cuts.
+  const int64_t nrb = div_up(Q, kPfUnitRows), words = div_up(div_up(hot_len, kPfKeys), 32);
+  for (w.seen_shift = 0; (int64_t(1) << w.seen_shift) < words;) ++w.seen_shift;
+  const size_t seen = w.blocks > 0 && w.tiles_bytes > 0 ? ((size_t)mask_b * mask_h * nrb * 8) << w.seen_shift : 0;
+  const size_t cuts = w.blocks > 0 ? (size_t)B * hq * nrb * sizeof(int2) : 0;
+  w.seen_off = (w.tiles_bytes + 255) & ~size_t(255);
+  w.cuts_off = w.seen_off + ((seen + 255) & ~size_t(255));
+  w.m_off = w.cuts_off + ((cuts + 255) & ~size_t(255));
   w.l_off = w.m_off + ((nrows * 4 + 255) & ~size_t(255));
   w.o_off = w.l_off + ((nrows * 4 + 255) & ~size_t(255));
   w.total = nrows > 0 ? w.o_off + nrows * D * 4 : w.tiles_bytes;
@@ -1333,7 +1548,7 @@ int kiv_prefill_attention(const kiv_attention_args_t *a, kiv_stream_t stream) {
   const PrefillWorkspace w = prefill_workspace(B, hq, D, Q, a->cold_len, a->hot_len,
                                                mode != PF_ARITH ? p.mask_b : 0, mode != PF_ARITH ? p.mask_h : 0);
   p.nsplit = w.nsplit;
-  p.sh = prefill_shares(Q, B * hq, a->cold_len, a->hot_len, mk != KIV_MASK_NONE, w.blocks);
+  p.sh = prefill_shares(Q, B * hq, a->cold_len, a->hot_len, mk != KIV_MASK_NONE, w.blocks, prefill_slots());
   p.ws_m = p.ws_l = p.ws_o = nullptr;
   if (w.total > 0 && (!a->workspace || a->workspace_bytes < w.total || ((uintptr_t)a->workspace & 255)))
     return fail(KIV_ERR_INVALID, "%s: needs a 256-byte aligned workspace of %zu bytes (kiv_prefill_workspace_size)",
@@ -1344,8 +1559,12 @@ int kiv_prefill_attention(const kiv_attention_args_t *a, kiv_stream_t stream) {
     p.ws_l = (float *)(ws + w.l_off);
     p.ws_o = (float *)(ws + w.o_off);
   }
+  p.seen = nullptr;
+  p.seen_shift = w.seen_shift;
+  p.cuts = w.blocks > 0 ? (int2 *)((char *)a->workspace + w.cuts_off) : nullptr;
   if (mode != PF_ARITH) {
     p.tiles = (uint8_t *)a->workspace;
+    if (w.blocks > 0) p.seen = (uint32_t *)((char *)a->workspace + w.seen_off);
     const dim3 cgrid((unsigned)div_up(div_up(a->hot_len, kPfKeys), kMaskTilesPerBlock), (unsigned)div_up(Q, kPfRows),
                      (unsigned)(p.mask_b * p.mask_h));
     if (cgrid.y > 65535 || cgrid.z > 65535) return fail(KIV_ERR_UNSUPPORTED, "%s: too many query rows", who);

@@ -133,6 +133,76 @@ def test_prefill_attention(cuda, case):
     check(q, cold_k, cold_v, hot_k, hot_v, scaling, mask=mask, causal=causal)
 
 
+def visible(pattern: str, Q: int, T: int, gen) -> torch.Tensor:
+    """[Q, T] visibility of a mask that need not follow the causal rule."""
+    i, t = torch.arange(Q)[:, None], torch.arange(T)[None, :]
+    causal = t <= i + (T - Q)
+    if pattern == "padded":  # bidirectional, the last columns padding
+        return (t < T - 37).expand(Q, T).clone()
+    if pattern == "prefix":
+        return causal | (t < 3 * T // 4)
+    if pattern == "window":
+        return causal & (t > i + (T - Q) - 200)
+    if pattern == "future":
+        return t >= i + (T - Q) - 64
+    if pattern == "documents":
+        return t // 300 == (i + T - Q) // 300
+    # whole 64 x 64 tiles hidden at random, and every column from 128 rows
+    # (a block of them) and from the last row
+    tiles = torch.rand(-(-Q // 64), -(-T // 64), generator=gen) < 0.2
+    vis = tiles.repeat_interleave(64, 0).repeat_interleave(64, 1)[:Q, :T].clone()
+    vis[:, 5] = True
+    vis[128:256] = False
+    vis[-1] = False
+    return vis
+
+
+VISIBLE = [
+    # name, B, Hq, Hkv, D, Q, retrieved P, hot T, dtype, pattern, mask rows of (batch, heads), float mask
+    ("padded_d128", 1, 4, 2, 128, 300, 0, 1900, torch.bfloat16, "padded", (1, 1), False),
+    ("padded_float_d64", 2, 4, 1, 64, 260, 0, 1000, torch.float16, "padded", (1, 1), True),
+    ("prefix_per_batch_d96", 3, 4, 2, 96, 200, 70, 900, torch.bfloat16, "prefix", (3, 1), False),
+    ("window_per_head_d32", 1, 6, 3, 32, 700, 0, 1100, torch.float16, "window", (1, 6), False),
+    ("future_retrieved_d64", 1, 4, 4, 64, 513, 100, 1400, torch.bfloat16, "future", (1, 1), False),
+    ("documents_d128_square", 1, 8, 2, 128, 1000, 0, 1000, torch.bfloat16, "documents", (1, 1), False),
+    ("tiles_per_batch_and_head_d64", 2, 3, 3, 64, 450, 0, 1300, torch.bfloat16, "tiles", (2, 3), False),
+    ("tiles_float_retrieved_d128", 1, 2, 1, 128, 400, 30, 700, torch.float16, "tiles", (1, 2), True),
+    # more tiles than a wave reads bits of at once (64 words of 32 tiles), a last word of few
+    ("many_tiles_d32", 1, 2, 2, 32, 130, 0, 64 * 2048 + 64 * 33 + 7, torch.bfloat16, "padded", (1, 1), False),
+    ("many_tiles_window_d32", 1, 2, 2, 32, 390, 0, 64 * 2048 + 64 * 31, torch.bfloat16, "window", (1, 1), False),
+    # the most units that are dealt in shares
+    ("1023_units_d32", 3, 341, 11, 32, 16, 0, 500, torch.float16, "future", (3, 1), False),
+]
+
+
+@pytest.mark.parametrize("case", VISIBLE, ids=[c[0] for c in VISIBLE])
+def test_prefill_attention_visible_tiles(cuda, case):
+    """Masks of any shape: the shares are cut where the visible tiles fall,
+    by batch row and head where the mask has them.  Rows that see nothing get
+    zeros, also where a whole block of rows sees nothing."""
+    name, B, hq, hkv, D, Q, P, T, dt, pattern, planes, as_float = case
+    print(f"prefill attention case {name}", flush=True)
+    gen = torch.Generator().manual_seed(sum(map(ord, name)))
+    q = rand((B, hq, Q, D), dt, gen).to(cuda)
+    hot_k, hot_v = (rand((B, hkv, T, D), dt, gen).to(cuda) for _ in range(2))
+    cold_k, cold_v = (rand((B, hkv, P, D), dt, gen).to(cuda) if P else None for _ in range(2))
+    vis = torch.stack([visible(pattern, Q, T, gen) for _ in range(planes[0] * planes[1])]).view(*planes, Q, T)
+    if pattern != "tiles":  # planes of their own: other columns hidden in each
+        for b in range(planes[0]):
+            for h in range(planes[1]):
+                vis[b, h, :, 64 * (b + h):64 * (b + h) + 20 * (b + h)] = False
+    mask = torch.where(vis, 0.0, float("-inf")).to(dt) if as_float else vis
+    out = prefill_attention(q, cold_k, cold_v, hot_k, hot_v, mask.to(cuda), D ** -0.5)
+    torch.cuda.synchronize()
+    seen = vis.any(-1).all(0).all(0) if P == 0 else torch.ones(Q, dtype=torch.bool)
+    assert torch.count_nonzero(out[:, ~seen.to(cuda)]) == 0
+    keep = seen.nonzero().flatten()
+    if T > 10000:  # rows of every unit, the first and last of each
+        keep = keep[(keep % 128 < 3) | (keep % 128 > 125) | (keep == Q - 1)]
+    at = keep.to(cuda)
+    check(q[:, :, at], cold_k, cold_v, hot_k, hot_v, D ** -0.5, mask=mask[:, :, keep], out=out[:, at])
+
+
 def test_prefill_attention_peaked_scores(cuda):
     """Queries aligned with a few keys (softmax close to one-hot): the
     probability rounding term is at its largest here."""

@@ -12,19 +12,20 @@ import pytest
 
 HEADER = Path(__file__).resolve().parents[1] / "kiv_amd" / "csrc" / "kiv_prefill_shares.h"
 
-# Prints, per shape "Q BH cold hot masked slots": blocks, units, fragments,
+# Prints, per shape "Q BH cold hot causal slots": blocks, units, fragments,
 # tiles taken, units not taken from first tile to last in one piece or in
 # consecutive fragments, and the largest and smallest share.
 WALK = r"""
 #include <stdio.h>
+#include <algorithm>
 #include <vector>
 #include "%s"
 using namespace kiv;
 int main() {
-  long long Q, BH, cold, hot, masked, slots;
-  while (scanf("%%lld %%lld %%lld %%lld %%lld %%lld", &Q, &BH, &cold, &hot, &masked, &slots) == 6) {
+  long long Q, BH, cold, hot, causal, slots;
+  while (scanf("%%lld %%lld %%lld %%lld %%lld %%lld", &Q, &BH, &cold, &hot, &causal, &slots) == 6) {
     const int nb = prefill_share_blocks(Q, BH, cold, hot, slots);
-    const PfShares sh = prefill_shares(Q, BH, cold, hot, masked, nb);
+    const PfShares sh = prefill_shares(Q, BH, cold, hot, causal, nb, slots);
     const long long units = (long long)sh.nrb * BH, grid = nb > 0 ? nb : units;
     std::vector<int> next(units, 0);  // first tile of the unit not taken yet
     std::vector<char> order(units, 1);
@@ -34,9 +35,9 @@ int main() {
       sh.first((int)i, (int)BH, bh, rb, w, w_end);
       long long mine = 0;
       while (w < w_end) {
+        const long long u = (long long)bh * sh.nrb + rb;
         const int us = sh.unit_start(bh, rb), ue = us + sh.weight(rb);
         const int t0 = w - us, t1 = w_end >= ue ? sh.tiles : w_end - us;
-        const long long u = (long long)bh * sh.nrb + rb;
         if (u < 0 || u >= units || t0 != next[u] || t1 <= t0) { if (u >= 0 && u < units) order[u] = 0; break; }
         next[u] = t1;
         mine += (w_end >= ue ? ue : w_end) - w;
@@ -75,7 +76,7 @@ def walk(tmp_path_factory):
 
 
 SHAPES = [
-    # Q, batch * heads, cold, hot, masked
+    # Q, batch * heads, cold, hot, causal
     (4096, 12, 0, 8192, 1), (777, 64, 0, 1531, 1), (1, 8, 1000, 3000, 0), (128, 1, 0, 256, 1), (129, 3, 65, 1100, 1),
     (513, 4, 0, 1537, 1), (200, 28, 256, 2048, 1), (500, 4, 70, 300, 1), (512, 256, 0, 520, 1), (4096, 12, 0, 8192, 0),
     # units of 2^31 tiles and more in all
@@ -88,7 +89,7 @@ SHAPES = [
 
 @pytest.mark.parametrize("shape", SHAPES, ids=["x".join(map(str, s)) for s in SHAPES])
 def test_every_tile_is_taken_once(walk, shape):
-    Q, bh, cold, hot, masked = shape
+    Q, bh, cold, hot, causal = shape
     blocks, units, frags, taken, bad, most, least = walk(*shape, 512)
     tiles = -(-cold // 64) + -(-hot // 64)
     assert units == -(-Q // 128) * bh
