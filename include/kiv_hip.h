@@ -312,10 +312,11 @@ int kiv_prefill_attention(const kiv_attention_args_t *args, kiv_stream_t stream)
 
 /* Workspace bytes kiv_prefill_attention needs for this shape (0: none): one
  * byte per 64 x 64 tile of query rows x hot columns per batch and q head for
- * a mask tensor's tile classes, plus fp32 partial rows when a unit of query
- * rows is divided among blocks (when the units are fewer than two rounds of
- * the GPU's block slots, as for the model's 4096-position chunks; up to
- * head_dim 128 two units of 128 rows a block, above it every row of each key
+ * a mask tensor's tile classes, a bit per tile for the visible ones, plus
+ * fp32 partial rows when a unit of query rows is divided among blocks (when
+ * the units are fewer than two rounds of the GPU's block slots, as for the
+ * model's 4096-position chunks; up to head_dim 128 two units a block, of 128
+ * rows or of the query's where it has fewer, above it every row of each key
  * split).  Their count depends on the current device's compute units: query
  * the size with the device of the call current.  The workspace must be
  * 256-byte aligned. */

@@ -85,7 +85,8 @@ struct PrefillParams {
   // rows and (running max, row sum) here and prefill_combine_kernel merges.
   int nsplit;
   float *ws_m, *ws_l, *ws_o;  // [nsplit][B*Q*Hq], [nsplit][B*Q*Hq], [nsplit][B*Q*Hq][D]
-  PfShares sh;                // head dims up to 128: the blocks' shares (then ws_* are per partial, see there)
+  PfShares sh;                // head dims up to 128: the blocks' shares (then ws_* are [2 * blocks][part_rows])
+  int part_rows;
   int2 *cuts;  // with shares, per unit: 2 * its first block + (not that block's first fragment), its last block
   // Mask tensors under shares: a bit per hot tile that a 64-row entry sees,
   // [Bm][Hm][2 * row blocks][1 << seen_shift] words, zero past the last tile
@@ -927,7 +928,7 @@ template <int DT, int KT, int MK> struct PfBlock32 : PfGeom<DT, KT, MK> {
     const float l_row = half_wave_sum(l_lane);
     if (qi >= p.qlen) return;
     if (partial >= 0) {
-      const int64_t sr = (int64_t)partial * kPfUnitRows + 32 * wave + row;
+      const int64_t sr = (int64_t)partial * p.part_rows + 32 * wave + row;
       float *po = p.ws_o + sr * D;
 #pragma unroll
       for (int dt = 0; dt < ND; ++dt)
@@ -1293,7 +1294,7 @@ __global__ void __launch_bounds__(kPfThreads) prefill_merge_kernel(PrefillParams
   const int r = blockIdx.x * rows_per_block + threadIdx.x / tpr, d0 = 4 * (threadIdx.x % tpr);
   const int qi = rb * kPfUnitRows + r;
   if ((int)threadIdx.x >= rows_per_block * tpr || r >= kPfUnitRows || qi >= p.qlen) return;
-  auto at = [&](int i) { return (int64_t)(i == i0 ? cut.x : 2 * i) * kPfUnitRows + r; };
+  auto at = [&](int i) { return (int64_t)(i == i0 ? cut.x : 2 * i) * p.part_rows + r; };
   // kMergeBatch partials' loads in flight together, folded by their largest
   // max (a unit of 9 partials, 28 x 16 rows: 10.6 us reading one at a time,
   // 4.0 in batches).
@@ -1433,6 +1434,9 @@ static int prefill_splits(int Q, int rows, int BH, int cold_len, int hot_len, in
 // Block slots of the attention kernel: two blocks per compute unit.
 static int prefill_slots() { return 2 * device_cu_count(); }
 
+// Rows of a partial: a unit's, of which one row block alone has only Q.
+static int part_rows(int Q) { return std::min(Q, kPfUnitRows); }
+
 struct PrefillWorkspace {
   size_t tiles_bytes, seen_off, cuts_off, m_off, l_off, o_off, total;
   int nsplit, blocks, seen_shift;
@@ -1446,7 +1450,7 @@ static PrefillWorkspace prefill_workspace(int B, int hq, int D, int Q, int cold_
   w.blocks = shares ? prefill_share_blocks(Q, B * hq, cold_len, hot_len, prefill_slots()) : 0;
   w.tiles_bytes = hot_len > 0 ? (size_t)mask_b * mask_h * div_up(Q, kPfRows) * div_up(hot_len, kPfKeys) : 0;
   // Partial rows: every row of each split, or two units a share.
-  const size_t nrows = shares ? (size_t)2 * w.blocks * kPfUnitRows : w.nsplit > 1 ? (size_t)B * Q * hq * w.nsplit : 0;
+  const size_t nrows = shares ? (size_t)2 * w.blocks * part_rows(Q) : w.nsplit > 1 ? (size_t)B * Q * hq * w.nsplit : 0;
   // With shares: the bits of a mask tensor's visible tiles and the units' cuts.
   const int64_t nrb = div_up(Q, kPfUnitRows), words = div_up(div_up(hot_len, kPfKeys), 32);
   for (w.seen_shift = 0; (int64_t(1) << w.seen_shift) < words;) ++w.seen_shift;
@@ -1549,6 +1553,7 @@ int kiv_prefill_attention(const kiv_attention_args_t *a, kiv_stream_t stream) {
                                                mode != PF_ARITH ? p.mask_b : 0, mode != PF_ARITH ? p.mask_h : 0);
   p.nsplit = w.nsplit;
   p.sh = prefill_shares(Q, B * hq, a->cold_len, a->hot_len, mk != KIV_MASK_NONE, w.blocks, prefill_slots());
+  p.part_rows = part_rows(Q);
   p.ws_m = p.ws_l = p.ws_o = nullptr;
   if (w.total > 0 && (!a->workspace || a->workspace_bytes < w.total || ((uintptr_t)a->workspace & 255)))
     return fail(KIV_ERR_INVALID, "%s: needs a 256-byte aligned workspace of %zu bytes (kiv_prefill_workspace_size)",
@@ -1603,7 +1608,7 @@ int kiv_prefill_attention(const kiv_attention_args_t *a, kiv_stream_t stream) {
       }
       if (w.blocks > 0) {
         const int rows_per_block = kPfThreads / (D / 4);
-        const dim3 mgrid((unsigned)div_up(std::min(Q, kPfUnitRows), rows_per_block), (unsigned)(p.sh.nrb * B * hq));
+        const dim3 mgrid((unsigned)div_up(part_rows(Q), rows_per_block), (unsigned)(p.sh.nrb * B * hq));
         if (dt == KIV_DTYPE_BF16)
           hipLaunchKernelGGL(prefill_merge_kernel<DT_BF16>, mgrid, dim3(kPfThreads), 0, st, p, D);
         else

@@ -66,6 +66,15 @@ def test_invalid_arguments_fail_without_gpu_work():
     assert lib.kiv_store_destroy(None) == 0
 
 
+@pytest.mark.parametrize("rows", [1, 16, 100])
+def test_prefill_workspace_holds_a_short_querys_rows_only(rows):
+    """Partial rows: at most two units a block slot (2 a compute unit, 256 of
+    them), of the query's rows, fp32 with a maximum and a sum each; beside
+    them a byte and a bit a tile, the units' cuts and the parts' alignment."""
+    need = _native.lib().kiv_prefill_workspace_size(1, 28, 128, rows, 256, 2048)
+    assert need <= 2 * 512 * rows * (128 * 4 + 8) + 28 * 2 * (32 + 8) + 28 * 8 + 6 * 256
+
+
 def test_struct_layouts_match_c():
     gcc = shutil.which("gcc")
     if gcc is None:
