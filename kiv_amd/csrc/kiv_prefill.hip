@@ -1125,19 +1125,24 @@ struct PfTable {
   }
 };
 
+// Word i of a mask tensor's own row blocks' bits, both 64-row entries.
+__device__ __forceinline__ uint32_t own_bits(const PrefillParams &p, int i) {
+  const int words = 1 << p.seen_shift;
+  const uint32_t *row = p.seen + ((int64_t)(i >> p.seen_shift) << (p.seen_shift + 1)) + (i & (words - 1));
+  return row[0] | row[words];
+}
 // Whether every row block of a mask tensor sees just the tiles that the causal
 // rule's weights count (p.sh): the shares need no table then.  Called by the
-// whole block.
-__device__ __forceinline__ bool sees_causal_tiles(const PrefillParams &p, int own) {
+// whole block; bits: own_bits of the thread's first word.
+__device__ __forceinline__ bool sees_causal_tiles(const PrefillParams &p, int own, uint32_t bits) {
   __shared__ int other[kPfThreads / 64];
-  const int nct = (p.cold_len + kPfKeys - 1) / kPfKeys, nrb = p.sh.nrb, words = 1 << p.seen_shift;
+  const int nct = (p.cold_len + kPfKeys - 1) / kPfKeys, nrb = p.sh.nrb;
   bool differs = false;
-#pragma unroll 4
   for (int i = threadIdx.x; i < own << p.seen_shift; i += kPfThreads) {
-    const int u = i >> p.seen_shift, at = i & (words - 1);
-    const uint32_t *row = p.seen + ((int64_t)u << (p.seen_shift + 1)) + at;
+    if (i >= kPfThreads) bits = own_bits(p, i);
+    const int u = i >> p.seen_shift, at = i & ((1 << p.seen_shift) - 1);
     const int n = p.sh.weight(own == nrb ? u : u % nrb) - nct - 32 * at;  // tiles from the word's first on
-    differs |= (row[0] | row[words]) != (n >= 32 ? ~0u : n <= 0 ? 0u : (1u << n) - 1u);
+    differs |= bits != (n >= 32 ? ~0u : n <= 0 ? 0u : (1u << n) - 1u);
   }
   const uint64_t any = __ballot(differs);
   if ((threadIdx.x & 63) == 0) other[threadIdx.x >> 6] = any != 0;
@@ -1196,10 +1201,14 @@ prefill_attn32_kernel(PrefillParams p) {
   constexpr bool kTable = MK != PF_ARITH;
   __shared__ int pre[kTable ? kPfMaxUnits : 1];
   const PfTable tab{p, pre, p.mask_b * p.mask_h * p.sh.nrb, p.mask_h == 1 ? p.hq : 1};
-  bool table = false;
-  if constexpr (kTable) table = p.sh.blocks > 0 && !sees_causal_tiles(p, tab.own);
+  uint32_t bits = 0u;
+  if (kTable && p.sh.blocks > 0 && (int)threadIdx.x < tab.own << p.seen_shift) bits = own_bits(p, threadIdx.x);
   // This block's units: a share's range of weights [w, w_end), or one unit.
-  int bh, rb, w, w_end, id;
+  int bh, rb, w, w_end, id = die_order(p.sh.blocks);
+  p.sh.first(id, p.batch * p.hq, bh, rb, w, w_end);
+  Blk blk(p);
+  bool table = false;
+  if constexpr (kTable) table = p.sh.blocks > 0 && !sees_causal_tiles(p, tab.own, bits);
   if (table) {
     PfShares sh = p.sh;
     fill_table(p, pre, tab.own);
@@ -1210,11 +1219,7 @@ prefill_attn32_kernel(PrefillParams p) {
     w = sh.start(id);
     w_end = sh.start(id + 1);
     tab.unit_of(w, bh, rb);
-  } else {
-    id = die_order(p.sh.blocks);
-    p.sh.first(id, p.batch * p.hq, bh, rb, w, w_end);
   }
-  Blk blk(p);
   const int w0 = w;
   while (w < w_end) {
     int us, ue;
@@ -1235,7 +1240,7 @@ prefill_attn32_kernel(PrefillParams p) {
     // else all are visible up to there.
     blk.set_unit(bh, rb, w - us, ends ? p.sh.tiles : w_end - us);
     if (table) {
-      const uint32_t bits = blk.seen_bits(0);
+      bits = blk.seen_bits(0);
       if (w > us) blk.t_begin = blk.locate(w - us, bits);
       if (!ends) blk.t_end = blk.locate(w_end - us, bits);
     }
