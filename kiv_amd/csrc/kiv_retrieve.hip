@@ -887,10 +887,10 @@ __global__ void __launch_bounds__(kScanMfmaThreads) coarse_scan_mfma_kernel(
     const char *__restrict__ summ, int64_t n_pages, int kr, const char *__restrict__ q, int64_t qs0,
     int64_t qs1, int64_t qs2, int hq, int hkv, int qlen, float scale, int round, uint32_t *__restrict__ keys,
     int64_t ld, const float *__restrict__ rad2, uint32_t *__restrict__ ubk, uint32_t *__restrict__ lbk,
-    const int32_t *__restrict__ ctl, AppendRows ap, int zrows) {
+    const int32_t *__restrict__ ctl, AppendRows ap) {
   static_assert(DT != DT_F32, "16-bit dtypes only");
   if ((ap.count > 0 || ap.hot_count > 0) && blockIdx.x == gridDim.x - 1) {
-    if (blockIdx.z == 0) append_rows(ap, blockIdx.y);  // the step's evicted rows (an extra block per kv row)
+    if (!SL || blockIdx.z == 0) append_rows(ap, blockIdx.y);  // the step's evicted rows (an extra block per kv row)
     return;
   }
   constexpr int64_t kRowBytes = (int64_t)KT * 64;  // 32 two-byte elements per K step
@@ -916,7 +916,8 @@ __global__ void __launch_bounds__(kScanMfmaThreads) coarse_scan_mfma_kernel(
   // Loads in the order they are used: the first 16 query rows' operands
   // and, for the bounds, the page row's radius and |s|, then the summaries,
   // so that the rows' norms are computed while the summaries are in flight.
-  const int mz = SL ? (int)blockIdx.z * zrows : 0, mend = SL ? min(GQ, mz + zrows) : GQ;  // this slice's query rows
+  // This slice's query rows.
+  const int mz = SL ? (int)blockIdx.z * kScanRowsPerSlice : 0, mend = SL ? min(GQ, mz + kScanRowsPerSlice) : GQ;
   uint4 q0[KT];
   q_tile(mz, q0);
   if constexpr (SL) ubk = nullptr;
@@ -3301,8 +3302,7 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
         if (mfma) {
           const int pages_per_block = (kScanMfmaThreads / 64) * kScanMfmaPages;
           const int blocks = (int)(((int64_t)N + pages_per_block - 1) / pages_per_block);
-          const int zrows = pr.ub ? G * Qp : std::min(G * Qp, kScanRowsPerSlice);
-          const unsigned zn = (unsigned)((G * Qp + zrows - 1) / zrows);
+          const unsigned zn = pr.ub ? 1u : (unsigned)((G * Qp + kScanRowsPerSlice - 1) / kScanRowsPerSlice);
           rc = with_dt(dt, [&](auto dtc) {
             constexpr int DTV = decltype(dtc)::value;
             if constexpr (DTV == DT_F32) {
@@ -3314,8 +3314,7 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
                 hipLaunchKernelGGL(kern, dim3(blocks + extra, s->kr, zn), dim3(kScanMfmaThreads), 0, st,
                                    (const char *)s->summ.ptr, (int64_t)N, s->kr, qp, a->q_stride[0], a->q_stride[1],
                                    a->q_stride[2], hq, hkv, Qp, a->scaling, round, (uint32_t *)s->coarse_keys.ptr, ld,
-                                   (const float *)s->radius.ptr, (uint32_t *)pr.ub, (uint32_t *)pr.lb, pr.ctl, apass,
-                                   zrows);
+                                   (const float *)s->radius.ptr, (uint32_t *)pr.ub, (uint32_t *)pr.lb, pr.ctl, apass);
                 return (int)KIV_OK;
               });
             }
