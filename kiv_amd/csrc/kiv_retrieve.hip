@@ -370,7 +370,8 @@ template <int NT> struct MemKeys4 {
 // sum and the number of scored entries in nz: a zero key is an entry that
 // was not scored (a pruned fine scan leaves them) and is not summed.
 template <int NT, typename Src>
-__device__ uint32_t row_bound(const Src &src, int k, SelSh<NT> &sh, float &mx, float &sum, int &nz) {
+__device__ int bound_candidates(const Src &src, int k, SelSh<NT> &sh, uint64_t *cand, float &mx, float &sum,
+                                int &nz) {
   constexpr int W = NT / 64;
   const int tid = threadIdx.x, wave = tid >> 6;
   uint32_t m[4] = {0u, 0u, 0u, 0u};
@@ -411,13 +412,6 @@ __device__ uint32_t row_bound(const Src &src, int k, SelSh<NT> &sh, float &mx, f
     nz += sh.fcnt[w];
     bound = min(bound, sh.wave_bound[w]);
   }
-  return bound;
-}
-// The composites of keys >= bound into cand[] (at most cap); returns their
-// number.
-template <int NT, typename Src>
-__device__ int place_candidates(const Src &src, uint32_t bound, SelSh<NT> &sh, uint64_t *cand, int cap) {
-  const int tid = threadIdx.x;
   if constexpr (Src::kManySteps) {
     // Many register steps per thread: a first pass sums the steps' ballot
     // counts, one LDS atomic per wave reserves the wave's range, a second
@@ -436,25 +430,18 @@ __device__ int place_candidates(const Src &src, uint32_t bound, SelSh<NT> &sh, u
         const uint64_t mask = __ballot(f);
         if (f) {
           const int pos = off + lane_rank(mask);
-          if (pos < cap) cand[pos] = x;
+          if (pos < kCandCap) cand[pos] = x;
         }
         off += __popcll(mask);
       });
     }
   } else {
     block_compact<NT>(src, [bound](uint64_t x) { return comp_key(x) >= bound; },
-                      [cand](int pos, uint64_t x) { cand[pos] = x; }, cap, &sh.ncand);
+                      [cand](int pos, uint64_t x) { cand[pos] = x; }, kCandCap, &sh.ncand);
   }
   __syncthreads();
   return sh.ncand;
 }
-template <int NT, typename Src>
-__device__ int bound_candidates(const Src &src, int k, SelSh<NT> &sh, uint64_t *cand, float &mx, float &sum,
-                                int &nz) {
-  const uint32_t bound = row_bound<NT>(src, k, sh, mx, sum, nz);
-  return place_candidates<NT>(src, bound, sh, cand, kCandCap);
-}
-
 // Calls ranked(x, r) for each of the top k composites of the C candidates
 // in cand[] (C <= kRankCap), r = its rank (0 = largest): a candidate's rank
 // is the number of larger candidates.  A group of tpc lanes (a power of two,
@@ -2628,13 +2615,15 @@ __global__ void __launch_bounds__(NT) fine_select_kernel(
     int zero_all, const int32_t *__restrict__ ctl, SelectGroups sg, int keep) {
   __shared__ SelSh<NT> sh;
   __shared__ SelSh<kSelThreads> sh_few;  // a wide block's few-page select
-  // [cand][plist], or the wide select's [keys][groups] in the same place.
+  // The wide select's [keys][groups] take the place of [cand][plist].
   constexpr size_t kPlain = kCandCap * sizeof(uint64_t) + kPageListCap * sizeof(int);
   constexpr size_t kWide = kGroupKeyCap * sizeof(uint64_t) + kGroupCap * sizeof(int);
-  __shared__ __align__(16) char pool[GR && kWide > kPlain ? kWide : kPlain];
+  __shared__ __align__(16) char pool[!GR ? 1 : kWide > kPlain ? kWide : kPlain];
+  __shared__ uint64_t cand_own[GR ? 1 : kCandCap];
+  __shared__ int plist_own[GR ? 1 : kPageListCap];
   __shared__ int gcnt[3];
-  uint64_t *cand = reinterpret_cast<uint64_t *>(pool);
-  int *plist = reinterpret_cast<int *>(cand + kCandCap);
+  uint64_t *cand = GR ? reinterpret_cast<uint64_t *>(pool) : cand_own;
+  int *plist = GR ? reinterpret_cast<int *>(cand + kCandCap) : plist_own;
   const int U = has_pages ? counters[0] : 0;
   const int n = U * page_size + partial_len;
   const int batch = GR ? sg.batch : (int)gridDim.x;
@@ -2817,13 +2806,13 @@ __device__ inline void clear_keys(const GatherArgs &ga, int i) {
 }
 
 // The fine telemetry (max and mean over the batch rows) and the pruning
-// control, run by one block of its own after the gather blocks: its global
-// reads then delay no copy.
-template <int DT> __device__ void gather_telemetry(const GatherArgs &ga) {
-  if (threadIdx.x >= 64) return;
+// control, run by one block of its own, so that its global reads delay no
+// copy.  WIDE: with the segments' sums of a wide select.
+template <int DT, bool WIDE> __device__ void gather_telemetry(const GatherArgs &ga) {
+  if (threadIdx.x >= (WIDE ? 64 : 1)) return;
   // Every load that the results need is issued before any is used: this
   // block's chain of round trips must not outlast the gather.
-  const int batch = ga.batch, lane = threadIdx.x;
+  const int batch = ga.batch, lane = (int)threadIdx.x;
   const int32_t *list_count = ga.list_count;
   const int U = ga.has_pages ? ga.counters[0] : 0;
   const int c0 = ga.ctl ? ga.ctl[0] : 0;
@@ -2837,8 +2826,8 @@ template <int DT> __device__ void gather_telemetry(const GatherArgs &ga) {
     float mr = ga.fine_stats[2 * r];
     double sr = ga.fine_stats[2 * r + 1];
     read += list_count[2 * batch + r];
-    if (ga.sums) {
-      // A wide select's segments, over the wave's lanes (nz -1: taken).
+    if constexpr (WIDE) {
+      // The segments, over the wave's lanes (nz -1: taken).
       double ts = 0.0;
       float ms = -INFINITY;
       int cs = 0;
@@ -2964,32 +2953,38 @@ template <int DT> __device__ void gather_block(const GatherArgs &ga, int bx, int
   }
 }
 
-// The first block runs the telemetry, the next gx * B gather (block 1 + i:
-// entries of batch row i / gx), any after them clear keys.
-template <int DT> __global__ void __launch_bounds__(256) gather_kernel(GatherArgs ga, int gx) {
-  const int i = (int)blockIdx.x - 1, gather_blocks = gx * ga.batch;
-  if (i < 0) gather_telemetry<DT>(ga);
+// gx * B blocks gather (block i: entries of batch row i / gx) and one more
+// runs the telemetry.  WIDE, after a wide select: that block is the launch's
+// first, as the segments' sums would make it outlast the gather, and blocks
+// after the gather's clear keys.  (One form for both: the smallest decode
+// step's launch 6.3 -> 6.6 us.)
+template <int DT, bool WIDE> __global__ void __launch_bounds__(256) gather_kernel(GatherArgs ga, int gx) {
+  const int i = (int)blockIdx.x - (WIDE ? 1 : 0), gather_blocks = gx * ga.batch;
+  if (WIDE && i < 0) gather_telemetry<DT, WIDE>(ga);
   else if (i < gather_blocks) gather_block<DT>(ga, i % gx, i / gx);
-  else clear_keys(ga, i - gather_blocks);
+  else if constexpr (WIDE) clear_keys(ga, i - gather_blocks);
+  else gather_telemetry<DT, WIDE>(ga);
 }
 
 // The gather plus the hot window's attention splits (kiv_retrieve_attend):
-// the first block runs the telemetry, the next gx * B gather, the s_hot * R
-// blocks after them each run one hot split of one kv row, any after those
-// clear keys.  The splits do not depend on the retrieval, so they run
-// alongside the gather instead of after it.
-template <int DT, int KT>
+// after the gather blocks, s_hot * R blocks each run one hot split of one kv
+// row.  The splits do not depend on the retrieval, so they run alongside the
+// gather instead of after it.
+template <int DT, int KT, bool WIDE>
 __global__ void __launch_bounds__(256) gather_attn_kernel(GatherArgs ga, AttnParams p, int gx, int s_hot) {
-  const int i = (int)blockIdx.x - 1, gather_blocks = gx * ga.batch, splits = s_hot * ga.batch * ga.hkv;
-  if (i < 0) {
-    gather_telemetry<DT>(ga);
+  const int i = (int)blockIdx.x - (WIDE ? 1 : 0);
+  const int gather_blocks = gx * ga.batch, splits = s_hot * ga.batch * ga.hkv;
+  if (WIDE && i < 0) {
+    gather_telemetry<DT, WIDE>(ga);
   } else if (i < gather_blocks) {
     gather_block<DT>(ga, i % gx, i / gx);
   } else if (i < gather_blocks + splits) {
     const int j = i - gather_blocks;
     attn_mfma_split<DT, KT>(p, j % s_hot, j / s_hot);
-  } else {
+  } else if constexpr (WIDE) {
     clear_keys(ga, i - gather_blocks - splits);
+  } else {
+    gather_telemetry<DT, WIDE>(ga);
   }
 }
 
@@ -3695,17 +3690,22 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
                          (const int32_t *)s->page_list.ptr, (const int32_t *)pr.plan, sel_plan ? 1 : 0, pr.ctl, sg,
                          heads ? 1 : 0);
     };
-    if (groups)
-      launch(sel_plan ? fine_select_kernel<1, kWideSelThreads, true, true>
-                      : fine_select_kernel<1, kWideSelThreads, true, false>, kWideSelThreads);
-    else if (wide)
-      with_select_chunks<kWideSelThreads>(cmax, [&](auto kern) { launch(kern, kWideSelThreads); }, [](auto vc) {
-        return fine_select_kernel<decltype(vc)::value, kWideSelThreads, false, true>;
-      });
-    else
-      with_select_chunks<kSelThreads>(cmax, [&](auto kern) { launch(kern, kSelThreads); }, [](auto vc) {
-        return fine_select_kernel<decltype(vc)::value, kSelThreads, false, true>;
-      });
+    auto by_bounds = [&](auto plc) {
+      constexpr bool PL = decltype(plc)::value;
+      if (groups) {
+        launch(fine_select_kernel<1, kWideSelThreads, true, PL>, kWideSelThreads);
+      } else if (wide) {
+        with_select_chunks<kWideSelThreads>(cmax, [&](auto kern) { launch(kern, kWideSelThreads); }, [](auto vc) {
+          return fine_select_kernel<decltype(vc)::value, kWideSelThreads, false, PL>;
+        });
+      } else {
+        with_select_chunks<kSelThreads>(cmax, [&](auto kern) { launch(kern, kSelThreads); }, [](auto vc) {
+          return fine_select_kernel<decltype(vc)::value, kSelThreads, false, PL>;
+        });
+      }
+    };
+    if (pr_ub) by_bounds(std::true_type{});
+    else by_bounds(std::false_type{});
     s->prof_end(KIV_STAGE_FINE_SELECT, st);
     KIV_HIP(hipGetLastError());
   }
@@ -3765,7 +3765,8 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
           return fail(KIV_ERR_UNSUPPORTED, "kiv_retrieve_attend: no fused path for fp32");
         } else {
           return with_kt(fa->kt, [&](auto ktc) {
-            auto kern = gather_attn_kernel<DTV, decltype(ktc)::value>;
+            constexpr int KTV = decltype(ktc)::value;
+            auto kern = groups ? gather_attn_kernel<DTV, KTV, true> : gather_attn_kernel<DTV, KTV, false>;
             if (fa->lds > 65536)
               KIV_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                           (int)fa->lds));
@@ -3776,8 +3777,12 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
       });
     } else {
       rc = with_dt(dt, [&](auto dtc) {
-        hipLaunchKernelGGL((gather_kernel<decltype(dtc)::value>), dim3(gx * (unsigned)B + 1 + clears), dim3(256), 0, st, ga,
-                           (int)gx);
+        constexpr int DTV = decltype(dtc)::value;
+        auto launch = [&](auto kern) {
+          hipLaunchKernelGGL(kern, dim3(gx * (unsigned)B + 1 + clears), dim3(256), 0, st, ga, (int)gx);
+        };
+        if constexpr (DTV == DT_F32) launch(gather_kernel<DTV, false>);  // its scan leaves no group maxima
+        else launch(groups ? gather_kernel<DTV, true> : gather_kernel<DTV, false>);
         return (int)KIV_OK;
       });
     }
