@@ -979,7 +979,9 @@ LONG_EDGES = [
 @pytest.mark.parametrize("name,w,batch,positions", LONG_EDGES, ids=[c[0] for c in LONG_EDGES])
 def test_long_query_edges(cuda, name, w, batch, positions, tier):
     """Long queries at the edges of the scans' tiles and passes, against the
-    oracle's bar, twice in a row (keys left behind would show in the second)."""
+    oracle's bar, twice in a row (keys left behind would show in the second).
+    Their rows are short enough for the select to clear them itself; see
+    test_long_query_clears_folded_keys for the wide select's."""
     data = generate(w, seed=17, batch=batch)
     g = torch.Generator().manual_seed(18)
     store, oracle, cfg = build(w, data, cuda, cold_tier=tier)
@@ -987,6 +989,52 @@ def test_long_query_edges(cuda, name, w, batch, positions, tier):
         q = data["q"].float().repeat(1, 1, positions, 1)
         q = (q + 0.2 * torch.randn(q.shape, generator=g)).to(w.dtype)
         check_retrieval(store, oracle, cfg, w, data, q, min_det_c=0.3)
+
+
+@pytest.mark.parametrize("tier", ["host", "hbm", "split"])
+@pytest.mark.parametrize("name,w,positions", [
+    ("qwen_d128", Workload("lc1", 28, 4, 128, torch.bfloat16, hot=16, cold=128 * 100 + 37, top_pages=32, top_p=256,
+                           segment=512), 40),
+    ("d64_page_48", Workload("lc2", 16, 2, 64, torch.float16, hot=16, cold=48 * 260 + 47, top_pages=40, top_p=100,
+                             segment=480, page_size=48), 60),
+], ids=["qwen_d128", "d64_page_48"])
+def test_long_query_clears_folded_keys(cuda, name, w, positions, tier):
+    """Long queries in passes over rows of more than 8,192 candidates, two
+    batch rows: keys and group maxima are folded with atomics, and blocks of
+    the gather launch clear them for the next call.  Each query asks for
+    another segment with lower scores than the one before, so that keys or
+    maxima left behind would win; rows evicted before the last one change the
+    candidates' number, and with it where the second batch row's keys and all
+    maxima lie.  The top score and the mean are this query's alone."""
+    data = generate(w, seed=61, batch=2)
+    g = torch.Generator().manual_seed(62)
+    first = w.cold - 3 * w.page_size - 11
+    part = dict(data, cold_k=data["cold_k"][:, :, :first], cold_v=data["cold_v"][:, :, :first])
+    store, oracle, cfg = build(w.with_cold(first), part, cuda, cold_tier=tier)
+    rows = torch.arange(w.num_q_heads) // w.groups
+    for call, scale in enumerate((1.0, 0.7, 0.5)):
+        if call == 2:
+            more = [data[n][:, :, first:] for n in ("cold_k", "cold_v")]
+            store.evict_from_hot(*(x.to(cuda) for x in more))
+            oracle.evict(*more)
+            part = data
+        t0 = (2 * call + 1) * w.segment
+        aim = data["cold_k"].float()[:, :, t0:t0 + w.segment].mean(2)[:, rows]  # the segment's centroid
+        q = scale * aim[:, :, None] + 0.2 * torch.randn(2, w.num_q_heads, positions, w.head_dim, generator=g)
+        q = q.to(w.dtype)
+        info = {}
+        check_retrieval(store, oracle, cfg, w, part, q, min_det_c=0.0, info=info)
+        cand = exact.candidate_ids(np.array(info["union"], dtype=np.int64), w.page_size,
+                                   store.num_pages * w.page_size, store.cold_length % w.page_size)
+        assert cand.size > 8192
+        lo, hi = score_interval(q.float().numpy(), data["cold_k"][:, :, torch.from_numpy(cand)].float().numpy(),
+                                w.scaling, DT[w.dtype], "activation")
+        lo, hi = lo.max(axis=(1, 2)), hi.max(axis=(1, 2))
+        fine = store.telemetry_snapshot()["recent"][-1]
+        assert lo.max() <= fine["top_score"] <= hi.max()
+        step = 2.0 ** -8 if w.dtype == torch.bfloat16 else 2.0 ** -11  # the mean's own rounding
+        slack = step * max(abs(lo.mean()), abs(hi.mean())) + 1e-4
+        assert lo.mean() - slack <= fine["mean_score"] <= hi.mean() + slack
 
 
 PARTIAL_ONLY = [
