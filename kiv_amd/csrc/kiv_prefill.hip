@@ -269,7 +269,6 @@ template <int DT, int KT, int MK> struct PfBlock : PfGeom<DT, KT, MK> {
   using Geom = PfGeom<DT, KT, MK>;
   using Geom::b, Geom::CPR, Geom::cold_kb, Geom::cold_vb, Geom::D, Geom::h, Geom::hot_kb, Geom::hot_vb, Geom::NT,
       Geom::nct, Geom::p, Geom::t_begin, Geom::t_end, Geom::tid, Geom::wave, Geom::lane, Geom::q0, Geom::z;
-  static constexpr int RG = 1;
   static constexpr int KROW = D + 8;        // K tile row stride in elements
   static constexpr int VROW = kPfKeys + 4;  // V^T tile row stride in elements
   static constexpr int KTILE = kPfKeys * KROW, VTILE = D * VROW;  // elements of one LDS tile
@@ -278,7 +277,7 @@ template <int DT, int KT, int MK> struct PfBlock : PfGeom<DT, KT, MK> {
   const uint8_t *tcls;  // LDS copy of this block's hot tile classes (mask tensors)
   bool cls_lds;
   int col, grp;
-  int qi[RG], qc[RG];  // the lane's query rows (rows past Q repeat row Q - 1's data)
+  int qi, qc;  // the lane's query row (rows past Q repeat row Q - 1's data)
   uint4 kreg[KJ], vreg[VJ][4];
 
   // Class of tile t, uniform over the block.
@@ -320,11 +319,8 @@ template <int DT, int KT, int MK> struct PfBlock : PfGeom<DT, KT, MK> {
     }
     col = lane & 15;
     grp = lane >> 4;
-#pragma unroll
-    for (int g = 0; g < RG; ++g) {
-      qi[g] = q0 + 16 * (RG * wave + g) + col;
-      qc[g] = min(qi[g], p.qlen - 1);
-    }
+    qi = q0 + 16 * wave + col;
+    qc = min(qi, p.qlen - 1);
   }
 
   // Loads tile t's K chunks (V key quads) into registers through a buffer
@@ -388,66 +384,51 @@ template <int DT, int KT, int MK> struct PfBlock : PfGeom<DT, KT, MK> {
     }
   }
 
-  // The lane's query fragments: row qc[g], dims 32 st + 8 grp .. + 7 of step st.
-  __device__ __forceinline__ void load_q(uint4 (&qx)[RG][KT]) const {
+  // The lane's query fragments: row qc, dims 32 st + 8 grp .. + 7 of step st.
+  __device__ __forceinline__ void load_q(uint4 (&qx)[KT]) const {
+    const char *qrow = p.q + ((int64_t)b * p.qs0 + (int64_t)h * p.qs1 + (int64_t)qc * p.qs2) * 2;
 #pragma unroll
-    for (int g = 0; g < RG; ++g) {
-      const char *qrow = p.q + ((int64_t)b * p.qs0 + (int64_t)h * p.qs1 + (int64_t)qc[g] * p.qs2) * 2;
-#pragma unroll
-      for (int st = 0; st < KT; ++st) qx[g][st] = load16(qrow + (32 * st + 8 * grp) * 2);
-    }
+    for (int st = 0; st < KT; ++st) qx[st] = load16(qrow + (32 * st + 8 * grp) * 2);
   }
 
   // MIXED tile t: scores become s * scaling * log2 e + bias (base 2), so the
   // tile's remaining factor is 1.
-  __device__ __forceinline__ void add_bias(f32x4_t (&s)[RG][4], int t) const {
+  __device__ __forceinline__ void add_bias(f32x4_t (&s)[4], int t) const {
     const bool cold = t < nct;
     const int key0 = (cold ? t : t - nct) * kPfKeys, n = (cold ? p.cold_len : p.hot_len) - key0;
+    const int64_t row_mo = this->row_mask_off(qc);
 #pragma unroll
-    for (int g = 0; g < RG; ++g) {
-      const int64_t row_mo = this->row_mask_off(qc[g]);
+    for (int sub = 0; sub < 4; ++sub) {
+      float bias[4];
+      this->bias4(cold, key0, n, 16 * sub + 4 * grp, qc, row_mo, bias);
 #pragma unroll
-      for (int sub = 0; sub < 4; ++sub) {
-        float bias[4];
-        this->bias4(cold, key0, n, 16 * sub + 4 * grp, qc[g], row_mo, bias);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) s[g][sub][i] = fmaf(s[g][sub][i], p.scale_log2, bias[i]);
-      }
+      for (int i = 0; i < 4; ++i) s[sub][i] = fmaf(s[sub][i], p.scale_log2, bias[i]);
     }
   }
 
   // The block's rows: normalised output, or (with key splits) this split's
   // unnormalised rows with their running max and row sum.
-  __device__ __forceinline__ void finish(const f32x4_t (&o)[RG][D / 16], const float (&m_run)[RG],
-                                         const float (&l_lane)[RG]) const {
+  __device__ __forceinline__ void finish(const f32x4_t (&o)[D / 16], float m_run, float l_lane) const {
+    const float l_row = half_wave_sum(row_pair_sum(l_lane));
+    if (qi >= p.qlen) return;
     if (p.nsplit > 1) {
+      const int64_t sr = this->split_row(qi);
+      float *po = p.ws_o + sr * D;
 #pragma unroll
-      for (int g = 0; g < RG; ++g) {
-        const float l_row = half_wave_sum(row_pair_sum(l_lane[g]));
-        if (qi[g] >= p.qlen) continue;
-        const int64_t sr = this->split_row(qi[g]);
-        float *po = p.ws_o + sr * D;
-#pragma unroll
-        for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<f32x4_t *>(po + 16 * dt + 4 * grp) = o[g][dt];
-        if (grp == 0) {
-          p.ws_m[sr] = m_run[g];
-          p.ws_l[sr] = l_row;
-        }
+      for (int dt = 0; dt < D / 16; ++dt) *reinterpret_cast<f32x4_t *>(po + 16 * dt + 4 * grp) = o[dt];
+      if (grp == 0) {
+        p.ws_m[sr] = m_run;
+        p.ws_l[sr] = l_row;
       }
       return;
     }
+    // A row with no visible key (fully masked) gets zeros.
+    const float inv = l_row > 0.f ? 1.f / l_row : 0.f;
+    char *orow = this->out_row(qi);
 #pragma unroll
-    for (int g = 0; g < RG; ++g) {
-      const float l_row = half_wave_sum(row_pair_sum(l_lane[g]));
-      if (qi[g] >= p.qlen) continue;
-      // A row with no visible key (fully masked) gets zeros.
-      const float inv = l_row > 0.f ? 1.f / l_row : 0.f;
-      char *orow = this->out_row(qi[g]);
-#pragma unroll
-      for (int dt = 0; dt < D / 16; ++dt)
-        *reinterpret_cast<uint2 *>(orow + (16 * dt + 4 * grp) * 2) = make_uint2(
-            pack2<DT>(o[g][dt][0] * inv, o[g][dt][1] * inv), pack2<DT>(o[g][dt][2] * inv, o[g][dt][3] * inv));
-    }
+    for (int dt = 0; dt < D / 16; ++dt)
+      *reinterpret_cast<uint2 *>(orow + (16 * dt + 4 * grp) * 2) =
+          make_uint2(pack2<DT>(o[dt][0] * inv, o[dt][1] * inv), pack2<DT>(o[dt][2] * inv, o[dt][3] * inv));
   }
 };
 
@@ -455,110 +436,75 @@ template <int DT, int KT, int MK> struct PfBlock : PfGeom<DT, KT, MK> {
 // of a 16-key sub-tile of K (A) and its own query row l % 16 (B), dims
 // 32 st + 8 (l / 16) .. + 7 of step st, and receives keys 4 (l / 16) + i of
 // the sub-tile for its row.
-template <int DT, int KT, int RG>
-__device__ __forceinline__ void pf_scores(f32x4_t (&s)[RG][4], const uint16_t *ks, const uint4 (&qx)[RG][KT], int col,
+template <int DT, int KT>
+__device__ __forceinline__ void pf_scores(f32x4_t (&s)[4], const uint16_t *ks, const uint4 (&qx)[KT], int col,
                                           int grp) {
   constexpr int KROW = 32 * KT + 8;
 #pragma unroll
-  for (int g = 0; g < RG; ++g)
-#pragma unroll
-    for (int sub = 0; sub < 4; ++sub) s[g][sub] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int sub = 0; sub < 4; ++sub) s[sub] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int st = 0; st < KT; ++st)
 #pragma unroll
     for (int sub = 0; sub < 4; ++sub) {
       const uint4 a = *reinterpret_cast<const uint4 *>(&ks[(16 * sub + col) * KROW + 32 * st + 8 * grp]);
-#pragma unroll
-      for (int g = 0; g < RG; ++g) s[g][sub] = mfma_16x16x32<DT>(a, qx[g][st], s[g][sub]);
+      s[sub] = mfma_16x16x32<DT>(a, qx[st], s[sub]);
     }
 }
-
 
 // Raises a row's running max (and rescales its accumulators) only when the
 // tile's max is more than 2^kRescaleSlack above it, so probabilities stay
 // below 256 and most tiles skip the rescale; the wave skips it when no lane
-// needs it.  pf_max_raise tests each lane's own maximum first: the row's
-// maximum exceeds the bound exactly when one of its four lanes' does (the
-// scale cc > 0 and its rounding are monotone), so the rows' maxima across
-// lanes are only formed on the tiles that raise one.
-template <int RG, int NO>
-__device__ __forceinline__ void pf_raise(const float (&mt)[RG], float (&m_run)[RG], float (&l_lane)[RG],
-                                         f32x4_t (&o)[RG][NO]) {
-  bool raise[RG], any_raise = false;
+// needs it.  Each lane's own maximum, over its 16 scores, is tested first: the
+// maximum of a row exceeds the bound exactly when that of one of its four
+// lanes (l, l ^ 16, l ^ 32, l ^ 48) does (the scale cc > 0 and its rounding
+// are monotone), so the rows' maxima across lanes are only formed on the tiles
+// that raise one.
+template <int NO>
+__device__ __forceinline__ void pf_max_raise(const f32x4_t (&s)[4], float cc, float &m_run, float &l_lane,
+                                             f32x4_t (&o)[NO]) {
+  float x = s[0][0];
 #pragma unroll
-  for (int g = 0; g < RG; ++g) {
-    raise[g] = mt[g] > m_run[g] + kRescaleSlack;
-    any_raise |= raise[g];
-  }
-  if (__ballot(any_raise)) {
+  for (int sub = 0; sub < 4; ++sub)
 #pragma unroll
-    for (int g = 0; g < RG; ++g) {
-      const float m_new = raise[g] ? mt[g] : m_run[g];
-      const float alpha = m_run[g] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[g] - m_new);
-      l_lane[g] *= alpha;
+    for (int i = 0; i < 4; ++i) x = fmaxf(x, s[sub][i]);
+  if (!__ballot(x * cc > m_run + kRescaleSlack)) return;
+  const float mt = half_wave_max(row_pair_max(x)) * cc;
+  const float m_new = mt > m_run + kRescaleSlack ? mt : m_run;
+  const float alpha = m_run == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
+  l_lane *= alpha;
 #pragma unroll
-      for (int dt = 0; dt < NO; ++dt) o[g][dt] *= alpha;
-      m_run[g] = m_new;
-    }
-  }
-}
-
-// Row maxima of one tile's scores in base-2 units (cc * s): the lane's 16
-// scores, then, on a tile that raises a row, the four lanes that share the
-// row (l, l ^ 16, l ^ 32, l ^ 48).
-template <int RG, int NO>
-__device__ __forceinline__ void pf_max_raise(const f32x4_t (&s)[RG][4], float cc, float (&m_run)[RG],
-                                             float (&l_lane)[RG], f32x4_t (&o)[RG][NO]) {
-  float x[RG];
-  bool over = false;
-#pragma unroll
-  for (int g = 0; g < RG; ++g) {
-    x[g] = s[g][0][0];
-#pragma unroll
-    for (int sub = 0; sub < 4; ++sub)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) x[g] = fmaxf(x[g], s[g][sub][i]);
-    over |= x[g] * cc > m_run[g] + kRescaleSlack;
-  }
-  if (__ballot(over)) {
-    float mt[RG];
-#pragma unroll
-    for (int g = 0; g < RG; ++g) mt[g] = half_wave_max(row_pair_max(x[g])) * cc;
-    pf_raise<RG, NO>(mt, m_run, l_lane, o);
-  }
+  for (int dt = 0; dt < NO; ++dt) o[dt] *= alpha;
+  m_run = m_new;
 }
 
 // Probabilities of one tile, 2^(cc s - m) rounded to the dtype and packed as
-// the B operand of O^T += V^T P^T: k index 8 g + i of pb[.][j] is key
+// the B operand of O^T += V^T P^T: k index 8 g + i of pb[j] is key
 // 4 g + i of sub-tile 2 j for i < 4, of sub-tile 2 j + 1 for i >= 4.  The
 // lane's share of each row sum grows by their fp32 values.  A row that has
 // seen no key keeps m = -inf; its probabilities are 0.
-template <int DT, int RG>
-__device__ __forceinline__ void pf_probs(const f32x4_t (&s)[RG][4], float cc, const float (&m_run)[RG],
-                                         float (&l_lane)[RG], uint4 (&pb)[RG][2]) {
+template <int DT>
+__device__ __forceinline__ void pf_probs(const f32x4_t (&s)[4], float cc, float m_run, float &l_lane,
+                                         uint4 (&pb)[2]) {
+  const float m_neg = m_run == -INFINITY ? 0.f : -m_run;
 #pragma unroll
-  for (int g = 0; g < RG; ++g) {
-    const float m_neg = m_run[g] == -INFINITY ? 0.f : -m_run[g];
+  for (int j = 0; j < 2; ++j) {
+    float e[8];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      float e[8];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        e[i] = __builtin_amdgcn_exp2f(fmaf(s[g][2 * j][i], cc, m_neg));
-        e[4 + i] = __builtin_amdgcn_exp2f(fmaf(s[g][2 * j + 1][i], cc, m_neg));
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) l_lane[g] += e[i];
-      pb[g][j] = make_uint4(pack2<DT>(e[0], e[1]), pack2<DT>(e[2], e[3]), pack2<DT>(e[4], e[5]), pack2<DT>(e[6], e[7]));
+    for (int i = 0; i < 4; ++i) {
+      e[i] = __builtin_amdgcn_exp2f(fmaf(s[2 * j][i], cc, m_neg));
+      e[4 + i] = __builtin_amdgcn_exp2f(fmaf(s[2 * j + 1][i], cc, m_neg));
     }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) l_lane += e[i];
+    pb[j] = make_uint4(pack2<DT>(e[0], e[1]), pack2<DT>(e[2], e[3]), pack2<DT>(e[4], e[5]), pack2<DT>(e[6], e[7]));
   }
 }
 
 // O^T += V^T P^T with v_mfma_f32_16x16x32 over 32 keys at a time: the A
 // operand holds the same keys of one dim from the V^T tile; every O^T entry
 // of a lane belongs to its query row.
-template <int DT, int D, int RG>
-__device__ __forceinline__ void pf_pv(f32x4_t (&o)[RG][D / 16], const uint4 (&pb)[RG][2], const uint16_t *vt, int col,
+template <int DT, int D>
+__device__ __forceinline__ void pf_pv(f32x4_t (&o)[D / 16], const uint4 (&pb)[2], const uint16_t *vt, int col,
                                       int grp) {
   constexpr int VROW = kPfKeys + 4;
 #pragma unroll
@@ -568,8 +514,7 @@ __device__ __forceinline__ void pf_pv(f32x4_t (&o)[RG][D / 16], const uint4 (&pb
       const uint16_t *vr = &vt[(16 * dt + col) * VROW + 32 * j + 4 * grp];
       const uint2 lo = *reinterpret_cast<const uint2 *>(vr), hi = *reinterpret_cast<const uint2 *>(vr + 16);
       const uint4 a = make_uint4(lo.x, lo.y, hi.x, hi.y);
-#pragma unroll
-      for (int g = 0; g < RG; ++g) o[g][dt] = mfma_16x16x32<DT>(a, pb[g][j], o[g][dt]);
+      o[dt] = mfma_16x16x32<DT>(a, pb[j], o[dt]);
     }
 }
 
@@ -1343,22 +1288,17 @@ template <int DT, int KT, int MK>
 __global__ void __launch_bounds__(kPfThreads) __attribute__((amdgpu_waves_per_eu(2)))
 prefill_attn_kernel(PrefillParams p) {
   using Blk = PfBlock<DT, KT, MK>;
-  constexpr int RG = Blk::RG, D = Blk::D;
+  constexpr int D = Blk::D;
   __shared__ __align__(16) uint16_t ks[Blk::KTILE];
   __shared__ __align__(16) uint16_t vt[Blk::VTILE];
   __shared__ uint8_t tcls[MK == PF_ARITH ? 1 : kPfLdsTiles];
   Blk blk(p, tcls);
-  uint4 qx[RG][KT];
+  uint4 qx[KT];
   blk.load_q(qx);
-  f32x4_t o[RG][D / 16];
-  float m_run[RG], l_lane[RG];  // l_lane: this lane's share of the row sum
+  f32x4_t o[D / 16];
 #pragma unroll
-  for (int g = 0; g < RG; ++g) {
-#pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt) o[g][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    m_run[g] = -INFINITY;
-    l_lane[g] = 0.f;
-  }
+  for (int dt = 0; dt < D / 16; ++dt) o[dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_lane = 0.f;  // l_lane: this lane's share of the row sum
   int t = blk.first_tile();
   if (t < blk.t_end) {
     blk.load_k(t);
@@ -1377,17 +1317,17 @@ prefill_attn_kernel(PrefillParams p) {
     // Scores in base-2 units are cc * s: FULL tiles keep the raw dot products
     // (cc = scaling * log2 e, folded into the exponent), MIXED tiles add the
     // bias first (cc = 1).
-    f32x4_t s[RG][4];
-    pf_scores<DT, KT, RG>(s, ks, qx, blk.col, blk.grp);
+    f32x4_t s[4];
+    pf_scores<DT, KT>(s, ks, qx, blk.col, blk.grp);
     float cc = p.scale_log2;
     if (cls == TILE_MIXED) {
       blk.add_bias(s, t);
       cc = 1.f;
     }
-    pf_max_raise<RG, D / 16>(s, cc, m_run, l_lane, o);
-    uint4 pb[RG][2];
-    pf_probs<DT, RG>(s, cc, m_run, l_lane, pb);
-    pf_pv<DT, D, RG>(o, pb, vt, blk.col, blk.grp);
+    pf_max_raise<D / 16>(s, cc, m_run, l_lane, o);
+    uint4 pb[2];
+    pf_probs<DT>(s, cc, m_run, l_lane, pb);
+    pf_pv<DT, D>(o, pb, vt, blk.col, blk.grp);
     t = tn;
   }
   blk.finish(o, m_run, l_lane);
