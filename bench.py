@@ -853,7 +853,7 @@ def prefill_chunk_run(args):
         "data": "synthetic (standard normal q, K, V)",
         "config": {"workload": f"{CHUNK_WORKLOAD}: 4096 query positions over 8192 hot keys (hot cap 4096 + "
                                "chunk 4096), 12/2 heads, D 128, boolean causal mask with offset 4096"},
-        "roofline": {"kernel": "prefill_attn_kernel (+ mask_tiles_kernel)", "bound": "mfma",
+        "roofline": {"kernel": "prefill_attn32_kernel (+ mask_tiles_kernel, prefill_merge_kernel)", "bound": "mfma",
                      "achieved": round(tflops, 1), "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(tflops / MFMA_BF16_PEAK_TFLOPS, 4), "traffic": None,
                      "flop_per_launch": useful_flop, "avg_us": round(avg, 2), "median_us": round(med, 2)},

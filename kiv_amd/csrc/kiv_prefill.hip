@@ -21,9 +21,9 @@
 //
 // Head dims up to 128 (prefill_attn32_kernel, below): 32 query rows a wave,
 // the work dealt to the GPU's block slots in equal shares (PfShares).  The
-// model's chunk, 4096 x 8192 keys of 12 heads under a boolean mask: 230.6 ->
-// 183.8 us a call, 155 GFLOP; the attention kernel about 160 us, matrix
-// cores busy 43% of its cycles (28% before), bound by the issue of the
+// model's chunk, 4096 x 8192 keys of 12 heads under a boolean mask: 230 ->
+// 181 to 189 us a call by the box, 155 GFLOP; the attention kernel's matrix
+// cores are busy 41% of its cycles (28% before), bound by the issue of the
 // softmax beside the matrix instructions with two waves a SIMD.
 //
 // Head dims above 128 (prefill_attn_kernel): wave w holds 16 query rows.

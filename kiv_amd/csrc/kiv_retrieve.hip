@@ -3115,11 +3115,13 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
   const int N = (int)s->num_pages;
   const int words = (N + 31) / 32;
   const int G = hq / hkv;
-  // Query positions per pass: the fine scan keeps the G*Qb query rows of a
-  // kv row in LDS.  Longer queries (a prefill chunk with live retrieval) run
-  // the scans once per pass of Qb positions: the union is the union of the
-  // passes' row lists and the fine keys accumulate with atomicMax, which is
-  // the max over every head and position.
+  // Query positions per pass: the fine scans that keep the G*Qb query rows of
+  // a kv row in LDS take Qb.  Longer queries (a prefill chunk with live
+  // retrieval) run the VALU scan once per pass and, on the matrix cores,
+  // fine_scan_query_kernel for what the first pass left; the coarse scan takes
+  // all positions, or as many as its keys' limit allows.  The union is that of
+  // every row list, and the fine keys accumulate with atomicMax, which is the
+  // max over every head and position.
   const int Qb = std::max(1, std::min(Q, (int)(kFineQueryBytes / ((int64_t)G * D * eb))));
   const int passes = (Q + Qb - 1) / Qb;
   const int64_t qstep = (int64_t)Qb * a->q_stride[2] * eb;  // bytes between passes' first positions
@@ -3280,7 +3282,9 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
       // kCoarseKeyBytes.  The coarse kernels keep no query rows in LDS, and
       // a launch over few rows is all latency (200 positions of 28 heads
       // over 1,024 pages in 8 passes: scan 110 us and select 55 us; in one
-      // pass of kScanRowsPerSlice rows a block 20 and 30 us).
+      // pass of kScanRowsPerSlice rows a block 20 and 30 us).  The keys stay
+      // allocated; half the limit costs 2 to 3% of such a retrieval over 262k
+      // to 1M tokens, a quarter 4% at 131k.
       const int64_t q_keys = (int64_t)B * hq * ld * 4;  // bytes of one position's keys
       const int Qc = passes == 1 ? Q : (int)std::min<int64_t>(Q, std::max<int64_t>(Qb, kCoarseKeyBytes / q_keys));
       const int rows_pass = B * hq * Qc;

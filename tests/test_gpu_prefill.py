@@ -252,9 +252,9 @@ def test_prefill_attention_fully_masked_rows_are_zero(cuda):
 def test_prefill_attention_model_chunk_full_size(cuda):
     """The whole-model run's chunk shape at full size: 4096 query positions
     over 8192 hot keys (hot cap 4096 + chunk 4096), 12 q / 2 kv heads, head
-    dim 128, bf16, the model's boolean causal mask.  This is the launch the
-    longest-first grid splits over key ranges and merges (3 splits on a
-    256-CU GPU).  The fp64 reference runs on the GPU, one head at a time, and
+    dim 128, bf16, the model's boolean causal mask.  This is the launch whose
+    blocks fill the GPU's slots with equal shares and whose cut units are
+    merged (512 shares of 384 units on a 256-CU GPU).  The fp64 reference runs on the GPU, one head at a time, and
     the bar is the module's."""
     B, hq, hkv, D, Q, T = 1, 12, 2, 128, 4096, 8192
     dt = torch.bfloat16
