@@ -442,6 +442,7 @@ __device__ int bound_candidates(const Src &src, int k, SelSh<NT> &sh, uint64_t *
   __syncthreads();
   return sh.ncand;
 }
+
 // Calls ranked(x, r) for each of the top k composites of the C candidates
 // in cand[] (C <= kRankCap), r = its rank (0 = largest): a candidate's rank
 // is the number of larger candidates.  A group of tpc lanes (a power of two,
@@ -2137,7 +2138,10 @@ __global__ void __launch_bounds__(256) fine_scan_mfma_kernel(
 // Candidates are the union pages' tokens, then the partial page's; a tile's
 // places past the last candidate (rows of the partial page's buffer not yet
 // written) store zero keys.
-template <int DT, int KT>
+// PLAN: with the select's plan as a batch row's first block; an instance of its
+// own, whose values spill 27 scalar registers around the scan's loop (none
+// without; the 64 kv rows above 87.4 -> 86.9 us).
+template <int DT, int KT, bool PLAN>
 __global__ void __launch_bounds__(256) fine_scan_heads_kernel(
     int union_src, const int32_t *__restrict__ row_pages, int row_pages_n, int words, int32_t *page_list,
     int32_t *counters, const uint64_t *__restrict__ ktab, int nchunks, int chunk_shift, int64_t page_bytes,
@@ -2175,7 +2179,8 @@ __global__ void __launch_bounds__(256) fine_scan_heads_kernel(
   // compute units, and behind them it would start when they end (1M tokens in
   // HBM with bounds, data cold: the launch 13.0 us with the plan last, 10.0
   // with it first, 9.6 without a plan).
-  const int plans = sp.plan ? 1 : 0, nscan = (int)gridDim.x - plans, bx = (int)blockIdx.x - plans;
+  constexpr int plans = PLAN ? 1 : 0;
+  const int nscan = (int)gridDim.x - plans, bx = (int)blockIdx.x - plans;
   int U = 0;
   if (union_src == UNION_ROWS) {
     U = rank_union<256>(row_pages, row_pages_n, words, ubits, upage, scan_tmp);
@@ -2186,10 +2191,12 @@ __global__ void __launch_bounds__(256) fine_scan_heads_kernel(
     U = counters[0];
   }
   auto page_of = [&](int v) -> int64_t { return union_src == UNION_ROWS ? upage[v] : page_list[v]; };
-  if (bx < 0) {
-    __shared__ SelSh<256> tsh;
-    select_plan<256>(sp, b, hkv, U, page_size, partial_len, page_of, tsh, scan_tmp);
-    return;
+  if constexpr (PLAN) {
+    if (bx < 0) {
+      __shared__ SelSh<256> tsh;
+      select_plan<256>(sp, b, hkv, U, page_size, partial_len, page_of, tsh, scan_tmp);
+      return;
+    }
   }
   const int split = U * page_size, n = split + partial_len, tiles = (n + 15) >> 4;
   const int64_t head_bytes = (int64_t)page_size * row_bytes;  // between a token's rows of two kv heads
@@ -3570,7 +3577,7 @@ static int retrieve_impl(kiv_store_t *s, const kiv_retrieve_args_t *a, hipStream
             if constexpr (KTV == 16) {
               return (int)KIV_ERR_UNSUPPORTED;
             } else {
-              auto kern = fine_scan_heads_kernel<DTV, KTV>;
+              auto kern = sp.plan ? fine_scan_heads_kernel<DTV, KTV, true> : fine_scan_heads_kernel<DTV, KTV, false>;
               hipLaunchKernelGGL(kern, dim3(nb_h + (sp.plan ? 1u : 0u), (unsigned)B), dim3(256), lds, st, union_src,
                                  (const int32_t *)s->row_pages.ptr, rows * kc, bwords, (int32_t *)s->page_list.ptr,
                                  (int32_t *)s->counters.ptr, (const uint64_t *)s->k_tab.ptr, (int)s->k_chunks.size(),
